@@ -41,6 +41,7 @@ struct TriplesState {
     double *U = nullptr;  // V pieces of one batch
     size_t u_cap = 0;
     double *F = nullptr, *E = nullptr;
+    int *queue = nullptr;  // W-build queue counters, kWQueues per batch of a call (at most one batch per work item)
 };
 
 struct scess_ctx {
@@ -118,6 +119,7 @@ void free_triples(TriplesState &t) {
     dfree(t.U);
     dfree(t.F);
     dfree(t.E);
+    dfree(t.queue);
     t = TriplesState{};
 }
 
@@ -464,6 +466,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     }
     HIP_TRY(c, hipMalloc((void **)&t.F, sizeof(double) * (t.ijk_all.size() / 3)));
     HIP_TRY(c, hipMalloc((void **)&t.E, sizeof(double)));
+    HIP_TRY(c, hipMalloc((void **)&t.queue, sizeof(int) * kWQueues * std::max<size_t>(t.work.size(), 1)));
     t.have = true;
     return SCESS_OK;
 }
@@ -521,16 +524,22 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     const size_t accb = prec == P64 || prec == PI8 ? 8 : 4;
     const int64_t wstride = vR * vR * vR;  // W in 8x8x8 blocks over vR^3
 
-    // batch size: a multiple of 8 occupied triples per launch (8 for 8-byte W, 16 for 4-byte W), so that
+    // batch size: a multiple of 8 occupied triples per launch (8 for the int8 mode, 16 else), so that
     // the XCD-ordered work-groups give each of the 8 XCDs whole triples (measured: the FP64 W-build at
     // o=50, v=500 is 27% faster than with one triple per launch, at the same HBM bytes per triple);
-    // fewer when the W sets (2 arrays x 2 sets x nbatch x vR^3) exceed a quarter of the free device memory
+    // fewer when the W sets (2 arrays x 2 sets x nbatch x vR^3) exceed a quarter of the free device memory.
+    // FP64: 16 against 8 (o=20, v=200 0.549 s against 0.560 s: fewer half-empty ends of launches); for small v
+    // as many as make 8 rounds of the W-build's items over its 512 work-groups, within 1 GiB of W
     int64_t nbatch = c->nbatch_req;
     if (nbatch <= 0) {
         const double per = 4.0 * (double)wstride * (double)accb;
         size_t fr = 0, tot = 0;
         const double budget = hipMemGetInfo(&fr, &tot) == hipSuccess ? 0.25 * (double)fr : 4.0e9;
-        nbatch = accb == 4 ? 16 : 8;
+        nbatch = prec == PI8 ? 8 : 16;
+        if (prec == P64) {
+            const int64_t nt = (v + 63) / 64, items = (v + 3) / 4 * nt * nt;
+            nbatch = std::max<int64_t>(16, std::min<int64_t>(8 * 512 / items, (int64_t)(1073741824.0 / per)));
+        }
         while (nbatch > 1 && nbatch * per > budget)
             nbatch /= 2;
     }
@@ -562,13 +571,14 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
         t.u_cap = uneed;
     }
     HIP_TRY(c, hipMemsetAsync(t.F, 0, sizeof(double) * nall, c->stream));
+    HIP_TRY(c, hipMemsetAsync(t.queue, 0, sizeof(int) * kWQueues * ((nshare + nbatch - 1) / nbatch), c->stream));
     const size_t wset = (size_t)nbatch * (size_t)wstride * accb;  // bytes of one set of W1 (or W2)
 
     const Operands &op = t.ops[prec];
     int blk = wbuild_tile(prec, (int)v);
     if (const char *ov = std::getenv("SCESS_WBUILD_BLK")) {  // tuning override: 1, 2, 4 or 5
         const int b = std::atoi(ov);
-        if (prec != PI8 && (b == 1 || b == 2 || b == 4 || b == 5))
+        if (prec != PI8 && prec != P64 && (b == 1 || b == 2 || b == 4 || b == 5))
             blk = b;
     }
     WBuildArgs wa = wbuild_args(t, prec, blk, wstride);
@@ -641,6 +651,7 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
         }
         const int nb = (int)std::min<int64_t>(nbatch, w_end - b0);
         wa.ijk = t.d_work_ijk + 3 * b0;
+        wa.queue = t.queue + kWQueues * k;
         ea.ijk = t.d_work_ijk + 3 * b0;
         wa.W1 = (char *)t.W1 + set * wset;
         wa.W2 = (char *)t.W2 + set * wset;
@@ -819,6 +830,8 @@ int scess_t_forward_noalloc(scess_ctx *c, int prec, double *e_t) {
 
     hipStream_t s = c->stream;
     hipError_t he = launch_fill_zero(F, nall, s);
+    if (he == hipSuccess && w_end > w_begin)  // the W-build's queue counters (two ints per slot of 8 bytes)
+        he = launch_fill_zero((double *)t.queue, kWQueues / 2 * (w_end - w_begin), s);
     bool cancelled = false;
     for (int64_t w = w_begin; w < w_end && he == hipSuccess; w++) {
         if (c->should_stop && ((w - w_begin) & 63) == 0) {
@@ -830,6 +843,7 @@ int scess_t_forward_noalloc(scess_ctx *c, int prec, double *e_t) {
             }
         }
         wa.ijk = t.d_work_ijk + 3 * w;
+        wa.queue = t.queue + kWQueues * (w - w_begin);
         ea.ijk = wa.ijk;
         he = launch_wbuild(prec, blk, wbuild_dma(), wa, 1, s);
         if (he == hipSuccess)
@@ -953,6 +967,9 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
         if (he == hipSuccess)
             he = hipEventCreateWithFlags(&evDone[q], hipEventDisableTiming);
     }
+    // the W-build's queue counters
+    if (he == hipSuccess)
+        he = hipMemsetAsync(t.queue, 0, sizeof(int) * kWQueues * std::max<size_t>(t.work.size(), 1), c->stream);
     // the W set zeroed by alloc on c->stream must be clear before the second stream writes it
     if (he == hipSuccess)
         he = hipStreamSynchronize(c->stream);
@@ -1011,6 +1028,7 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
                 if (b >= 2)
                     e = hipStreamWaitEvent(ws, evDone[b & 1], 0);
                 wa.ijk = t.d_work_ijk + 3 * w0;
+                wa.queue = t.queue + kWQueues * b;
                 wa.W1 = W1[b & 1];
                 wa.W2 = W2[b & 1];
                 if (e == hipSuccess)

@@ -37,6 +37,11 @@ template <int N> __device__ inline void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// s_waitcnt vmcnt(0) lgkmcnt(0)
+__device__ inline void wait_vm_lgkm0() { __builtin_amdgcn_s_waitcnt(7 << 4); }
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) const double lds_double;
+
 // Work-group id -> logical id so that consecutive logical ids run on the same
 // XCD: the dispatcher hands work-groups to the 8 XCDs of the MI355X round-robin,
 // and neighbouring work items share operand rows (one L2 per XCD).
@@ -95,7 +100,10 @@ struct WBuildArgs {
     // power-of-two scale and T2 serves both terms)
     double scale;
     int slices;    // PI8 digits per element
+    int nbatch;    // batch entries of the launch (set by launch_wbuild)
+    int *queue;    // FP64: kWQueues counters of this launch, zero before it
 };
+constexpr int kWQueues = 8;
 
 // Tile configuration: 2x2 waves, each owning blk x blk MFMA 16x16 blocks.
 int wbuild_tile(int prec, int v);  // returns blk for this precision and size

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstdlib>
+#include <type_traits>
 
 namespace scess {
 
@@ -718,186 +719,315 @@ __global__ __launch_bounds__(256) void wbuild_dma_kernel(WBuildArgs a) {
 // Whether the fixed index of segment s (get_seg numbering) sits on operand A (else on B).
 __device__ inline bool seg_fx_on_a(bool fam1, int s) { return fam1 && (s == 0 || s == 2 || s == 6 || s == 7); }
 
-// ------------------------------- W build, FP64, F fixed indices per work-group
-// wbuild_dma_kernel<P64, 2, STAGES> with F (2 or 4) outputs per work-group: the 64 x 64 tile (tr, tc)
-// of W for the fixed indices fx0 = F g .. fx0 + F - 1. In every segment exactly one operand depends on
-// the fixed index (seg_fx_on_a), so a stage holds the other operand's tile once (tile 0) and the
-// fixed-index operand's tile of each fixed index (tiles 1 .. F): F + 1 tiles of 8 KiB for F outputs,
-// where F one-index work-groups load 2F. 2F waves; wave w computes fixed index w >> 1, columns
-// 32 (w & 1) .. + 31 of the tile, all 64 rows (eight 16 x 16 blocks, 32 MFMAs per barrier against 16).
-// The fragments and the order of the MFMAs into each accumulator are those of wbuild_dma_kernel, so W
-// is bitwise the same. F = 4: 512 threads, 80 KiB of LDS and at most 128 registers (four waves per
-// SIMD), so two work-groups fill a CU.
-template <int F, int STAGES>
-__global__ __launch_bounds__(64 * 2 * F) __attribute__((amdgpu_waves_per_eu(4))) void wbuild_fx_kernel(WBuildArgs a) {
-    constexpr int RB = 128, VPR = 8;  // 16 doubles per row chunk, as eight 16-byte vectors
-    constexpr int OPB = 64 * RB;      // bytes of one operand tile chunk (8 KiB)
-    constexpr int NW = 2 * F;                        // waves
-    constexpr int NLW = (F + 1) * OPB / 1024 / NW;  // 1 KiB wave loads per wave per stage
-    static_assert((F + 1) * OPB / 1024 % NW == 0, "loads split evenly over the waves");
-    static_assert(STAGES == 2 || STAGES == 3, "stages");
-    __shared__ __attribute__((aligned(1024))) char lds[STAGES][(F + 1) * OPB];
+// ------------------------------------------------------------ W build, FP64
+// Four waves, one fixed index each: the tile (tr, tc) of W for the fixed indices fx0 = 4 g .. fx0 + 3. In
+// every segment exactly one operand depends on the fixed index (seg_fx_on_a), so an LDS stage holds the
+// other operand's tile once (tile 0) and the fixed-index operand's tile of each index (tiles 1 .. 4): five
+// tiles for four outputs, where four one-index work-groups load eight. Two work-groups fill a CU.
+//
+// A wave owns all RB x CB 16 x 16 blocks of its index, so every wave of a work-group has the same work also
+// in the tiles at the edge. The nb = ceil(v / 16) blocks of an edge are dealt out evenly over nt = ceil(v / 64)
+// tiles (B = ceil(nb / nt) or B - 1 blocks each; v = 200: 4 + 3 + 3 + 3), so no tile is nearly empty.
+//
+// The loop is bound by the matrix pipes (64 cycles per FP64 MFMA), so everything else is put under them:
+// operand fragments are read one k-step ahead of their MFMAs; the only barrier of a chunk stands before its
+// last k-step, after which the freed stage takes the loads of chunk c + 2 (in flight for a whole chunk) and the
+// first fragments of chunk c + 1 are read. k-step t of a 16-deep chunk multiplies k = 4 t .. 4 t + 3, so the
+// last chunk of a segment runs only the steps that hold k < v (or o): K costs 220, not 240, at o=20, v=200.
+// LDS rows are 128 bytes, 16-byte vector p of row r at slot p ^ swz(r); since swz(16 x + r) =
+// swz(r) ^ (2 x & 7), fragment (block x, step t) sits at lane offset so[t ^ x] + 2048 x: four offsets in all.
+//
+// Measured (E(T) per pass, same box; before: eight waves of 64 x 32 without balanced tiles, look-ahead or queue):
+// o=20, v=200 0.786 s -> 0.549 s, 1/16 of o=30, v=300 0.582 s -> 0.515 s. At v = 300 the pipes are busy 82-85% of
+// the cycles, at a clock that falls as they fill (busy x clock stayed at 1.76 GHz over four very different forms of
+// the kernel, 75% at 2.35 GHz to 85% at 2.08 GHz): the rest of the way to 78.6 TFLOP/s is power.
+// Segment s as in get_seg, one byte each: the orbital (0 = i, 1 = j, 2 = k) of the operand with the fixed index
+// (bits 0-1; X or TM), whether its rows are strided by v (bit 2: [row][fx], else [fx][row]), whether it is operand
+// A (bit 3), and the orbital pair q, r of the other operand T[q][r] or Rn[q][r] (bits 4-5, 6-7).
+constexpr uint64_t wseg_byte(int p, int strided, int fa, int q, int r) {
+    return (uint64_t)(p | strided << 2 | fa << 3 | q << 4 | r << 6);
+}
+constexpr uint64_t kWSeg1 = wseg_byte(0, 0, 1, 2, 1) | wseg_byte(0, 0, 0, 1, 2) << 8 | wseg_byte(1, 1, 1, 2, 0) << 16 |
+                            wseg_byte(2, 1, 0, 1, 0) << 24 | wseg_byte(2, 0, 0, 1, 0) << 32 |
+                            wseg_byte(0, 1, 0, 1, 2) << 40 | wseg_byte(1, 0, 1, 2, 0) << 48 |
+                            wseg_byte(0, 1, 1, 2, 1) << 56;
+constexpr uint64_t kWSeg2 = wseg_byte(1, 0, 0, 0, 2) | wseg_byte(2, 1, 0, 0, 1) << 8 | wseg_byte(2, 0, 0, 0, 1) << 16 |
+                            wseg_byte(1, 1, 0, 0, 2) << 24;
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wf = wave >> 1, wp = wave & 1;  // fixed index (0 .. F-1) and column half of this wave
-    const int lr = lane & 15, lq = lane >> 4;
+template <int B> struct WBuild64 {
+    static constexpr int F = 4, RB128 = 128, TB = 16 * B * RB128, SB = (F + 1) * TB;
+    static constexpr int HN = (2 * B + 3) / 4;  // 1 KiB (8-row) wave loads of a tile per wave
+    const WBuildArgs &a;
+    char *lds;
+    int lane, wave, v, bat;
+    int64_t ijk;  // i, j, k (<= 4096) in 16 bits each
+    int fx0;
+    bool deg;
+    int r0, c0, rb, cb;  // first row / column and number of 16-row blocks of the tile
+    int nseg1, nseg;     // segments of family 1, and in all (i == j: only six of family 1)
+    uint32_t so[4];
 
-    const int nt2 = a.nt * a.nt;
-    const int nfg = (a.v + F - 1) / F;  // fixed-index groups per family
-    const int gx = gridDim.x;
-    const int lin = xcd_remap(blockIdx.y * gx + blockIdx.x, gx * gridDim.y);
-    const int bat = lin / gx;
-    int bid = lin - bat * gx;
-    const bool fam1 = bid < nfg * nt2;
-    if (!fam1)
-        bid -= nfg * nt2;
-    const int fg = bid / nt2;
-    const int tt = bid - fg * nt2;
-    const int tr = tt / a.nt, tc = tt - tr * a.nt;
-    const int *q = a.ijk + 3 * bat;
-    const int64_t i = q[0], j = q[1], k = q[2];
-    const int v = a.v;
-    const int r0 = tr * 64, c0 = tc * 64;
-    const int64_t fx0 = (int64_t)F * fg;
-    const int64_t fx1 = min(fx0 + 1, (int64_t)v - 1);  // gives the address step per fixed index
-    // fixed indices past v load the operand rows of index v - 1; their waves compute and store nothing
-    const bool live = fx0 + wf < v;
+    // loads: segment position, chunk in it, and the segment's bases (uniform) and lane offsets
+    int ls, lk, nch, tail;
+    bool fa;
+    const char *shb, *fxb;
+    int64_t dfx;
+    uint32_t osh[HN], ofx[HN];
 
-    const bool deg = a.halve && i == j;
-    if (deg && !fam1)
-        return;  // the whole work-group: W2 of this entry is not used
-    const int nseg = fam1 ? (deg ? 6 : 8) : 4;
-    const int total = fam1 ? (deg ? 3 : 4) * (a.nchv + a.ncho) : 2 * (a.nchv + a.ncho);
+    __device__ WBuild64(const WBuildArgs &a_, char *lds_) : a(a_), lds(lds_) {}
 
-    bool vr[4], vc[2];
+    __device__ inline void set_seg() {
+        const bool fam1 = ls < nseg1;
+        const int sgi = !fam1 ? ls - nseg1 : deg ? halved_seg(ls) : ls;
+        const int d = (int)((fam1 ? kWSeg1 : kWSeg2) >> (8 * sgi)) & 255;
+        const bool fterm = sgi < (fam1 ? 4 : 2), strided = d & 4;
+        fa = d & 8;
+        nch = fterm ? a.nchv : a.ncho;
+        tail = ((fterm ? v : a.o) - 16 * (nch - 1) + 3) >> 2;  // k-steps of the segment's last chunk
+        const int64_t rowb = fterm ? a.rbv : a.rbo, vrow = v * rowb;
+        auto orb = [=](int n) { return (ijk >> (16 * n)) & 0xffff; };
+        dfx = strided ? rowb : vrow;
+        const int64_t lfx = strided ? vrow : rowb;
+        const int q0 = fa ? c0 : r0, p0 = fa ? r0 : c0;  // first row of the shared and of the fixed-index tiles
+        shb = (fterm ? a.T : a.Rn) + ((orb(d >> 4 & 3) * a.o + orb(d >> 6)) * v + q0) * rowb;
+        fxb = (fterm ? a.X : a.TM) + orb(d & 3) * v * vrow + fx0 * dfx + p0 * lfx;
 #pragma unroll
-    for (int x = 0; x < 4; x++)
-        vr[x] = r0 + x * 16 < v;
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-        vc[y] = c0 + wp * 32 + y * 16 < v;
-
-    d4 acc[4][2];
-#pragma unroll
-    for (int x = 0; x < 4; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++)
-            acc[x][y] = d4{};
-
-    // wave load L = u * NW + wave fills LDS KiB L of a stage: tile L / 8 (a constant of u, since NW is 4
-    // or 8), rows 8 (L % 8) .. + 7; the lane's row in its tile and the byte offset of the logical vector
-    // it fetches (fixed per lane)
-    constexpr auto tile_of = [](int u) { return u * NW / 8; };
-    int lrow[NLW], lvoff[NLW];
-#pragma unroll
-    for (int u = 0; u < NLW; u++) {
-        const int L = u * NW + wave;
-        const int r = (L & 7) * 8 + (lane >> 3), p = lane & 7;
-        lrow[u] = r;
-        lvoff[u] = (p ^ lds_swz<VPR>(r)) * 16;
+        for (int h = 0; h < HN; h++) {
+            const int r = 8 * (wave + 4 * h) + (lane >> 3);
+            const uint32_t vo = ((lane & 7) ^ lds_swz<8>(r)) * 16;
+            // rows past v load row v - 1 (valid memory whose outputs are never stored)
+            osh[h] = (uint32_t)min(r, v - 1 - q0) * (uint32_t)rowb + vo;
+            ofx[h] = (uint32_t)min(r, v - 1 - p0) * (uint32_t)lfx + vo;
+        }
     }
 
-    // this lane's load addresses at k-chunk 0 of segment sgi (rows past v load row v - 1, valid memory
-    // whose outputs are never stored); a chunk adds kc * RB
-    const char *pl[NLW];
-    int nch = 0;
-    bool fa = false;
-    auto set_seg = [&](int sgi) {
-        const Seg s0 = get_seg(a, fam1, sgi, i, j, k, fx0);
-        const Seg s1 = get_seg(a, fam1, sgi, i, j, k, fx1);  // address arithmetic only: the step per index
-        fa = seg_fx_on_a(fam1, sgi);
-        nch = s0.nch;
-        const int64_t dfx = fa ? s1.A - s0.A : s1.B - s0.B;  // bytes per fixed index (0 if fx1 == fx0)
+    // Loads h of the next chunk into stage st
+    __device__ inline void issue(int st, int h) const {
+        char *base = lds + st * SB;
+        const int64_t ko = (int64_t)lk * RB128;
+        const int u = wave + 4 * h;
+        if (u < 2 * (fa ? cb : rb))
+            __builtin_amdgcn_global_load_lds((const void *)(shb + ko + osh[h]), (lds_void *)(base + u * 1024), 16, 0, 0);
+        if (u < 2 * (fa ? rb : cb))
 #pragma unroll
-        for (int u = 0; u < NLW; u++) {
-            const int tl = tile_of(u);
-            // tile 0: the operand without the fixed index; tile 1 + t: the one with it, index fx0 + t
-            const bool use_a = (tl == 0) != fa;
-            const int64_t t = tl == 0 ? 0 : min(fx0 + tl - 1, (int64_t)v - 1) - fx0;
-            const char *base = (use_a ? s0.A : s0.B) + t * dfx;
-            const int64_t ld = use_a ? s0.lda : s0.ldb;
-            const int row = min((use_a ? r0 : c0) + lrow[u], v - 1);
-            pl[u] = base + row * ld + lvoff[u];
-        }
-    };
-    set_seg(0);
-    int s = 0, kc = 0, famask = 0;  // famask bit st: the chunk in stage st has the fixed index on A
-    auto issue = [&](int st) {
-        char *base = lds[st];
-        const int64_t off = (int64_t)kc * RB;
-#pragma unroll
-        for (int u = 0; u < NLW; u++)
-            __builtin_amdgcn_global_load_lds((const void *)(pl[u] + off),
-                                             (lds_void *)(base + (u * NW + wave) * 1024), 16, 0, 0);
-        famask = fa ? famask | (1 << st) : famask & ~(1 << st);
-        if (++kc == nch) {
-            kc = 0;
-            if (++s < nseg)
-                set_seg(deg ? halved_seg(s) : s);
-        }
-    };
-    auto frag = [&](const char *op, int rr, int lv) { return op + rr * RB + ((lv ^ lds_swz<VPR>(rr)) * 16); };
-    auto compute = [&](int st) {
-        const bool sa = (famask >> st) & 1;
-        const char *T0 = lds[st], *Tf = lds[st] + (1 + wf) * OPB;
-        const char *As = sa ? Tf : T0, *Bs = sa ? T0 : Tf;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {  // two k-pairs per 16-byte vector
-            d2 af[4], bf[2];
-#pragma unroll
-            for (int x = 0; x < 4; x++)
-                af[x] = *(const d2 *)frag(As, x * 16 + lr, 2 * lq + h);
-#pragma unroll
-            for (int y = 0; y < 2; y++)
-                bf[y] = *(const d2 *)frag(Bs, wp * 32 + y * 16 + lr, 2 * lq + h);
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (vr[x])
-#pragma unroll
-                        for (int y = 0; y < 2; y++)
-                            if (vc[y])
-                                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[x][t], bf[y][t], acc[x][y], 0, 0, 0);
-        }
-    };
-
-#pragma unroll
-    for (int st = 0; st < STAGES - 1; st++)
-        if (st < total)
-            issue(st);
-    for (int c = 0; c < total; c++) {
-        // this wave's loads of chunk c have landed once at most the next chunk's are outstanding
-        if (STAGES > 2 && c + 1 < total)
-            wait_vm<(STAGES > 2 ? NLW : 0)>();
-        else
-            wait_vm<0>();
-        __syncthreads();  // every wave's chunk c is in LDS; stage (c - 1) % STAGES is free again
-        if (c + STAGES - 1 < total)
-            issue((c + STAGES - 1) % STAGES);
-        if (live)
-            compute(c % STAGES);
+            for (int t = 0; t < F; t++)  // fixed indices past v load index v - 1
+                __builtin_amdgcn_global_load_lds((const void *)(fxb + min(t, v - 1 - fx0) * dfx + ko + ofx[h]),
+                                                 (lds_void *)(base + (1 + t) * TB + u * 1024), 16, 0, 0);
     }
-    if (!live)
-        return;
+    // After all loads of a chunk: its k-steps and (bit 3) whether A carries the fixed index; moves to the next
+    __device__ inline int next() {
+        const int info = (lk == nch - 1 ? tail : 4) | (fa ? 8 : 0);
+        if (++lk == nch) {
+            lk = 0;
+            if (++ls < nseg)
+                set_seg();
+        }
+        return info;
+    }
 
-    double *W = (double *)(fam1 ? a.W1 : a.W2) + (int64_t)bat * a.wstride;
-    const int nbR = a.vR >> 3;
-    const int64_t fx = fx0 + wf;
-    const int64_t fbase = ((int64_t)(fx >> 3) * nbR) * nbR * 512 + (fx & 7) * 64;
+    // The chunks, whose first two (infos cur, nxt) are being loaded, for a tile of RB x CB blocks
+    template <int RB, int CB> __device__ inline void run(int cur, int nxt) {
+        const int nc = a.nchv + a.ncho, total1 = nseg1 / 2 * nc, total = nseg / 2 * nc;  // chunks of family 1, of both
+        d4 acc[RB][CB];
+        double fr[2][RB], fc[2][CB];
 #pragma unroll
-    for (int x = 0; x < 4; x++)
+        for (int x = 0; x < RB; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++) {
-            const int col = c0 + wp * 32 + y * 16 + lr;
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = d4{};
+        lds_char *pa, *pb;  // the wave's A and B tiles of the chunk whose fragments are read
+        auto tiles = [&](int st, int info) {
+            lds_char *t0 = (lds_char *)lds + st * SB, *tf = t0 + (1 + wave) * TB;
+            pa = info & 8 ? tf : t0;
+            pb = info & 8 ? t0 : tf;
+        };
+        auto read = [&](auto tc, int buf) {
+            constexpr int t = decltype(tc)::value;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = r0 + x * 16 + lq + 4 * r;
-                if (row < v && col < v)
-                    W[fbase + ((int64_t)(row >> 3) * nbR + (col >> 3)) * 512 + (row & 7) * 8 + (col & 7)] = acc[x][y][r];
+            for (int x = 0; x < RB; x++)
+                fr[buf][x] = *(lds_double *)(pa + so[t ^ x] + x * 2048);
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[buf][y] = *(lds_double *)(pb + so[t ^ y] + y * 2048);
+        };
+        // row x of blocks of the k-step in buffer buf. The rows are kept apart so that other work stands between
+        // them: an MFMA holds the pipe for 64 cycles, under which the wave reads fragments and issues loads.
+        // (Fragments read just before an MFMA would hold it up, as its wait counts the new reads too.)
+        auto row = [&](int buf, int x) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[buf][x], fc[buf][y], acc[x][y], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        using std::integral_constant;
+        // a k-step, with the fragments of the next one (t) read into the other buffer after its first row
+        auto step = [&](int buf, auto tc) {
+            row(buf, 0);
+            read(tc, buf ^ 1);
+#pragma unroll
+            for (int x = 1; x < RB; x++)
+                row(buf, x);
+        };
+        auto move = [&]() {  // buffer 0 to buffer 1
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+                fr[1][x] = fr[0][x];
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[1][y] = fc[0][y];
+        };
+        wait_vm_lgkm0();
+        __syncthreads();
+        tiles(0, cur);
+        read(integral_constant<int, 0>{}, 0);
+        for (int c = 0; c < total; c++) {
+            // all k-steps of chunk c but its last, whose fragments end up in buffer 1
+            const int steps = cur & 7;
+            if (steps >= 2) {
+                step(0, integral_constant<int, 1>{});
+                if (steps >= 3) {
+                    step(1, integral_constant<int, 2>{});
+                    if (steps == 4)
+                        step(0, integral_constant<int, 3>{});
+                    else
+                        move();
+                }
+            } else {
+                move();
             }
+            int nn = 0;
+            const bool more = c + 1 < total, load = c + 2 < total;
+            if (more) {
+                // chunk c + 1, in flight since the last step of chunk c - 1, and this wave's reads of stage c:
+                // the stage takes chunk c + 2
+                wait_vm_lgkm0();
+                __syncthreads();
+            }
+            row(1, 0);
+            if (more) {
+                tiles((c + 1) & 1, nxt);
+                read(integral_constant<int, 0>{}, 0);
+            }
+#pragma unroll
+            for (int x = 1; x < (RB > HN ? RB : HN + 1); x++) {
+                if (load && x <= HN)
+                    issue(c & 1, x - 1);
+                if (x < RB)
+                    row(1, x);
+            }
+            if (load)
+                nn = next();
+            cur = nxt;
+            nxt = nn;
+            if (c + 1 != total1 && c + 1 != total)
+                continue;
+            // a family is complete: element (fixed, row, col) of W in 8x8x8 blocks (r0 and c0 are multiples of 16)
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // keeps the store addresses from being formed, and held, before the loop
+            const int fx = fx0 + wave, lr = ln & 15, lq = ln >> 4, nbR = a.vR >> 3;
+            double *W = (double *)(c + 1 == total1 ? a.W1 : a.W2) + (int64_t)bat * a.wstride +
+                        (((int64_t)(fx >> 3) * nbR + (r0 >> 3)) * nbR + (c0 >> 3)) * 512 + (fx & 7) * 64 + lq * 8 +
+                        (lr >> 3) * 512 + (lr & 7);
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    double *Wr = W + (int64_t)(2 * x + (r >> 1)) * nbR * 512 + (r & 1) * 32;
+                    const bool ok = fx < v && r0 + x * 16 + lq + 4 * r < v;
+#pragma unroll
+                    for (int y = 0; y < CB; y++) {
+                        if (ok && c0 + y * 16 + lr < v)
+                            Wr[y * 1024] = acc[x][y][r];
+                        acc[x][y][r] = 0.0;
+                    }
+                }
         }
+    }
+};
+
+// Work items are dealt out at run time. An item is one tile of one unit, a unit the nt^2 tiles of one (triple,
+// group of four fixed indices); units go round-robin to 8 queues, one per XCD (work-group w runs on XCD w % 8), so
+// the tiles of a unit, which share operand rows, meet in one L2. A work-group that finds its queue empty takes from
+// the next one. (As one work-group per item the launch kept 1.3 of the two work-groups that fit a CU resident at
+// v = 200: tiles and triples with i == j differ in cost by up to 4x, and work-groups are placed in order.)
+template <int B>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B >= 3 ? 2 : 4))) void
+wbuild_f64_kernel(WBuildArgs a) {
+    __shared__ __attribute__((aligned(1024))) char lds[2 * WBuild64<B>::SB];
+    WBuild64<B> w(a, lds);
+    w.lane = threadIdx.x & 63;
+    w.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    w.v = a.v;
+    const int nt2 = a.nt * a.nt, nfg = (a.v + 3) / 4, units = nfg * a.nbatch, nb = (a.v + 15) >> 4;
+    const int lr = w.lane & 15, lq = w.lane >> 4;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        w.so[u] = lr * 128 + ((2 * u + (lq >> 1)) ^ lds_swz<8>(lr)) * 16 + (lq & 1) * 8;
+    // the next item as 8 * (place in its queue) + queue, or -1: every queue's counter only grows, so each
+    // work-group comes to -1 (thread 0 only)
+    auto take = [&]() {
+        for (int n = 0; n < 8; n++) {
+            const int q = (blockIdx.x + n) & 7, len = (units - q + 7) / 8 * nt2;
+            const int at = len > 0 ? atomicAdd(&a.queue[q], 1) : 0;
+            if (at < len)
+                return 8 * at + q;
+        }
+        return -1;
+    };
+    // hands thread 0's item to the work-group through the (idle) stages: two work-groups of B = 4 fill the LDS
+    auto share = [&](int mine) {
+        __syncthreads();
+        if (threadIdx.x == 0)
+            *(int *)lds = mine;
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane(*(int *)lds);
+        __syncthreads();
+        return item;
+    };
+    int mine = threadIdx.x == 0 ? take() : 0;
+    for (int item = share(mine); item >= 0; item = share(mine)) {
+        const int at = item >> 3, un = at / nt2, tt = at - un * nt2, unit = un * 8 + (item & 7);
+        w.bat = unit / nfg;
+        w.fx0 = 4 * (unit - w.bat * nfg);
+        const int tr = tt / a.nt, tc = tt - tr * a.nt;
+        const int *q = a.ijk + 3 * w.bat;
+        const int qi = __builtin_amdgcn_readfirstlane(q[0]), qj = __builtin_amdgcn_readfirstlane(q[1]),
+                  qk = __builtin_amdgcn_readfirstlane(q[2]);
+        w.ijk = (int64_t)qk << 32 | (int64_t)qj << 16 | qi;
+        w.deg = a.halve && qi == qj;
+        const int tr0 = tr * nb / a.nt, tc0 = tc * nb / a.nt;
+        w.rb = (tr + 1) * nb / a.nt - tr0;
+        w.cb = (tc + 1) * nb / a.nt - tc0;
+        w.r0 = 16 * tr0;
+        w.c0 = 16 * tc0;
+        w.nseg1 = w.deg ? 6 : 8;
+        w.nseg = w.deg ? 6 : 12;
+        w.ls = w.lk = 0;
+        w.set_seg();
+        int info[2];
+#pragma unroll
+        for (int st = 0; st < 2; st++) {  // an item has at least six chunks
+#pragma unroll
+            for (int h = 0; h < WBuild64<B>::HN; h++)
+                w.issue(st, h);
+            info[st] = w.next();
+        }
+        if (threadIdx.x == 0)
+            mine = take();  // under the first loads
+        constexpr int L = B > 1 ? B - 1 : 1;
+        if (w.rb == B) {
+            if (w.cb == B)
+                w.template run<B, B>(info[0], info[1]);
+            else
+                w.template run<B, L>(info[0], info[1]);
+        } else {
+            if (w.cb == B)
+                w.template run<L, B>(info[0], info[1]);
+            else
+                w.template run<L, L>(info[0], info[1]);
+        }
+    }
 }
 
 // ------------------------------------------------------ W build, int8 digits
@@ -1153,7 +1283,7 @@ int i8_fixed_per_group(int slices) { return slices == 5 ? 2 : 1; }
 // and FP32; 4 for BF16x3, whose three MFMAs per product need the larger register tile to keep
 // LDS reads per MFMA low.
 int wbuild_tile(int prec, int v) {
-    if (prec == PI8)
+    if (prec == PI8 || prec == P64)
         return 2;
     if (prec == PB3 && v >= 240)
         return 4;
@@ -1162,28 +1292,33 @@ int wbuild_tile(int prec, int v) {
     return 1;
 }
 
+// FP64: a.nt = ceil(v / 64) tiles of B = ceil(ceil(v / 16) / nt) or B - 1 blocks per edge
+static hipError_t launch_wbuild_f64(WBuildArgs a, int nbatch, hipStream_t s) {
+    // the lane offsets of a tile's rows are 32 bits wide (so for every v <= 2620, the largest whose o = 2
+    // integrals fit in 288 GB)
+    if (64.0 * a.v * (double)a.rbv >= 4294967296.0)
+        return hipErrorInvalidValue;
+    const int nb = (a.v + 15) / 16, b = (nb + a.nt - 1) / a.nt;
+    // as many work-groups as fit the chip (two per CU for B >= 3: 80 or 60 KiB of LDS and 256 registers each;
+    // four for the smaller tiles), or one per item
+    const int64_t items = (int64_t)((a.v + 3) / 4) * nbatch * a.nt * a.nt;
+    if (items > 0x0fffffff)
+        return hipErrorInvalidValue;
+    const dim3 grid((unsigned)std::min<int64_t>(items, 256 * (b >= 3 ? 2 : 4)));
+    a.nbatch = nbatch;
+    switch (b) {
+    case 1: hipLaunchKernelGGL(wbuild_f64_kernel<1>, grid, dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL(wbuild_f64_kernel<2>, grid, dim3(256), 0, s, a); break;
+    case 3: hipLaunchKernelGGL(wbuild_f64_kernel<3>, grid, dim3(256), 0, s, a); break;
+    case 4: hipLaunchKernelGGL(wbuild_f64_kernel<4>, grid, dim3(256), 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 template <int PREC>
 static hipError_t launch_wbuild_p(int blk, bool dma, const WBuildArgs &a, int nbatch, hipStream_t s) {
     const dim3 grid((unsigned)(2 * a.ntile1), (unsigned)nbatch);
-    if constexpr (PREC == P64) {
-        // FP64 64 x 64 tiles: four fixed indices per work-group (SCESS_WBUILD_F2=0: one, tuning override)
-        const char *e = std::getenv("SCESS_WBUILD_F2");
-        if (dma && blk == 2 && !(e && std::atoi(e) == 0)) {
-            const dim3 g2((unsigned)(2 * ((a.v + 1) / 2) * a.nt * a.nt), (unsigned)nbatch);
-            const char *es = std::getenv("SCESS_WBUILD_STAGES");  // tuning override: 3 (two indices)
-            const char *ef = std::getenv("SCESS_WBUILD_FX");      // tuning override: 2 fixed indices
-            if ((ef && std::atoi(ef) == 2) || (es && std::atoi(es) == 3)) {
-                if (es && std::atoi(es) == 3)
-                    hipLaunchKernelGGL((wbuild_fx_kernel<2, 3>), g2, dim3(256), 0, s, a);
-                else
-                    hipLaunchKernelGGL((wbuild_fx_kernel<2, 2>), g2, dim3(256), 0, s, a);
-            } else {
-                const dim3 g4((unsigned)(2 * ((a.v + 3) / 4) * a.nt * a.nt), (unsigned)nbatch);
-                hipLaunchKernelGGL((wbuild_fx_kernel<4, 2>), g4, dim3(512), 0, s, a);
-            }
-            return hipGetLastError();
-        }
-    }
     if (dma && (blk == 2 || blk == 4 || (blk == 5 && PREC != P32))) {
         // two stages: more resident work-groups per CU beat deeper prefetch (sweeps at v = 300)
         int st = 2;
@@ -1240,7 +1375,7 @@ hipError_t launch_wbuild(int prec, int blk, bool dma, const WBuildArgs &a, int n
         return hipErrorInvalidValue;
     }
     if (prec == P64)
-        return launch_wbuild_p<P64>(blk, dma, a, nbatch, s);
+        return launch_wbuild_f64(a, nbatch, s);
     if (prec == P32)
         return launch_wbuild_p<P32>(blk, dma, a, nbatch, s);
     return launch_wbuild_p<PB3>(blk, dma, a, nbatch, s);
