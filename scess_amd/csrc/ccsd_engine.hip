@@ -99,6 +99,64 @@ __global__ __launch_bounds__(256) void permute_split_kernel(PermArgs a, int64_t 
     o[8] = lo;
 }
 
+// A whole einsum of a small system in one launch, straight from the operands: G lanes per output element, lane g
+// summing k = g, g + G, ... (then a fixed xor tree). The operand offsets of up to KT values of the summed index are
+// decomposed once per work-group into LDS. Bound by launches, not by the chip: the CCSD of a water-sized molecule is
+// some 60 contractions of microseconds per iteration, which as permute, permute, zero fill, GEMM, permute with two
+// allocations each took 39 ms for o=5, v=19 (11 iterations).
+struct ContractArgs {
+    int no, nk;                 // output and summed dimensions
+    int od[MAXD], kd[MAXD];     // their extents, last fastest
+    int64_t oa[MAXD], ob[MAXD], oc[MAXD];  // strides of the output dimensions in A, B (0 where absent) and C
+    int64_t ka[MAXD], kb[MAXD];            // strides of the summed dimensions in A and B
+    const double *A, *B;
+    double *C;
+    double alpha, beta;
+    int n, K, glog;             // outputs, summed extent, log2 of G
+};
+constexpr int kContractTable = 2048;
+
+__global__ __launch_bounds__(256) void contract_kernel(ContractArgs a) {
+    __shared__ int ta[kContractTable], tb[kContractTable];
+    const int G = 1 << a.glog, g = threadIdx.x & (G - 1);
+    const int64_t out = (int64_t)blockIdx.x * (256 >> a.glog) + (threadIdx.x >> a.glog);
+    const bool live = out < a.n;
+    int64_t pa = 0, pb = 0, pc = 0;
+    int r = live ? (int)out : 0;
+    for (int d = a.no - 1; d >= 0; d--) {
+        const int q = r / a.od[d], i = r - q * a.od[d];
+        pa += i * a.oa[d];
+        pb += i * a.ob[d];
+        pc += i * a.oc[d];
+        r = q;
+    }
+    double s = 0.0;
+    for (int k0 = 0; k0 < a.K; k0 += kContractTable) {
+        const int kn = min(a.K - k0, kContractTable);
+        if (k0)
+            __syncthreads();
+        for (int k = threadIdx.x; k < kn; k += 256) {
+            int q = k0 + k, xa = 0, xb = 0;  // the operands hold less than 2^31 elements here
+            for (int d = a.nk - 1; d >= 0; d--) {
+                const int t = q / a.kd[d], i = q - t * a.kd[d];
+                xa += i * (int)a.ka[d];
+                xb += i * (int)a.kb[d];
+                q = t;
+            }
+            ta[k] = xa;
+            tb[k] = xb;
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int k = g; k < kn; k += G)
+            s += a.A[pa + ta[k]] * a.B[pb + tb[k]];
+    }
+    for (int m = G >> 1; m >= 1; m >>= 1)
+        s += __shfl_xor(s, m, 64);
+    if (live && g == 0)
+        a.C[pc] = a.beta == 0.0 ? a.alpha * s : a.beta * a.C[pc] + a.alpha * s;
+}
+
 // out = alpha * x + beta * y (elementwise)
 __global__ __launch_bounds__(256) void axpby_kernel(double *out, const double *x, const double *y, double alpha,
                                                     double beta, int64_t n) {
@@ -140,7 +198,7 @@ __global__ __launch_bounds__(256) void jacobi_kernel(double *t1, double *t2, con
 }
 
 // partial dot products, fixed order: part[block] = sum over the block's range
-__global__ __launch_bounds__(256) void dot_kernel(const double *x, const double *y, int64_t n, double *part) {
+__device__ inline void dot_body(const double *x, const double *y, int64_t n, double *part) {
     __shared__ double rs[256], rc[256];
     const int64_t per = (n + gridDim.x - 1) / gridDim.x;
     const int64_t b0 = (int64_t)blockIdx.x * per, b1 = min(n, b0 + per);
@@ -168,6 +226,15 @@ __global__ __launch_bounds__(256) void dot_kernel(const double *x, const double 
     }
     if (threadIdx.x == 0)
         part[blockIdx.x] = rs[0] + rc[0];
+}
+
+// dot_kernel of x with each of up to kMaxDots vectors y (blockIdx.y): the same ranges and order
+constexpr int kDotBlocks = 256;
+struct DotVecs {
+    const double *y[Engine::kMaxDots];
+};
+__global__ __launch_bounds__(256) void dots_kernel(const double *x, DotVecs v, int64_t n, double *part) {
+    dot_body(x, v.y[blockIdx.y], n, part + (int64_t)blockIdx.y * gridDim.x);
 }
 
 hipError_t ccsd_jacobi(double *t1, double *t2, const double *e, int o, int v, hipStream_t s) {
@@ -365,32 +432,65 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         return d;
     };
     const int64_t nb = prod(Lb), M = prod(Lm), N = prod(Ln), K = prod(Lk);
+    // Small FP64 contractions in one launch (contract_kernel). The line is where its products at some 0.5 TFLOP/s
+    // cost what the GEMM path's extra launches do (about 40 us): 1 << 24 products.
+    if (prec == P64 && nb * M * N * std::max<int64_t>(K, 1) <= (int64_t)1 << 24 && A.size() < (int64_t)1 << 31 &&
+        B->size() < (int64_t)1 << 31) {
+        contract(la, A, lb, *B, lc, Lk, C, alpha, beta);
+        return;
+    }
     // operands in [batch][M][K] and [batch][N][K]: FP64, or (BF16x3 products) pre-split rows of
-    // Ks = Kp / 2 eight-byte slots, written by the permute itself
+    // Ks = Kp / 2 eight-byte slots, written by the permute itself. An FP64 operand that has that order
+    // already is used as it is; of the orders of the summed labels, the one in which more of it is.
     const bool split = prec == PB3 && M > 0 && N > 0 && K > 0;
     const int64_t Ks = split ? (K + 31) / 32 * 16 : K;
-    DTensor Ap, Bp, Cp = alloc({nb, M, N}, true);
+    if (!split) {
+        std::string Lk2;
+        for (char x : lb)
+            if (Lk.find(x) != std::string::npos)
+                Lk2 += x;
+        const auto as_is = [&](const std::string &lk) {
+            return (la == Lb + Lm + lk ? A.size() : 0) + (lb == Lb + Ln + lk ? B->size() : 0);
+        };
+        if (as_is(Lk2) > as_is(Lk))
+            Lk = Lk2;
+    }
+    // the GEMM writes (or adds to) C itself where C has the order [batch][M][N]
+    const bool direct = lc == Lb + Lm + Ln && M > 0 && N > 0 && K > 0 && (beta == 0.0 || beta == 1.0);
+    DTensor Ap, Bp, Cp;
+    const double *pA = A.p, *pB = B->p;
+    if (!direct)
+        Cp = alloc({nb, M, N}, K == 0);
     if (split) {
         Ap = permute_split(la, A.p, A.dims, Lb + Lm + Lk, dims_of(Lb + Lm + Lk), K);
         Bp = permute_split(lb, B->p, B->dims, Lb + Ln + Lk, dims_of(Lb + Ln + Lk), K);
+        pA = Ap.p;
+        pB = Bp.p;
     } else {
-        Ap = alloc({nb, M, K});
-        Bp = alloc({nb, N, K});
-        permute(la, A.p, A.dims, Lb + Lm + Lk, Ap.p, dims_of(Lb + Lm + Lk), 1.0, 0.0);
-        permute(lb, B->p, B->dims, Lb + Ln + Lk, Bp.p, dims_of(Lb + Ln + Lk), 1.0, 0.0);
+        if (la != Lb + Lm + Lk) {
+            Ap = alloc({nb, M, K});
+            permute(la, A.p, A.dims, Lb + Lm + Lk, Ap.p, dims_of(Lb + Lm + Lk), 1.0, 0.0);
+            pA = Ap.p;
+        }
+        if (lb != Lb + Ln + Lk) {
+            Bp = alloc({nb, N, K});
+            permute(lb, B->p, B->dims, Lb + Ln + Lk, Bp.p, dims_of(Lb + Ln + Lk), 1.0, 0.0);
+            pB = Bp.p;
+        }
     }
     if (M > 0 && N > 0 && K > 0) {
         GemmArgs g{};
         g.nseg = 1;
         g.M = (int)M;
         g.N = (int)N;
-        g.alpha = 1.0;
+        g.alpha = direct ? alpha : 1.0;
+        g.ow = !direct || beta == 0.0;
         g.splits = 1;
         g.seg[0].K1 = 1;
         g.seg[0].K2 = (int)Ks;
-        g.seg[0].A = {Ap.p, Ks, 0, 1, M * Ks};
-        g.seg[0].B = {Bp.p, Ks, 0, 1, N * Ks};
-        g.C = Cp.p;
+        g.seg[0].A = {pA, Ks, 0, 1, M * Ks};
+        g.seg[0].B = {pB, Ks, 0, 1, N * Ks};
+        g.C = direct ? C.p : Cp.p;
         g.sCm = N;
         g.sCn = 1;
         g.sCb = M * N;
@@ -412,28 +512,88 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         }
         check(launch_gemm(g, (int)nb, stream), "einsum gemm");
     }
-    permute(Lb + Lm + Ln, Cp.p, dims_of(Lb + Lm + Ln), lc, C.p, C.dims, alpha, beta);
+    if (!direct)
+        permute(Lb + Lm + Ln, Cp.p, dims_of(Lb + Lm + Ln), lc, C.p, C.dims, alpha, beta);
+}
+
+// C = beta C + alpha sum over the labels lk of A B, by contract_kernel
+void Engine::contract(const std::string &la, const DTensor &A, const std::string &lb, const DTensor &B,
+                      const std::string &lc, const std::string &lk, DTensor &C, double alpha, double beta) {
+    if (lc.size() > MAXD || lk.size() > MAXD)
+        throw std::runtime_error("contract: rank");
+    auto stride = [](const std::string &l, const DTensor &t, char x) -> int64_t {
+        const auto p = l.find(x);
+        if (p == std::string::npos)
+            return 0;
+        int64_t s = 1;
+        for (size_t d = p + 1; d < t.dims.size(); d++)
+            s *= t.dims[d];
+        return s;
+    };
+    ContractArgs a{};
+    a.no = (int)lc.size();
+    a.nk = (int)lk.size();
+    a.n = 1;
+    a.K = 1;
+    for (int d = 0; d < a.no; d++) {
+        a.od[d] = (int)C.dims[d];
+        a.n *= a.od[d];
+        a.oa[d] = stride(la, A, lc[d]);
+        a.ob[d] = stride(lb, B, lc[d]);
+        a.oc[d] = stride(lc, C, lc[d]);
+    }
+    for (int d = 0; d < a.nk; d++) {
+        a.kd[d] = (int)A.dims[la.find(lk[d])];
+        a.K *= a.kd[d];
+        a.ka[d] = stride(la, A, lk[d]);
+        a.kb[d] = stride(lb, B, lk[d]);
+    }
+    if (a.n == 0)
+        return;
+    a.A = A.p;
+    a.B = B.p;
+    a.C = C.p;
+    a.alpha = alpha;
+    a.beta = beta;
+    // lanes per output: up to 64, while a lane keeps 16 terms or more and the launch fewer than 2^18 lanes
+    while (a.glog < 6 && (a.K >> a.glog) >= 32 && ((int64_t)a.n << a.glog) < (1 << 17))
+        a.glog++;
+    const int64_t per = 256 >> a.glog, blocks = (a.n + per - 1) / per;
+    hipLaunchKernelGGL(contract_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    check(hipGetLastError(), "contract");
+}
+
+void Engine::dots(const double *x, const double *const *y, int m, int64_t n, double *out) {
+    if (m < 1 || m > kMaxDots)
+        throw std::runtime_error("dots: count");
+    if (!dotbuf)
+        check(hipMalloc((void **)&dotbuf, sizeof(double) * kDotBlocks * kMaxDots), "hipMalloc dot");
+    DotVecs v{};
+    for (int q = 0; q < m; q++)
+        v.y[q] = y[q];
+    hipLaunchKernelGGL(dots_kernel, dim3(kDotBlocks, m), dim3(256), 0, stream, x, v, n, dotbuf);
+    check(hipGetLastError(), "dot");
+    double h[kDotBlocks * kMaxDots];
+    check(hipMemcpyAsync(h, dotbuf, sizeof(double) * kDotBlocks * m, hipMemcpyDeviceToHost, stream), "dot copy");
+    check(hipStreamSynchronize(stream), "dot sync");
+    for (int q = 0; q < m; q++) {
+        double s = 0.0, c = 0.0;
+        for (int i = 0; i < kDotBlocks; i++) {
+            const double z = h[q * kDotBlocks + i], u = s + z;
+            if (std::fabs(s) >= std::fabs(z))
+                c += (s - u) + z;
+            else
+                c += (z - u) + s;
+            s = u;
+        }
+        out[q] = s + c;
+    }
 }
 
 double Engine::dot(const double *x, const double *y, int64_t n) {
-    const int nblk = 256;
-    if (!dotbuf)
-        check(hipMalloc((void **)&dotbuf, sizeof(double) * nblk), "hipMalloc dot");
-    hipLaunchKernelGGL(dot_kernel, dim3(nblk), dim3(256), 0, stream, x, y, n, dotbuf);
-    check(hipGetLastError(), "dot");
-    double h[nblk];
-    check(hipMemcpyAsync(h, dotbuf, sizeof(h), hipMemcpyDeviceToHost, stream), "dot copy");
-    check(hipStreamSynchronize(stream), "dot sync");
-    double s = 0.0, c = 0.0;
-    for (int i = 0; i < nblk; i++) {
-        const double u = s + h[i];
-        if (std::fabs(s) >= std::fabs(h[i]))
-            c += (s - u) + h[i];
-        else
-            c += (h[i] - u) + s;
-        s = u;
-    }
-    return s + c;
+    double r;
+    dots(x, &y, 1, n, &r);
+    return r;
 }
 
 Engine::~Engine() {
@@ -533,19 +693,19 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
     const int64_t O = o, Vv = v;
     DTensor tau = E.alloc({O, O, Vv, Vv});
     make_tau(E, t1, t2, tau);
-    DTensor Foo = E.alloc({O, O}, true), Fvv = E.alloc({Vv, Vv}, true), Fov = E.alloc({O, Vv}, true);
+    DTensor Foo = E.alloc({O, O}), Fvv = E.alloc({Vv, Vv}), Fov = E.alloc({O, Vv});
     E.einsum("kcld,ilcd->ki", L_ovov, &tau, Foo, 1.0, 0.0);
     E.einsum("kcld,klad->ac", L_ovov, &tau, Fvv, -1.0, 0.0);
     E.einsum("kcld,ld->kc", L_ovov, &t1, Fov, 1.0, 0.0);
 
     // -- T1 equation (RCCSD.cpp:117-138)
-    DTensor t1n = E.alloc({O, Vv}, true);
-    E.einsum("ac,ic->ia", Fvv, &t1, t1n, 1.0, 1.0);
+    DTensor t1n = E.alloc({O, Vv});
+    E.einsum("ac,ic->ia", Fvv, &t1, t1n, 1.0, 0.0);
     E.einsum("ki,ka->ia", Foo, &t1, t1n, -1.0, 1.0);
     E.einsum("kc,kica->ia", Fov, &t2, t1n, 2.0, 1.0);
     E.einsum("kc,ikca->ia", Fov, &t2, t1n, -1.0, 1.0);
     {
-        DTensor Fov_t1 = E.alloc({O, O}, true);
+        DTensor Fov_t1 = E.alloc({O, O});
         E.einsum("kc,ic->ki", Fov, &t1, Fov_t1, 1.0, 0.0);
         E.einsum("ki,ka->ia", Fov_t1, &t1, t1n, 1.0, 1.0);
     }
@@ -557,31 +717,29 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
     E.einsum("kcli,klac->ia", ovoo, &tau, t1n, 1.0, 1.0);
 
     // -- T2 equation
-    DTensor t2n = E.alloc({O, O, Vv, Vv}, true);
+    DTensor t2n = E.alloc({O, O, Vv, Vv});
+    E.axpby(t2n.p, oovv_phys.p, t2driver.p, 1.0, 1.0, t2n.size());  // (no driver: a copy)
     {
         // tmp2(a,b,i,c) = -kibc,ka + (ia|cb); abic,jc->ijab, without forming the o v^3 tmp2:
         //   sum_c (ia|cb) t_j^c  and  -sum_k t_k^a sum_c (ki|bc) t_j^c
-        DTensor X = E.alloc({O, O, Vv, Vv}, true);
+        DTensor X = E.alloc({O, O, Vv, Vv});
         E.einsum("iacb,jc->ijab", ovvv, &t1, X, 1.0, 0.0);
-        DTensor M = E.alloc({O, O, Vv, O}, true);  // M[k][i][b][j] = sum_c (ki|bc) t_j^c
+        DTensor M = E.alloc({O, O, Vv, O});  // M[k][i][b][j] = sum_c (ki|bc) t_j^c
         E.einsum("kibc,jc->kibj", oovv, &t1, M, 1.0, 0.0);
         E.einsum("kibj,ka->ijab", M, &t1, X, -1.0, 1.0);
         plus_transpose_add(E, t2n, X, 1.0);
     }
     {
         // tmp2(a,k,i,j) = kcai,jc + (ia|jk); akij,kb->ijab
-        DTensor tmp = E.alloc({Vv, O, O, O}, true);
+        DTensor tmp = E.alloc({Vv, O, O, O});
         E.einsum("kcai,jc->akij", ovvo, &t1, tmp, 1.0, 0.0);
         E.einsum("iajk->akij", ovoo, nullptr, tmp, 1.0, 1.0);
-        DTensor X = E.alloc({O, O, Vv, Vv}, true);
+        DTensor X = E.alloc({O, O, Vv, Vv});
         E.einsum("akij,kb->ijab", tmp, &t1, X, 1.0, 0.0);
         plus_transpose_add(E, t2n, X, -1.0);
     }
-    E.axpby(t2n.p, t2n.p, oovv_phys.p, 1.0, 1.0, t2n.size());
-    if (t2driver.p)
-        E.axpby(t2n.p, t2n.p, t2driver.p, 1.0, 1.0, t2n.size());
 
-    DTensor Loo = E.alloc({O, O}, true), Lvv = E.alloc({Vv, Vv}, true);
+    DTensor Loo = E.alloc({O, O}), Lvv = E.alloc({Vv, Vv});
     E.copy(Loo, Foo);
     E.einsum("lcki,lc->ki", ovoo, &t1, Loo, 2.0, 1.0);
     E.einsum("kcli,lc->ki", ovoo, &t1, Loo, -1.0, 1.0);
@@ -606,14 +764,14 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
         E.einsum("abcd,ijcd->ijab", Wvvvv, &tau, t2n, 1.0, 1.0);
     } else {
         ladder_from_factor(E, tau, t2n);
-        DTensor Z = E.alloc({O, Vv, O, O}, true);  // Z[k][a][i][j] = sum_cd (kd|ac) tau_ij^cd
+        DTensor Z = E.alloc({O, Vv, O, O});  // Z[k][a][i][j] = sum_cd (kd|ac) tau_ij^cd
         E.einsum("kdac,ijcd->kaij", ovvv, &tau, Z, 1.0, 0.0);
         E.einsum("kaij,kb->ijab", Z, &t1, t2n, -1.0, 1.0);
         // sum_cd (kc|bd) tau_ij^cd = Z[k][b][j][i] (tau_ij^cd = tau_ji^dc)
         E.einsum("kbji,ka->ijab", Z, &t1, t2n, -1.0, 1.0);
     }
     {
-        DTensor X = E.alloc({O, O, Vv, Vv}, true);
+        DTensor X = E.alloc({O, O, Vv, Vv});
         E.einsum("ac,ijcb->ijab", Lvv, &t2, X, 1.0, 0.0);
         plus_transpose_add(E, t2n, X, 1.0);
         E.einsum("ki,kjab->ijab", Loo, &t2, X, 1.0, 0.0);
@@ -629,7 +787,7 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
     E.einsum("lckd,ilad->akic", ovov, &t2, Wvoov, -0.5, 1.0);
     E.einsum("ldkc,ilad->akic", ovov, &t2, Wvoov, 1.0, 1.0);
     {
-        DTensor tmp = E.alloc({O, O, Vv, O}, true);
+        DTensor tmp = E.alloc({O, O, Vv, O});
         E.einsum("ldkc,id->lkci", ovov, &t1, tmp, 1.0, 0.0);
         E.einsum("lkci,la->akic", tmp, &t1, Wvoov, -1.0, 1.0);
     }
@@ -638,12 +796,12 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
     E.einsum("lcki,la->akci", ovoo, &t1, Wvovo, -1.0, 1.0);
     E.einsum("lckd,ilda->akci", ovov, &t2, Wvovo, -0.5, 1.0);
     {
-        DTensor tmp = E.alloc({O, Vv, O, O}, true);
+        DTensor tmp = E.alloc({O, Vv, O, O});
         E.einsum("lckd,id->lcki", ovov, &t1, tmp, 1.0, 0.0);
         E.einsum("lcki,la->akci", tmp, &t1, Wvovo, -1.0, 1.0);
     }
     {
-        DTensor X = E.alloc({O, O, Vv, Vv}, true);
+        DTensor X = E.alloc({O, O, Vv, Vv});
         E.einsum("akic,kjcb->ijab", Wvoov, &t2, X, 2.0, 0.0);
         E.einsum("akci,kjcb->ijab", Wvovo, &t2, X, -1.0, 1.0);
         plus_transpose_add(E, t2n, X, 1.0);

@@ -43,7 +43,13 @@ struct Engine {
                           const std::string &lo, const std::vector<int64_t> &odims, int64_t K);
     // C = beta C + alpha einsum(spec, A, B); B == nullptr for a pure permutation
     void einsum(const std::string &spec, const DTensor &A, const DTensor *B, DTensor &C, double alpha, double beta);
+    // one launch of a small einsum (labels lk summed), see contract_kernel
+    void contract(const std::string &la, const DTensor &A, const std::string &lb, const DTensor &B, const std::string &lc,
+                  const std::string &lk, DTensor &C, double alpha, double beta);
     double dot(const double *x, const double *y, int64_t n);  // compensated, deterministic
+    // out[q] = dot(x, y[q]) for q < m <= kMaxDots, one launch and one copy
+    static constexpr int kMaxDots = 8;
+    void dots(const double *x, const double *const *y, int m, int64_t n, double *out);
 };
 
 // Resident integral blocks of SolveRCCSD_DIIS (src/Quantum/CC/RCCSD.cpp:31-44), row-major with

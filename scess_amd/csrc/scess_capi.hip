@@ -1493,6 +1493,7 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
             HIP_TRY(c, scess::ccsd_jacobi(z1.p, t2.p, S.e.p, (int)o, (int)v, c->stream));
         }
         std::vector<scess::DTensor> amps, errs;
+        double dotB[MAX_DIIS_VECS][MAX_DIIS_VECS] = {};  // products of the error vectors
         double E_last = 1.7976931348623157e308;
         bool converged = false;
         int it = 0;
@@ -1519,17 +1520,27 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
                 if ((int)errs.size() > MAX_DIIS_VECS) {
                     amps.erase(amps.begin());
                     errs.erase(errs.begin());
+                    for (int i = 0; i + 1 < MAX_DIIS_VECS; i++)
+                        for (int j = 0; j + 1 < MAX_DIIS_VECS; j++)
+                            dotB[i][j] = dotB[i + 1][j + 1];
                 }
+                // the products of the new error vector with all of them (the others are known)
+                const int n = (int)errs.size();
+                const double *ys[MAX_DIIS_VECS];
+                double d[MAX_DIIS_VECS];
+                for (int j = 0; j < n; j++)
+                    ys[j] = errs[j].p;
+                E.dots(errs[n - 1].p, ys, n, nt, d);
+                for (int j = 0; j < n; j++)
+                    dotB[n - 1][j] = dotB[j][n - 1] = d[j];
             }
             if (it >= DIIS_START) {
                 const int n = (int)errs.size();
                 std::vector<double> B((n + 1) * (n + 1), -1.0), rhs(n + 1, 0.0);
                 B[n * (n + 1) + n] = 0.0;
                 for (int i = 0; i < n; i++)
-                    for (int j = 0; j <= i; j++) {
-                        const double d = E.dot(errs[i].p, errs[j].p, nt);
-                        B[i * (n + 1) + j] = B[j * (n + 1) + i] = d;
-                    }
+                    for (int j = 0; j < n; j++)
+                        B[i * (n + 1) + j] = dotB[i][j];
                 double mx = 0.0;
                 for (int i = 0; i < n; i++)
                     for (int j = 0; j < n; j++)
@@ -1548,7 +1559,8 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
             }
             const double Ecur = S.energy(E, t1, t2);
             const double dE = std::fabs(Ecur - E_last);
-            const double rms = std::sqrt(std::max(0.0, E.dot(change.p, change.p, nt))) / std::sqrt((double)nt);
+            const int ne = (int)errs.size() - 1;  // the newest error vector is `change`
+            const double rms = std::sqrt(std::max(0.0, dotB[ne][ne])) / std::sqrt((double)nt);
             E_last = Ecur;
             res->last_dE = dE;
             res->last_rms = rms;

@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
                 if (m < g.M && n < g.N) {
                     if (g.splits == 1) {
                         double *cp = g.C + (int64_t)beta * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
-                        *cp += g.alpha * acc[x][y][r];
+                        *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
                     } else {
                         g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
                     }
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(256) void gemm_kn_kernel(GemmGroup gg) {
                             row = (int64_t)bq * g.sCb + (int64_t)(m - bq * g.mfold) * g.sCm;
                         }
                         double *cp = g.C + row + (int64_t)n * g.sCn;
-                        *cp += g.alpha * acc[x][y][r];
+                        *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
                     } else {
                         g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
                     }
@@ -617,7 +617,8 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     }
     for (; p < g.splits; p++)
         s += src[(int64_t)p * mn];
-    g.C[(int64_t)m * g.sCm + (int64_t)n * g.sCn] += g.alpha * s;
+    double *cp = g.C + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+    *cp = g.ow ? g.alpha * s : *cp + g.alpha * s;
 }
 
 // gemm_reduce_kernel for problem blockIdx.y of a group
@@ -642,7 +643,8 @@ __global__ __launch_bounds__(256) void gemm_reduce_group_kernel(GemmGroup gg) {
     }
     for (; p < g.splits; p++)
         s += src[(int64_t)p * mn];
-    g.C[(int64_t)m * g.sCm + (int64_t)n * g.sCn] += g.alpha * s;
+    double *cp = g.C + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+    *cp = g.ow ? g.alpha * s : *cp + g.alpha * s;
 }
 
 // ------------------------------------------- GEMM with K-contiguous operands
@@ -1009,7 +1011,7 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
                 if (m < g.M && n < g.N) {
                     if (g.splits == 1) {
                         double *cp = g.C + (int64_t)beta * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
-                        *cp += g.alpha * acc[x][y][r];
+                        *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
                     } else {
                         g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
                     }

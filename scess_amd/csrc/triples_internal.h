@@ -174,6 +174,7 @@ struct GemmArgs {
     double alpha;
     int splits;
     double *scratch;  // splits * M * N
+    int ow;           // C[b][m][n] is overwritten, not added to
     // products in P64 (default), P32 or PB3 on the K-contiguous path; FP64 inputs are rounded (split
     // into hi + lo bf16 for PB3) in registers, each 16-deep K chunk is summed on the MFMA in FP32
     // and added to FP64 accumulators. Other layouts always use FP64.
