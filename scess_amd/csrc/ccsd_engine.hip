@@ -31,6 +31,7 @@ struct PermArgs {
     double *out;
     double alpha, beta;    // out = beta * out + alpha * in[perm]
     int64_t n;
+    int64_t row, pitch;    // rows of `row` outputs start `pitch` apart (row 0: contiguous)
 };
 
 // Input offset of an output position: the output multi-index decomposed with 64-bit divisions. The
@@ -64,7 +65,8 @@ __global__ __launch_bounds__(256) void permute_kernel(PermArgs a) {
     PermWalk w;
     w.init(a, lin);
     const double x = a.alpha * a.in[w.off];
-    a.out[lin] = a.beta == 0.0 ? x : a.beta * a.out[lin] + x;
+    const int64_t at = a.row ? lin / a.row * a.pitch + lin % a.row : lin;
+    a.out[at] = a.beta == 0.0 ? x : a.beta * a.out[at] + x;
 }
 
 // Permute into pre-split BF16x3 rows: element (row, k) of the permuted operand (a.odims, flattened
@@ -97,6 +99,87 @@ __global__ __launch_bounds__(256) void permute_split_kernel(PermArgs a, int64_t 
     uint16_t *o = out + row * 2 * Kp + (k >> 3) * 16 + (k & 7);
     o[0] = hi;
     o[8] = lo;
+}
+
+// Packed operands of the FP64 particle-particle ladder (ladder_symmetric): over pairs c >= d (plus) and c > d (minus)
+//   tau+_ij[cd] = (tau_ij^cd + tau_ij^dc) / 2 (tau_ij^cc for c = d), i >= j,   tau-_ij[cd] = (tau_ij^cd - tau_ij^dc) / 2, i > j
+// at row i (i + 1) / 2 + j (i (i - 1) / 2 + j), column c (c + 1) / 2 + d (c (c - 1) / 2 + d). One work-group per (32 x 32
+// tile pair, ij); the transposed tile goes through LDS.
+__device__ inline int64_t tri(int64_t c) { return c * (c + 1) / 2; }
+
+// plus[d <= c] and minus[d < c] of the v x v matrix x (row pitch ld) for its tile (tc, td), tc >= td: wx (x + x^T), with
+// the diagonal wd x, and wx (x - x^T)
+__device__ inline void pack_pair(const double *x, int64_t ld, int v, int tc, int td, double wx, double wd, double *plus,
+                                 double *minus) {
+    __shared__ double up[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int r = ty; r < 32; r += 8) {  // tile (td, tc), element (d, c)
+        const int d = td * 32 + r, c = tc * 32 + tx;
+        up[r][tx] = d < v && c < v ? x[d * ld + c] : 0.0;
+    }
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8) {
+        const int c = tc * 32 + r, d = td * 32 + tx;
+        if (c >= v || d > c)
+            continue;
+        const double a = x[c * ld + d], b = up[tx][r];
+        plus[tri(c) + d] = d == c ? wd * a : wx * (a + b);
+        if (minus && d < c)
+            minus[tri(c - 1) + d] = wx * (a - b);
+    }
+}
+
+// tile pair number -> (tc, td), tc >= td
+__device__ inline void tile_pair(int t, int &tc, int &td) {
+    tc = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+    while (tri(tc + 1) <= t)
+        tc++;
+    while (tri(tc) > t)
+        tc--;
+    td = t - (int)tri(tc);
+}
+
+__global__ __launch_bounds__(256) void pack_tau_kernel(const double *tau, int o, int v, double *plus, int64_t lp,
+                                                       double *minus, int64_t lm) {
+    int tc, td, i, j;
+    tile_pair(blockIdx.x, tc, td);
+    tile_pair(blockIdx.y, i, j);
+    pack_pair(tau + ((int64_t)i * o + j) * v * v, v, v, tc, td, 0.5, 1.0, plus + (tri(i) + j) * lp,
+              i > j ? minus + (tri(i - 1) + j) * lm : nullptr);
+}
+
+// (ac|bd) +- (ad|bc) of one strip: I[(a - a0, c)][(b, d)] with nb values of b; row (a - a0) nb + b
+__global__ __launch_bounds__(256) void pack_int_kernel(const double *I, int nb, int v, double *plus, int64_t lp,
+                                                       double *minus, int64_t lm) {
+    int tc, td;
+    tile_pair(blockIdx.x, tc, td);
+    const int64_t row = blockIdx.y, al = row / nb, b = row - al * nb;
+    pack_pair(I + (al * v * nb + b) * v, (int64_t)nb * v, v, tc, td, 1.0, 1.0, plus + row * lp, minus + row * lm);
+}
+
+// R_ij^ab += R+ + R-, R_ji^ab += R+ - R- and R_ij^ba = R_ji^ab for a strip's rows (a, b <= a); one thread per (i >= j, row)
+__global__ __launch_bounds__(256) void ladder_scatter_kernel(const double *rp, const double *rm, int a0, int nb, int rows,
+                                                             int o, int v, double *R) {
+    const int row = blockIdx.x * 256 + threadIdx.x;
+    if (row >= rows)
+        return;
+    int i, j;
+    tile_pair(blockIdx.y, i, j);
+    const int al = row / nb, b = row - al * nb, a = a0 + al;
+    if (b > a)
+        return;
+    const int64_t np = tri(o), nm = tri(o - 1), vv = (int64_t)v * v;
+    const double p = rp[row * np + blockIdx.y], m = i > j ? rm[row * nm + tri(i - 1) + j] : 0.0;
+    double *x = R + ((int64_t)i * o + j) * vv, *y = R + ((int64_t)j * o + i) * vv;
+    const int64_t ab = (int64_t)a * v + b, ba = (int64_t)b * v + a;
+    x[ab] += p + m;
+    if (i != j)
+        y[ab] += p - m;
+    if (a != b) {
+        x[ba] += p - m;
+        if (i != j)
+            y[ba] += p + m;
+    }
 }
 
 // A whole einsum of a small system in one launch, straight from the operands: G lanes per output element, lane g
@@ -338,10 +421,12 @@ static PermArgs perm_args(const std::string &li, const double *in, const std::ve
 
 void Engine::permute(const std::string &li, const double *in, const std::vector<int64_t> &idims,
                      const std::string &lo, double *out, const std::vector<int64_t> &odims, double alpha,
-                     double beta) {
-    const PermArgs a = perm_args(li, in, idims, lo, out, odims, alpha, beta);
+                     double beta, int64_t row, int64_t pitch) {
+    PermArgs a = perm_args(li, in, idims, lo, out, odims, alpha, beta);
     if (a.n == 0)
         return;
+    a.row = row == pitch ? 0 : row;
+    a.pitch = pitch;
     hipLaunchKernelGGL(permute_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
     check(hipGetLastError(), "permute");
 }
@@ -439,21 +524,110 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         contract(la, A, lb, *B, lc, Lk, C, alpha, beta);
         return;
     }
-    // operands in [batch][M][K] and [batch][N][K]: FP64, or (BF16x3 products) pre-split rows of
-    // Ks = Kp / 2 eight-byte slots, written by the permute itself. An FP64 operand that has that order
-    // already is used as it is; of the orders of the summed labels, the one in which more of it is.
+    if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff || nb > 65535)
+        throw std::runtime_error("einsum " + spec + ": extent too large");
+    auto splits_of = [&](int64_t batch, int64_t m, int64_t n, int64_t k, GemmArgs &g, DTensor &scr) {
+        // few output tiles over a long K (e.g. Foo, the T1 terms): split K so that every CU has work; the partial
+        // tiles are added in split order (deterministic)
+        const int64_t e = prec == P64 ? 128 : 64, tiles = batch * ((m + e - 1) / e) * ((n + e - 1) / e);
+        if (prec == P64 ? tiles < 512 && k >= 2048 : tiles < 256 && k >= 8192)
+            g.splits = prec == P64 ? (int)std::min<int64_t>({1024 / tiles, k / 1024, 256})
+                                   : (int)std::min<int64_t>({512 / tiles, k / 2048, 256});
+        if (g.splits > 1) {
+            scr = alloc({g.splits, batch, m, n});
+            g.scratch = scr.p;
+        } else {
+            g.splits = 1;
+        }
+    };
+    // A large FP64 operand whose last label is summed is read in place when its other labels are [K1][M] or
+    // [Mo][K1][Mi] (runs of summed and free ones): rows of stride sr in K1 pieces of the last label, Mo as a batch. Only
+    // the other operand is permuted. (At o=20, v=200 a permute of the 1.28 GB (kd|ac) costs 0.7-1.8 ms, the GEMM 0.4.)
+    if (prec == P64 && nb == 1 && M > 0 && N > 0 && K > 0) {
+        auto in_place = [&](const std::string &l, const DTensor &T, const std::string &l2, const DTensor &T2,
+                            const std::string &Ln2) -> bool {
+            if (l.size() < 3 || Lk.find(l.back()) == std::string::npos || T.size() < T2.size() || T.size() < 1 << 20)
+                return false;
+            std::string part[3];  // Mo, K1, Mi
+            size_t at = 0;
+            for (size_t d = 0; d + 1 < l.size(); d++) {
+                const bool sum = Lk.find(l[d]) != std::string::npos;
+                if (sum && at == 0)
+                    at = 1;
+                else if (!sum && at == 1)
+                    at = 2;
+                else if (sum && at == 2)
+                    return false;
+                part[at] += l[d];
+            }
+            const int64_t k2 = T.dims.back(), mo = prod(part[0]), k1 = prod(part[1]), mi = prod(part[2]);
+            if (part[1].empty() || part[2].empty() || k2 < 8 || k2 % 2 || mo > 65535 || (mo > 1 && mi < 96))
+                return false;  // (a batch of few rows would leave most of a 128-row tile empty)
+            const int64_t n = prod(Ln2);
+            const std::string lo2 = Ln2 + part[1] + l.back(), lx = part[0] + part[2] + Ln2;
+            DTensor P2, X, scr;
+            const double *p2 = T2.p;
+            if (l2 != lo2) {
+                P2 = alloc({n, K});
+                permute(l2, T2.p, T2.dims, lo2, P2.p, dims_of(lo2), 1.0, 0.0);
+                p2 = P2.p;
+            }
+            const bool direct = lc == lx && (beta == 0.0 || beta == 1.0);
+            if (!direct)
+                X = alloc({mo, mi, n});
+            GemmArgs g{};
+            g.nseg = 1;
+            g.M = (int)mi;
+            g.N = (int)n;
+            g.alpha = direct ? alpha : 1.0;
+            g.ow = !direct || beta == 0.0;
+            g.splits = 1;
+            g.seg[0].K1 = (int)k1;
+            g.seg[0].K2 = (int)k2;
+            g.seg[0].A = {T.p, k2, mi * k2, 1, k1 * mi * k2};
+            g.seg[0].B = {p2, K, k2, 1, 0};
+            g.C = direct ? C.p : X.p;
+            g.sCm = n;
+            g.sCn = 1;
+            g.sCb = mi * n;
+            splits_of(mo, mi, n, K, g, scr);
+            check(launch_gemm(g, (int)mo, stream), "einsum gemm");
+            if (!direct)
+                permute(lx, X.p, dims_of(lx), lc, C.p, C.dims, alpha, beta);
+            return true;
+        };
+        if (in_place(la, A, lb, *B, Ln) || in_place(lb, *B, la, A, Lm))
+            return;
+    }
+    // operands in [batch][M][K] and [batch][N][K]: FP64 rows of an even pitch (16-byte aligned), or (BF16x3 products)
+    // pre-split rows of Ks = Kp / 2 eight-byte slots, written by the permute itself. An FP64 operand that has such
+    // rows already is used as it is, with its own order of the free labels; of the orders of the summed labels, the one
+    // in which more of it is.
     const bool split = prec == PB3 && M > 0 && N > 0 && K > 0;
-    const int64_t Ks = split ? (K + 31) / 32 * 16 : K;
-    if (!split) {
+    const int64_t Ks = split ? (K + 31) / 32 * 16 : prec == P64 ? (K + 1) / 2 * 2 : K;
+    if (prec == P64 && Ks == K) {
+        auto free_order = [&](const std::string &l, const std::string &Lf) {  // Lf in the order of l, if the batch leads
+            std::string f;
+            for (char x : l)
+                if (Lf.find(x) != std::string::npos)
+                    f += x;
+            return f;
+        };
         std::string Lk2;
         for (char x : lb)
             if (Lk.find(x) != std::string::npos)
                 Lk2 += x;
+        const std::string Lm2 = free_order(la, Lm), Ln2 = free_order(lb, Ln);
         const auto as_is = [&](const std::string &lk) {
-            return (la == Lb + Lm + lk ? A.size() : 0) + (lb == Lb + Ln + lk ? B->size() : 0);
+            return (la == Lb + Lm2 + lk ? A.size() : 0) + (lb == Lb + Ln2 + lk ? B->size() : 0);
         };
         if (as_is(Lk2) > as_is(Lk))
             Lk = Lk2;
+        // (another order of C's labels costs a permute of C, at most the operand's)
+        if (la == Lb + Lm2 + Lk && (Lm2 == Lm || A.size() >= C.size()))
+            Lm = Lm2;
+        if (lb == Lb + Ln2 + Lk && (Ln2 == Ln || B->size() >= C.size()))
+            Ln = Ln2;
     }
     // the GEMM writes (or adds to) C itself where C has the order [batch][M][N]
     const bool direct = lc == Lb + Lm + Ln && M > 0 && N > 0 && K > 0 && (beta == 0.0 || beta == 1.0);
@@ -467,14 +641,14 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         pA = Ap.p;
         pB = Bp.p;
     } else {
-        if (la != Lb + Lm + Lk) {
-            Ap = alloc({nb, M, K});
-            permute(la, A.p, A.dims, Lb + Lm + Lk, Ap.p, dims_of(Lb + Lm + Lk), 1.0, 0.0);
+        if (la != Lb + Lm + Lk || Ks != K) {
+            Ap = alloc({nb, M, Ks});
+            permute(la, A.p, A.dims, Lb + Lm + Lk, Ap.p, dims_of(Lb + Lm + Lk), 1.0, 0.0, K, Ks);
             pA = Ap.p;
         }
-        if (lb != Lb + Ln + Lk) {
-            Bp = alloc({nb, N, K});
-            permute(lb, B->p, B->dims, Lb + Ln + Lk, Bp.p, dims_of(Lb + Ln + Lk), 1.0, 0.0);
+        if (lb != Lb + Ln + Lk || Ks != K) {
+            Bp = alloc({nb, N, Ks});
+            permute(lb, B->p, B->dims, Lb + Ln + Lk, Bp.p, dims_of(Lb + Ln + Lk), 1.0, 0.0, K, Ks);
             pB = Bp.p;
         }
     }
@@ -487,7 +661,7 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         g.ow = !direct || beta == 0.0;
         g.splits = 1;
         g.seg[0].K1 = 1;
-        g.seg[0].K2 = (int)Ks;
+        g.seg[0].K2 = (int)(split ? Ks : K);
         g.seg[0].A = {pA, Ks, 0, 1, M * Ks};
         g.seg[0].B = {pB, Ks, 0, 1, N * Ks};
         g.C = direct ? C.p : Cp.p;
@@ -495,21 +669,9 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
         g.sCn = 1;
         g.sCb = M * N;
         g.prec = split ? PB3S : prec;
-        if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff || nb > 65535)
-            throw std::runtime_error("einsum " + spec + ": extent too large");
-        // few output tiles over a long K (e.g. Foo, the T1 terms): split K so that ~512 work-groups
-        // run; the partial tiles are added in split order (deterministic)
-        const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
         DTensor scr;
-        if (nb == 1 && tiles < 256 && K >= 8192) {
-            g.splits = (int)std::min<int64_t>({512 / tiles, K / 2048, 256});
-            if (g.splits > 1) {
-                scr = alloc({g.splits, M, N});
-                g.scratch = scr.p;
-            } else {
-                g.splits = 1;
-            }
-        }
+        if (nb == 1)
+            splits_of(1, M, N, K, g, scr);
         check(launch_gemm(g, (int)nb, stream), "einsum gemm");
     }
     if (!direct)
@@ -653,7 +815,7 @@ void CcsdState::ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R) {
                 g.seg[0].A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};  // rows (a, c), K = P contiguous
                 g.seg[0].B = {Lvv.p + b0 * v * nP, nP, 0, 1, 0};
             }
-            check(hipMemsetAsync(I.p, 0, sizeof(double) * (size_t)I.size(), E.stream), "memset I");
+            g.ow = 1;
             g.C = I.p;
             g.prec = split ? PB3S : E.prec;
             g.sCm = tb * v;
@@ -686,6 +848,85 @@ void CcsdState::ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R) {
             h.sCn = v * v;
             check(launch_gemm(h, (int)ta, E.stream), "ladder contraction");
         }
+    }
+}
+
+// The same ladder in FP64 at less than a third of the products. R_ij^ab = R_ji^ba (tau_ij^cd = tau_ji^dc), so only b <= a
+// is regenerated and contracted, in strips of TA values of a; and with s+- = (ac|bd) +- (ad|bc) and tau+- (pack_tau_kernel)
+//   R_ij^ab = sum_{c>=d} s+ tau+ + sum_{c>d} s- tau-,   R_ji^ab = the same with minus,
+// so the sum over (c, d) and the pairs (i, j) halve: o^2 v^4 / 4 products for the contraction and naux v^4 / 2 for the
+// integrals. Bound by the GEMMs' matrix pipes; the packing passes read a strip's integrals and write them once.
+void CcsdState::ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R) {
+    const int64_t nP = naux, pp = v * (v + 1) / 2, pm = v * (v - 1) / 2, np = o * (o + 1) / 2, nm = o * (o - 1) / 2;
+    const int64_t lp = (pp + 1) / 2 * 2, lm = std::max<int64_t>((pm + 1) / 2 * 2, 2);  // 16-byte rows
+    // strips of at most 32 a and 512 MiB of integrals, of even width (their diagonal blocks are half wasted: 8 of 200 a
+    // cost 52% of the full square, 32 cost 58%)
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(32, ((int64_t)512 << 20) / (8 * v * v * v)));
+    const int64_t strips = (v + most - 1) / most;
+    const int64_t TA = (v + strips - 1) / strips, nt = (v + 31) / 32;
+    const unsigned tp = (unsigned)(nt * (nt + 1) / 2);
+    DTensor tp_ = E.alloc({np, lp}), tm_ = E.alloc({std::max<int64_t>(nm, 1), lm});
+    hipLaunchKernelGGL(pack_tau_kernel, dim3(tp, (unsigned)np), dim3(256), 0, E.stream, tau.p, (int)o, (int)v, tp_.p, lp,
+                       tm_.p, lm);
+    check(hipGetLastError(), "pack tau");
+    DTensor I = E.alloc({TA, v, v, v}), sp = E.alloc({TA * v, lp}), sm = E.alloc({TA * v, lm});
+    DTensor rp = E.alloc({TA * v, np}), rm = E.alloc({TA * v, std::max<int64_t>(nm, 1)});
+    for (int64_t a0 = 0; a0 < v; a0 += TA) {
+        const int64_t ta = std::min(TA, v - a0), nb = a0 + ta, rows = ta * nb;
+        // I[(a,c)][(b,d)] = sum_P L[a][c][P] L[b][d][P], b < a0 + ta
+        GemmArgs g{};
+        g.nseg = 1;
+        g.M = (int)(ta * v);
+        g.N = (int)(nb * v);
+        g.alpha = 1.0;
+        g.splits = 1;
+        g.seg[0].K1 = 1;
+        g.seg[0].K2 = (int)nP;
+        g.seg[0].A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};
+        g.seg[0].B = {Lvv.p, nP, 0, 1, 0};
+        g.C = I.p;
+        g.sCm = nb * v;
+        g.sCn = 1;
+        g.ow = 1;
+        check(launch_gemm(g, 1, E.stream), "ladder integrals");
+        hipLaunchKernelGGL(pack_int_kernel, dim3(tp, (unsigned)rows), dim3(256), 0, E.stream, I.p, (int)nb, (int)v, sp.p, lp,
+                           sm.p, lm);
+        check(hipGetLastError(), "pack integrals");
+        auto contract = [&](const DTensor &S, const DTensor &T, int64_t ld, int64_t K, int64_t N, DTensor &out) {
+            if (K < 1 || N < 1)
+                return;
+            GemmArgs h{};
+            h.nseg = 1;
+            h.M = (int)rows;
+            h.N = (int)N;
+            h.alpha = 1.0;
+            h.splits = 1;
+            h.seg[0].K1 = 1;
+            h.seg[0].K2 = (int)K;
+            h.seg[0].A = {S.p, ld, 0, 1, 0};
+            h.seg[0].B = {T.p, ld, 0, 1, 0};
+            h.C = out.p;
+            h.sCm = N;
+            h.sCn = 1;
+            h.ow = 1;
+            const int64_t tiles = ((rows + 127) / 128) * ((N + 127) / 128);
+            DTensor scr;
+            if (tiles < 512 && K >= 2048) {  // two work-groups per CU
+                h.splits = (int)std::max<int64_t>(1, std::min<int64_t>({1024 / tiles, K / 1024, 32}));
+                if (h.splits > 1) {
+                    scr = E.alloc({h.splits, rows, N});
+                    h.scratch = scr.p;
+                }
+            }
+            check(launch_gemm(h, 1, E.stream), "ladder contraction");
+        };
+        contract(sp, tp_, lp, pp, np, rp);
+        contract(sm, tm_, lm, pm, nm, rm);
+        if (pm == 0 && nm > 0)
+            check(hipMemsetAsync(rm.p, 0, sizeof(double) * (size_t)rm.size(), E.stream), "memset R-");
+        hipLaunchKernelGGL(ladder_scatter_kernel, dim3((unsigned)((rows + 255) / 256), (unsigned)np), dim3(256), 0, E.stream,
+                           rp.p, rm.p, (int)a0, (int)nb, (int)rows, (int)o, (int)v, R.p);
+        check(hipGetLastError(), "ladder scatter");
     }
 }
 
@@ -763,7 +1004,10 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
         E.einsum("kcbd,ka->abcd", ovvv, &t1, Wvvvv, -1.0, 1.0);
         E.einsum("abcd,ijcd->ijab", Wvvvv, &tau, t2n, 1.0, 1.0);
     } else {
-        ladder_from_factor(E, tau, t2n);
+        if (E.prec == P64 && O * (O + 1) / 2 <= 65535)  // (pairs are a grid dimension)
+            ladder_symmetric(E, tau, t2n);
+        else  // (its rounding is kept: packing would split and round other values)
+            ladder_from_factor(E, tau, t2n);
         DTensor Z = E.alloc({O, Vv, O, O});  // Z[k][a][i][j] = sum_cd (kd|ac) tau_ij^cd
         E.einsum("kdac,ijcd->kaij", ovvv, &tau, Z, 1.0, 0.0);
         E.einsum("kaij,kb->ijab", Z, &t1, t2n, -1.0, 1.0);

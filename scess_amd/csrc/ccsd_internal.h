@@ -36,7 +36,8 @@ struct Engine {
     void copy(DTensor &dst, const DTensor &src);
     void axpby(double *out, const double *x, const double *y, double alpha, double beta, int64_t n);
     void permute(const std::string &li, const double *in, const std::vector<int64_t> &idims, const std::string &lo,
-                 double *out, const std::vector<int64_t> &odims, double alpha, double beta);
+                 double *out, const std::vector<int64_t> &odims, double alpha, double beta, int64_t row = 0,
+                 int64_t pitch = 0);  // rows of `row` outputs `pitch` apart (0: contiguous)
     // the permutation of `in` (labels li -> lo, output dims odims) written as pre-split BF16x3 rows of its
     // last K elements (rows padded to a multiple of 32 k); returned as rows x Kp/2 eight-byte slots
     DTensor permute_split(const std::string &li, const double *in, const std::vector<int64_t> &idims,
@@ -56,11 +57,12 @@ struct Engine {
 // the reference's index order, plus the optional Cholesky factor of (ac|bd).
 struct CcsdState {
     bool have = false;
-    int64_t o = 0, v = 0, naux = 0;
+    int64_t o = 0, v = 0, naux = 0;  // naux: pitch of the rows of Lvv (even, zero padded)
     DTensor ovov, oovv, ovvo, ovvv, ovoo, oooo_phys, vvvv_phys, oovv_phys, L_oovv_phys, L_ovov, Lvv, e;
     DTensor t2driver, f12energy;
     void make_tau(Engine &E, const DTensor &t1, const DTensor &t2, DTensor &tau);
     void ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R);
+    void ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R);
     void update(Engine &E, DTensor &t1, DTensor &t2);  // one Jacobi update (UpdateAmplitudes)
     double energy(Engine &E, const DTensor &t1, const DTensor &t2);
 };

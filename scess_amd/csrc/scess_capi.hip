@@ -1359,9 +1359,16 @@ int scess_ccsd_set_inputs(scess_ctx *c, const scess_ccsd_in *in) {
             S.vvvv_phys = E.alloc({v, v, v, v});
             E.einsum("acbd->abcd", vvvv, nullptr, S.vvvv_phys, 1.0, 0.0);
         } else {
-            S.naux = in->naux;
-            // kept as [a][c][P]: the ladder's tile regeneration contracts over the contiguous P
+            // kept as [a][c][P]: the ladder's tile regeneration contracts over the contiguous P; rows of an even
+            // length (a zero more for an odd naux), so that they are 16-byte aligned
+            S.naux = (in->naux + 1) / 2 * 2;
             S.Lvv = upload_colmajor(E, in->chol_vv, {v, v, in->naux});
+            if (S.naux != in->naux) {
+                scess::DTensor padded = E.alloc({v, v, S.naux}, true);
+                HIP_TRY(c, hipMemcpy2DAsync(padded.p, 8 * S.naux, S.Lvv.p, 8 * in->naux, 8 * in->naux, v * v,
+                                            hipMemcpyDeviceToDevice, c->stream));
+                S.Lvv = std::move(padded);
+            }
         }
         S.e = E.alloc({o + v});
         E.upload(S.e, in->e);

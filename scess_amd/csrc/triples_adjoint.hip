@@ -597,13 +597,14 @@ __global__ __launch_bounds__(256) void gemm_kn_kernel(GemmGroup gg) {
         }
 }
 
+// (blockIdx.y: batch entry; only gemm_nt_kernel has more than one)
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (int64_t)g.M * g.N)
         return;
     const int m = (int)(idx / g.N), n = (int)(idx - (int64_t)m * g.N);
-    const int64_t mn = (int64_t)g.M * g.N;
-    const double *src = g.scratch + idx;
+    const int64_t mn = (int64_t)g.M * g.N * gridDim.y;
+    const double *src = g.scratch + (int64_t)blockIdx.y * g.M * g.N + idx;
     double s = 0.0;
     int p = 0;
     for (; p + 8 <= g.splits; p += 8) {  // eight loads in flight, added in split order
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     }
     for (; p < g.splits; p++)
         s += src[(int64_t)p * mn];
-    double *cp = g.C + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+    double *cp = g.C + (int64_t)blockIdx.y * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
     *cp = g.ow ? g.alpha * s : *cp + g.alpha * s;
 }
 
@@ -1020,6 +1021,245 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
         }
 }
 
+// ------------------------------------------- FP64 GEMM with K-contiguous operands
+// The same contraction for one segment of FP64 products whose rows are 16-byte aligned. Four waves own the quadrants of
+// a tile of up to 128 x 128, two work-groups fill a CU (64 KiB of LDS, 256 registers). The ceil(M / 16) blocks of the
+// rows are dealt out evenly over ceil(M / 128) tiles and a tile's blocks over its two halves, the columns alike, so no
+// tile or wave is nearly empty (N = 400: 7 + 6 + 6 + 6 blocks; the 64 x 128 tiles of gemm_kc_kernel ran 3.1 tiles as 4).
+// The loop is that of the FP64 W-build: bound by the matrix pipes, fragments read one k-step (4 of a chunk's 16 k) ahead
+// of their MFMAs, one barrier per chunk before its last step, after which the freed stage takes the loads of the chunk
+// after the next; the last chunk of a row runs only the k-steps that exist, its k past K2 set to zero in registers.
+template <int RB, int CB> struct GemmNT {
+    // state shared with the kernel
+    const GemmArgs &g;
+    char *lds;
+    int lane, wave, wr, wc, m0, n0, rb, cb, beta, split;
+    uint32_t so[4];
+    uint32_t oa[4], ob[4];
+    const double *pa, *pb;   // operand rows m0, n0 at the next chunk to load
+    int k2c, nk2, left;      // its place in the row, chunks of a row, chunks left to load
+
+    static constexpr int OPB = 128 * 128;  // bytes of an operand's stage
+
+    // the next chunk into stage st: returns its k-steps, with bit 3 set when the last is partly past K2 (the lane
+    // offsets of its vectors were clamped into the row)
+    __device__ inline int issue(int st) {
+        char *base = lds + st * 2 * OPB;
+        const int rem = k2c == nk2 - 1 ? g.seg[0].K2 - 16 * k2c : 16;
+        const int last = (rem - 1) & ~1;  // first k of the last vector of the row
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            const int u = wave + 4 * h, hf = u >> 3, bl = (u >> 1) & 3;  // LDS rows 8 u .. 8 u + 7: block bl of half hf
+            const int r = 8 * (u & 7) + (lane >> 3), k = min(2 * ((lane & 7) ^ kswz(r)), last);
+            if (bl < (rb + 1 - hf) >> 1)
+                __builtin_amdgcn_global_load_lds((const void *)((const char *)pa + oa[h] + 8 * k),
+                                                 (lds_void *)(base + u * 1024), 16, 0, 0);
+            if (bl < (cb + 1 - hf) >> 1)
+                __builtin_amdgcn_global_load_lds((const void *)((const char *)pb + ob[h] + 8 * k),
+                                                 (lds_void *)(base + OPB + u * 1024), 16, 0, 0);
+        }
+        pa += 16;
+        pb += 16;
+        if (++k2c == nk2) {
+            k2c = 0;
+            pa += g.seg[0].A.s1 - 16 * nk2;
+            pb += g.seg[0].B.s1 - 16 * nk2;
+        }
+        left--;
+        return (rem + 3) >> 2 | (rem & 3 ? 8 : 0);
+    }
+
+    __device__ inline void run(int total, int cur, int nxt) {
+        d4 acc[RB][CB];
+        double fr[2][RB], fc[2][CB];
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = d4{};
+        lds_char *qa, *qb;
+        auto tiles = [&](int st) {
+            qa = (lds_char *)lds + st * 2 * OPB + wr * (OPB / 2);
+            qb = (lds_char *)lds + st * 2 * OPB + OPB + wc * (OPB / 2);
+        };
+        auto read = [&](auto tc, int buf) {
+            constexpr int t = decltype(tc)::value;
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+                fr[buf][x] = *(lds_double *)(qa + so[t ^ x] + x * 2048);
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[buf][y] = *(lds_double *)(qb + so[t ^ y] + y * 2048);
+        };
+        auto row = [&](int buf, int x) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[buf][x], fc[buf][y], acc[x][y], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // a k-step, with the fragments of the next one (t) read into the other buffer after its first row
+        auto step = [&](int buf, auto tc) {
+            row(buf, 0);
+            read(tc, buf ^ 1);
+#pragma unroll
+            for (int x = 1; x < RB; x++)
+                row(buf, x);
+        };
+        auto move = [&]() {  // buffer 0 to buffer 1
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+                fr[1][x] = fr[0][x];
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[1][y] = fc[0][y];
+        };
+        using std::integral_constant;
+        const int lq = lane >> 4, keep = g.seg[0].K2 & 3;
+        wait_vm_lgkm0();
+        __syncthreads();
+        tiles(0);
+        read(integral_constant<int, 0>{}, 0);
+        for (int c = 0; c < total; c++) {
+            // all k-steps of chunk c but its last, whose fragments end up in buffer 1
+            const int steps = cur & 7;
+            if (steps >= 2) {
+                step(0, integral_constant<int, 1>{});
+                if (steps >= 3) {
+                    step(1, integral_constant<int, 2>{});
+                    if (steps == 4)
+                        step(0, integral_constant<int, 3>{});
+                    else
+                        move();
+                }
+            } else {
+                move();
+            }
+            const bool more = c + 1 < total;
+            if (more) {
+                // chunk c + 1, in flight since the last step of chunk c - 1, and this wave's reads of this stage
+                wait_vm_lgkm0();
+                __syncthreads();
+            }
+            if (cur & 8) {  // k past K2
+#pragma unroll
+                for (int x = 0; x < RB; x++)
+                    fr[1][x] = lq < keep ? fr[1][x] : 0.0;
+#pragma unroll
+                for (int y = 0; y < CB; y++)
+                    fc[1][y] = lq < keep ? fc[1][y] : 0.0;
+            }
+            row(1, 0);
+            if (more) {
+                tiles((c + 1) & 1);
+                read(integral_constant<int, 0>{}, 0);
+            }
+            cur = nxt;
+            if (left > 0)
+                nxt = issue(c & 1);
+#pragma unroll
+            for (int x = 1; x < RB; x++)
+                row(1, x);
+        }
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // keeps the store addresses from being formed, and held, before the loop
+        const int lr = ln & 15, lqs = ln >> 4;
+        const int mw = m0 + wr * 16 * ((rb + 1) >> 1), nw = n0 + wc * 16 * ((cb + 1) >> 1);
+        const int mend = min(g.M, m0 + 16 * rb), nend = min(g.N, n0 + 16 * cb);
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = mw + x * 16 + lqs + 4 * r;
+#pragma unroll
+                for (int y = 0; y < CB; y++) {
+                    const int n = nw + y * 16 + lr;
+                    if (m < mend && n < nend) {
+                        if (g.splits == 1) {
+                            double *cp = g.C + (int64_t)beta * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+                            *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
+                        } else {
+                            g.scratch[(((int64_t)split * gridDim.y + beta) * g.M + m) * g.N + n] = acc[x][y][r];
+                        }
+                    }
+                }
+            }
+    }
+};
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_nt_kernel(GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) char lds[4 * 128 * 128];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nbm = (g.M + 15) >> 4, nbn = (g.N + 15) >> 4, ntm = (nbm + 7) >> 3, ntn = (nbn + 7) >> 3;
+    // tiles of one (batch, split) on one XCD, so the tiles sharing an operand panel share its L2
+    const int nx = gridDim.x, ny = gridDim.y;
+    const int lin = xcd_remap(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z), nx * ny * gridDim.z);
+    const int bx = lin % nx, byz = lin / nx;
+    const int tm = bx / ntn, tn = bx - tm * ntn;
+    const int beta = byz % ny, split = byz / ny;
+    const int am = (int)((int64_t)tm * nbm / ntm), an = (int)((int64_t)tn * nbn / ntn);
+    const int rb = (int)((int64_t)(tm + 1) * nbm / ntm) - am, cb = (int)((int64_t)(tn + 1) * nbn / ntn) - an;
+    const int quad = wave ^ (lin & 3);  // the uneven quadrants of neighbouring tiles on different SIMDs
+    const int nk2 = (g.seg[0].K2 + 15) >> 4, total = g.seg[0].K1 * nk2;
+    const int c_begin = (int)((int64_t)total * split / g.splits), c_end = (int)((int64_t)total * (split + 1) / g.splits);
+    const int k1 = c_begin / nk2, k2c = c_begin - k1 * nk2;
+    const int nr = (rb + 1 - (quad >> 1)) >> 1, nc = (cb + 1 - (quad & 1)) >> 1;  // blocks of this wave's quadrant
+    // Every wave passes the same barriers, one per chunk, whatever the form of its quadrant. A quadrant without
+    // blocks (a tile of one block row or column) runs as one block whose results lie past the tile, and are not stored.
+    auto go = [&](auto rbc, auto cbc) {
+        GemmNT<decltype(rbc)::value, decltype(cbc)::value> w{g, lds};
+        w.lane = lane;
+        w.wave = wave;
+        w.wr = quad >> 1;
+        w.wc = quad & 1;
+        w.m0 = 16 * am;
+        w.n0 = 16 * an;
+        w.rb = rb;
+        w.cb = cb;
+        w.beta = beta;
+        w.split = split;
+        w.k2c = k2c;
+        w.nk2 = nk2;
+        w.left = c_end - c_begin;
+        const GemmOp &A = g.seg[0].A, &B = g.seg[0].B;
+        w.pa = A.base + (int64_t)beta * A.sb + (int64_t)k1 * A.s1 + 16 * k2c + (int64_t)w.m0 * A.sr;
+        w.pb = B.base + (int64_t)beta * B.sb + (int64_t)k1 * B.s1 + 16 * k2c + (int64_t)w.n0 * B.sr;
+        const int lr = lane & 15, lq = lane >> 4;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            w.so[u] = lr * 128 + ((2 * u + (lq >> 1)) ^ kswz(lr)) * 16 + (lq & 1) * 8;
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            // rows past M (N) load the last one
+            const int u = wave + 4 * h, hf = u >> 3, r = 8 * (u & 7) + (lane >> 3);
+            w.oa[h] = (uint32_t)min(r + hf * 16 * ((rb + 1) >> 1), g.M - 1 - w.m0) * (uint32_t)(8 * A.sr);
+            w.ob[h] = (uint32_t)min(r + hf * 16 * ((cb + 1) >> 1), g.N - 1 - w.n0) * (uint32_t)(8 * B.sr);
+        }
+        const int run_total = w.left;
+        if (run_total == 0) {  // a split without chunks: zero partials
+            w.run(0, 0, 0);
+            return;
+        }
+        const int i0 = w.issue(0), i1 = w.left > 0 ? w.issue(1) : 0;
+        w.run(run_total, i0, i1);
+    };
+    using std::integral_constant;
+    auto cols = [&](auto rbc) {
+        switch (nc) {
+        case 4: go(rbc, integral_constant<int, 4>{}); break;
+        case 3: go(rbc, integral_constant<int, 3>{}); break;
+        case 2: go(rbc, integral_constant<int, 2>{}); break;
+        default: go(rbc, integral_constant<int, 1>{}); break;
+        }
+    };
+    switch (nr) {
+    case 4: cols(integral_constant<int, 4>{}); break;
+    case 3: cols(integral_constant<int, 3>{}); break;
+    case 2: cols(integral_constant<int, 2>{}); break;
+    default: cols(integral_constant<int, 1>{}); break;
+    }
+}
+
 // 0: not K-contiguous; 1: K-contiguous; 2: K-contiguous with 16-byte aligned rows (vector loads)
 static int k_contiguous(const GemmArgs &g) {
     int r = 2;
@@ -1089,6 +1329,17 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
             return hipErrorInvalidValue;
     }
     if (const int kc = k_contiguous(g)) {
+        // FP64: 128 x 128 tiles; rows of a tile at lane offsets of 32 bits
+        const GemmSeg &s0 = g.seg[0];
+        const double far = 128.0 * 8.0 * (double)std::max(s0.A.sr, s0.B.sr);
+        if (g.prec == P64 && kc == 2 && g.nseg == 1 && s0.K2 >= 1 && s0.K1 >= 1 && g.M >= 1 && g.N >= 1 &&
+            s0.A.sr >= 0 && s0.B.sr >= 0 && far < 4294967296.0) {
+            const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+            if (tiles > 0x7fffffff)
+                return hipErrorInvalidValue;
+            hipLaunchKernelGGL(gemm_nt_kernel, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256), 0, s,
+                               g);
+        } else {
         // 64x64 tiles: for FP64 MFMA more resident work-groups beat larger register tiles
         int blk = 2;
         if (const char *e = std::getenv("SCESS_GEMM_BLK"))  // tuning override: 2 or 4 (FP64 only)
@@ -1126,6 +1377,7 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
         SCESS_KC(4, true, P64, false) SCESS_KC(4, false, P64, false)
         return hipErrorInvalidValue;
 #undef SCESS_KC
+        }
     } else if (kn_modes(g)) {
         GemmGroup gg;
         gg.g[0] = g;
@@ -1151,7 +1403,7 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
     if (e != hipSuccess || g.splits == 1)
         return e;
     const int64_t n = (int64_t)g.M * g.N;
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 

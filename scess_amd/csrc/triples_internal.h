@@ -173,7 +173,7 @@ struct GemmArgs {
     int64_t sCm, sCn, sCb;
     double alpha;
     int splits;
-    double *scratch;  // splits * M * N
+    double *scratch;  // splits * M * N (times the batch for K-contiguous FP64 operands)
     int ow;           // C[b][m][n] is overwritten, not added to
     // products in P64 (default), P32 or PB3 on the K-contiguous path; FP64 inputs are rounded (split
     // into hi + lo bf16 for PB3) in registers, each 16-deep K chunk is summed on the MFMA in FP32
