@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libscess_gpu.so")
 CLI = os.path.join(HERE, "scess_cc")
 CPP_CHECK = os.path.join(ROOT, "tests", "cpp", "triples_function_check")
 SO_CHECK = os.path.join(ROOT, "tests", "cpp", "spin_orbital_check")
-SOURCES = ["triples_kernels.hip", "triples_adjoint.hip", "ccsd_engine.hip", "scess_capi.hip", "cc_api.cpp",
+SOURCES = ["triples_kernels.hip", "triples_adjoint.hip", "ccsd_engine.hip", "scess_capi.hip", "buffers.cpp", "cc_api.cpp",
            "scf_host.cpp", "spin_orbital_cc.cpp", "regression.cpp"]
 ARCH = "gfx950"
 

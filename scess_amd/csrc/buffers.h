@@ -1,0 +1,44 @@
+// Device blocks kept by a context between calls, and copies between pageable host memory and the device.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <vector>
+
+namespace scess {
+
+// Device memory of one context: freed blocks are kept, up to kMaxCached bytes in all, and handed out again; the rest goes
+// back to the runtime, and everything at the end of the context. Stream ordered: a block is reused by work on the same
+// stream (or ordered after it). A call's dozens of allocations otherwise cost more than its kernels for small systems,
+// and the mapping of freshly allocated memory some milliseconds per GiB for large ones.
+class BlockCache {
+public:
+    static constexpr size_t kMaxCached = (size_t)6 << 30;
+    ~BlockCache() { flush(); }
+    hipError_t get(void **p, size_t bytes, hipStream_t s);
+    void put(void *p);  // null is allowed
+    void flush();
+
+private:
+    struct Block {
+        void *p;
+        size_t bytes;
+        hipStream_t s;
+    };
+    std::vector<Block> free_, used_;
+    size_t cached_ = 0;
+};
+
+// Copies of any size between pageable host memory and the device, ordered on stream s as hipMemcpyAsync would be. Large
+// ones go through a ring of pinned chunks shared by the process, filled or emptied by a few threads: one thread's
+// memcpy (and its page faults in a new array) runs at 5-13 GB/s, the link at 50 (gradients of o=20, v=200 to the host,
+// 1.6 GB: 100 ms -> 30; transform of 58 functions, 91 MB each way: 14.7 -> 9.6). copy_to_host returns when the data is
+// there; copy_to_device when `h` has been read.
+hipError_t copy_to_host(void *h, const void *d, size_t bytes, hipStream_t s);
+hipError_t copy_to_device(void *d, const void *h, size_t bytes, hipStream_t s);
+// The ring and its threads exist while a context does
+void copies_retain();
+void copies_release();
+
+}  // namespace scess

@@ -331,18 +331,18 @@ DTensor::~DTensor() { release(); }
 
 void DTensor::release() {
     if (p)
-        (void)hipFreeAsync(p, s);
+        home->put(p);
     p = nullptr;
 }
 
-DTensor::DTensor(DTensor &&o) noexcept : p(o.p), dims(std::move(o.dims)), s(o.s) { o.p = nullptr; }
+DTensor::DTensor(DTensor &&o) noexcept : p(o.p), dims(std::move(o.dims)), home(o.home) { o.p = nullptr; }
 
 DTensor &DTensor::operator=(DTensor &&o) noexcept {
     if (this != &o) {
         release();
         p = o.p;
         dims = std::move(o.dims);
-        s = o.s;
+        home = o.home;
         o.p = nullptr;
     }
     return *this;
@@ -363,21 +363,20 @@ static void check(hipError_t e, const char *what) {
 DTensor Engine::alloc(std::vector<int64_t> dims, bool zero) {
     DTensor t;
     t.dims = std::move(dims);
-    t.s = stream;
+    t.home = blocks;
     const size_t bytes = sizeof(double) * (size_t)std::max<int64_t>(t.size(), 1);
-    check(hipMallocAsync((void **)&t.p, bytes, stream), "hipMallocAsync (CCSD tensor)");
+    check(blocks->get((void **)&t.p, bytes, stream), "device allocation (CCSD tensor)");
     if (zero)
         check(hipMemsetAsync(t.p, 0, bytes, stream), "hipMemsetAsync");
     return t;
 }
 
 void Engine::upload(DTensor &t, const double *host) {
-    check(hipMemcpyAsync(t.p, host, sizeof(double) * (size_t)t.size(), hipMemcpyHostToDevice, stream), "upload");
+    check(copy_to_device(t.p, host, sizeof(double) * (size_t)t.size(), stream), "upload");
 }
 
 void Engine::download(const DTensor &t, double *host) {
-    check(hipMemcpyAsync(host, t.p, sizeof(double) * (size_t)t.size(), hipMemcpyDeviceToHost, stream), "download");
-    check(hipStreamSynchronize(stream), "download sync");
+    check(copy_to_host(host, t.p, sizeof(double) * (size_t)t.size(), stream), "download");
 }
 
 void Engine::copy(DTensor &dst, const DTensor &src) {

@@ -1,6 +1,7 @@
 // Device tensors, the einsum engine and the closed-shell CCSD state.
 #pragma once
 
+#include "buffers.h"
 #include "triples_internal.h"
 
 #include <cstdint>
@@ -13,7 +14,7 @@ namespace scess {
 struct DTensor {
     double *p = nullptr;
     std::vector<int64_t> dims;
-    hipStream_t s = nullptr;  // stream-ordered allocation (hipMallocAsync / hipFreeAsync)
+    BlockCache *home = nullptr;  // where the allocation goes back to
     DTensor() = default;
     DTensor(const DTensor &) = delete;
     DTensor &operator=(const DTensor &) = delete;
@@ -27,6 +28,7 @@ struct DTensor {
 // Stream-ordered tensor operations; errors are thrown as std::runtime_error.
 struct Engine {
     hipStream_t stream = nullptr;
+    BlockCache *blocks = nullptr;  // of the context; outlives every tensor
     double *dotbuf = nullptr;
     int prec = 0;  // product precision of the einsum contractions (P64, P32, PB3), see GemmArgs::prec
     ~Engine();

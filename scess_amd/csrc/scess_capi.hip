@@ -56,6 +56,7 @@ struct scess_ctx {
     int ccsd_prec = 0;               // product precision of the CCSD residual contractions
     void *scratch = nullptr;         // this device's address of the static scratch array
     int int8_digits = kI8DefaultDigits;  // digits per element of SCESS_PREC_OZAKI (next scess_t_set_inputs)
+    scess::BlockCache blocks;        // device memory of t and of the engine's tensors
     TriplesState t;
     scess::Engine eng;
     scess::CcsdState cc;
@@ -88,44 +89,49 @@ int hip_fail(scess_ctx *c, hipError_t e, const char *what) {
             return hip_fail((c), e__, #expr);             \
     } while (0)
 
+// Blocks go back to the context's cache; nothing on the device uses them any more
 template <class T>
-void dfree(T *&p) {
-    if (p) {
-        (void)hipFree((void *)p);
-        p = nullptr;
-    }
+void dfree(scess_ctx *c, T *&p) {
+    c->blocks.put((void *)p);
+    p = nullptr;
 }
 
-void free_triples(TriplesState &t) {
+template <class T>
+hipError_t dmalloc(scess_ctx *c, T **p, size_t bytes) {
+    return c->blocks.get((void **)p, bytes, c->stream);
+}
+
+void free_triples(scess_ctx *c) {
+    TriplesState &t = c->t;
     for (auto &op : t.ops) {
-        dfree(op.X);
-        dfree(op.T);
-        dfree(op.Rn);
-        dfree(op.TM);
+        dfree(c, op.X);
+        dfree(c, op.T);
+        dfree(c, op.Rn);
+        dfree(c, op.TM);
         op = Operands{};
     }
-    dfree(t.S);
-    dfree(t.t1);
-    dfree(t.e);
-    dfree(t.ev);
-    dfree(t.d_ijk_all);
-    dfree(t.d_orbits);
-    dfree(t.d_orbtab);
-    dfree(t.W1);
-    dfree(t.W2);
-    dfree(t.d_work_ijk);
-    dfree(t.d_work_index);
-    dfree(t.partials);
-    dfree(t.U);
-    dfree(t.F);
-    dfree(t.E);
-    dfree(t.queue);
+    dfree(c, t.S);
+    dfree(c, t.t1);
+    dfree(c, t.e);
+    dfree(c, t.ev);
+    dfree(c, t.d_ijk_all);
+    dfree(c, t.d_orbits);
+    dfree(c, t.d_orbtab);
+    dfree(c, t.W1);
+    dfree(c, t.W2);
+    dfree(c, t.d_work_ijk);
+    dfree(c, t.d_work_index);
+    dfree(c, t.partials);
+    dfree(c, t.U);
+    dfree(c, t.F);
+    dfree(c, t.E);
+    dfree(c, t.queue);
     t = TriplesState{};
 }
 
 int upload(scess_ctx *c, const double *h, size_t n, double **d) {
-    HIP_TRY(c, hipMalloc((void **)d, sizeof(double) * std::max<size_t>(n, 1)));
-    HIP_TRY(c, hipMemcpyAsync(*d, h, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, dmalloc(c, d, sizeof(double) * std::max<size_t>(n, 1)));
+    HIP_TRY(c, scess::copy_to_device(*d, h, sizeof(double) * n, c->stream));
     return SCESS_OK;
 }
 
@@ -181,12 +187,14 @@ int scess_create(scess_ctx **out, int device) {
         return SCESS_ERR_HIP;
     }
     c->eng.stream = c->stream;
+    c->eng.blocks = &c->blocks;
     if (scratch_address(device, &c->scratch) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         (void)hipStreamDestroy(c->stream2);
         delete c;
         return SCESS_ERR_HIP;
     }
+    scess::copies_retain();
     *out = c;
     return SCESS_OK;
 }
@@ -196,12 +204,14 @@ void scess_destroy(scess_ctx *c) {
         return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    free_triples(c->t);
+    free_triples(c);
     c->cc = scess::CcsdState{};
+    c->blocks.flush();
     (void)hipStreamSynchronize(c->stream);
     (void)hipStreamSynchronize(c->stream2);
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->stream2);
+    scess::copies_release();
     delete c;
 }
 
@@ -256,7 +266,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
         return fail(c, SCESS_ERR_ARG, "scess_t_set_inputs: prec_mask must be a non-empty subset of bits 0..3");
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    free_triples(c->t);
+    free_triples(c);
     TriplesState &t = c->t;
     const int64_t o = in->o, v = in->v;
     t.o = (int)o;
@@ -267,17 +277,17 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     double *r_ovvv = nullptr, *r_ovoo = nullptr, *r_ovov = nullptr, *r_t2 = nullptr;
     int rc = SCESS_OK;
     auto cleanup = [&]() {
-        dfree(r_ovvv);
-        dfree(r_ovoo);
-        dfree(r_ovov);
-        dfree(r_t2);
+        dfree(c, r_ovvv);
+        dfree(c, r_ovoo);
+        dfree(c, r_ovov);
+        dfree(c, r_t2);
     };
     if ((rc = upload(c, in->ovvv, (size_t)(o * v * v * v), &r_ovvv)) ||
         (rc = upload(c, in->ovoo, (size_t)(o * v * o * o), &r_ovoo)) ||
         (rc = upload(c, in->ovov, (size_t)(o * v * o * v), &r_ovov)) ||
         (rc = upload(c, in->t2, (size_t)(o * o * v * v), &r_t2))) {
         cleanup();
-        free_triples(t);
+        free_triples(c);
         return rc;
     }
     // t1 as [o][vR] (ColMajor (i,a) -> row-major i, zero-padded rows) and the virtual energies padded to vR
@@ -291,14 +301,14 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     if ((rc = upload(c, t1r.data(), t1r.size(), &t.t1)) || (rc = upload(c, in->e, (size_t)(o + v), &t.e)) ||
         (rc = upload(c, evr.data(), evr.size(), &t.ev))) {
         cleanup();
-        free_triples(t);
+        free_triples(c);
         return rc;
     }
     auto pack = [&](int mode, int prec, const double *src, void **dst, int64_t rows, int64_t kpad) -> int {
         const size_t bytes = (size_t)rows * (size_t)kpad * (prec == P64 ? 8 : 4);
-        hipError_t e = hipMalloc(dst, std::max<size_t>(bytes, 16));
+        hipError_t e = dmalloc(c, dst, std::max<size_t>(bytes, 16));
         if (e != hipSuccess)
-            return hip_fail(c, e, "hipMalloc (packed operand)");
+            return hip_fail(c, e, "device allocation (packed operand)");
         e = launch_pack(mode, prec, src, *dst, (int)o, (int)v, kpad, c->stream);
         if (e != hipSuccess)
             return hip_fail(c, e, "pack kernel");
@@ -307,9 +317,9 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     // PI8: one power-of-two scale per tensor (|x| 2^-e <= 0.498), then the digit slices
     auto pack_i8 = [&](Operands &op, const double *ovvv, const double *t2, const double *ovoo) -> int {
         unsigned long long *dmax = nullptr;
-        hipError_t e = hipMalloc((void **)&dmax, 3 * sizeof(unsigned long long));
+        hipError_t e = dmalloc(c, &dmax, 3 * sizeof(unsigned long long));
         if (e != hipSuccess)
-            return hip_fail(c, e, "hipMalloc");
+            return hip_fail(c, e, "device allocation");
         unsigned long long hmax[3] = {0, 0, 0};
         e = hipMemsetAsync(dmax, 0, sizeof(hmax), c->stream);
         if (e == hipSuccess)
@@ -322,7 +332,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
             e = hipMemcpyAsync(hmax, dmax, sizeof(hmax), hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess)
             e = hipStreamSynchronize(c->stream);
-        (void)hipFree(dmax);
+        dfree(c, dmax);
         if (e != hipSuccess)
             return hip_fail(c, e, "PI8 scales");
         int ex[3];
@@ -355,9 +365,9 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
                      {PACK_TM, t2, &op.TM, o * v * v, op.oK, 32, op.eT}};
         for (const Job &jb : jobs) {
             const size_t bytes = (size_t)jb.rows * (size_t)jb.kpad * (size_t)op.slices;
-            e = hipMalloc(jb.dst, std::max<size_t>(bytes, 16));
+            e = dmalloc(c, jb.dst, std::max<size_t>(bytes, 16));
             if (e != hipSuccess)
-                return hip_fail(c, e, "hipMalloc (packed operand)");
+                return hip_fail(c, e, "device allocation (packed operand)");
             e = launch_pack_i8(jb.mode, jb.src, *jb.dst, (int)o, (int)v, jb.kpad, jb.gran, std::ldexp(1.0, -jb.e),
                                op.slices, c->stream);
             if (e != hipSuccess)
@@ -367,7 +377,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     };
     if ((rc = pack(PACK_S, P64, r_ovov, (void **)&t.S, o * o * v, v))) {
         cleanup();
-        free_triples(t);
+        free_triples(c);
         return rc;
     }
     for (int p = 0; p < kNumPrec; p++) {
@@ -382,7 +392,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
         if (p == PI8) {
             if ((rc = pack_i8(op, r_ovvv, r_t2, r_ovoo))) {
                 cleanup();
-                free_triples(t);
+                free_triples(c);
                 return rc;
             }
             t.have_prec[p] = true;
@@ -393,7 +403,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
             (rc = pack(PACK_RN, p, r_ovoo, &op.Rn, o * o * v, op.oK)) ||
             (rc = pack(PACK_TM, p, r_t2, &op.TM, o * v * v, op.oK))) {
             cleanup();
-            free_triples(t);
+            free_triples(c);
             return rc;
         }
         t.have_prec[p] = true;
@@ -401,7 +411,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     hipError_t se = hipStreamSynchronize(c->stream);
     cleanup();
     if (se != hipSuccess) {
-        free_triples(t);
+        free_triples(c);
         return hip_fail(c, se, "scess_t_set_inputs");
     }
 
@@ -429,15 +439,15 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     {
         std::vector<uint64_t> tab;
         if (!orbit_table(t.orbits, tab)) {  // unreachable for v <= 4096 (nb <= 512)
-            free_triples(t);
+            free_triples(c);
             return fail(c, SCESS_ERR_ARG, "scess_t_set_inputs: too many virtual blocks for the orbit table");
         }
-        HIP_TRY(c, hipMalloc((void **)&t.d_orbtab, sizeof(uint64_t) * tab.size()));
+        HIP_TRY(c, dmalloc(c, &t.d_orbtab, sizeof(uint64_t) * tab.size()));
         HIP_TRY(c, hipMemcpy(t.d_orbtab, tab.data(), sizeof(uint64_t) * tab.size(), hipMemcpyHostToDevice));
     }
-    HIP_TRY(c, hipMalloc((void **)&t.d_ijk_all, sizeof(int) * t.ijk_all.size()));
+    HIP_TRY(c, dmalloc(c, &t.d_ijk_all, sizeof(int) * t.ijk_all.size()));
     HIP_TRY(c, hipMemcpy(t.d_ijk_all, t.ijk_all.data(), sizeof(int) * t.ijk_all.size(), hipMemcpyHostToDevice));
-    HIP_TRY(c, hipMalloc((void **)&t.d_orbits, sizeof(int) * t.orbits.size()));
+    HIP_TRY(c, dmalloc(c, &t.d_orbits, sizeof(int) * t.orbits.size()));
     HIP_TRY(c, hipMemcpy(t.d_orbits, t.orbits.data(), sizeof(int) * t.orbits.size(), hipMemcpyHostToDevice));
     {
         // F_ijk is invariant under permutations of (i, j, k), so a triple with j == k is evaluated
@@ -457,16 +467,16 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
         }
         t.work_ijk = wijk;
         const size_t nw = std::max<size_t>(t.work.size(), 1);
-        HIP_TRY(c, hipMalloc((void **)&t.d_work_ijk, sizeof(int) * 3 * nw));
-        HIP_TRY(c, hipMalloc((void **)&t.d_work_index, sizeof(int) * nw));
+        HIP_TRY(c, dmalloc(c, &t.d_work_ijk, sizeof(int) * 3 * nw));
+        HIP_TRY(c, dmalloc(c, &t.d_work_index, sizeof(int) * nw));
         if (!t.work.empty()) {
             HIP_TRY(c, hipMemcpy(t.d_work_ijk, wijk.data(), sizeof(int) * wijk.size(), hipMemcpyHostToDevice));
             HIP_TRY(c, hipMemcpy(t.d_work_index, t.work.data(), sizeof(int) * t.work.size(), hipMemcpyHostToDevice));
         }
     }
-    HIP_TRY(c, hipMalloc((void **)&t.F, sizeof(double) * (t.ijk_all.size() / 3)));
-    HIP_TRY(c, hipMalloc((void **)&t.E, sizeof(double)));
-    HIP_TRY(c, hipMalloc((void **)&t.queue, sizeof(int) * kWQueues * std::max<size_t>(t.work.size(), 1)));
+    HIP_TRY(c, dmalloc(c, &t.F, sizeof(double) * (t.ijk_all.size() / 3)));
+    HIP_TRY(c, dmalloc(c, &t.E, sizeof(double)));
+    HIP_TRY(c, dmalloc(c, &t.queue, sizeof(int) * kWQueues * std::max<size_t>(t.work.size(), 1)));
     t.have = true;
     return SCESS_OK;
 }
@@ -550,24 +560,24 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     // batch b + 1 writes the other one
     const size_t wneed = 2 * (size_t)nbatch * (size_t)wstride * accb;
     if (t.wbytes < wneed) {
-        dfree(t.W1);
-        dfree(t.W2);
+        dfree(c, t.W1);
+        dfree(c, t.W2);
         t.wbytes = 0;
-        HIP_TRY(c, hipMalloc(&t.W1, wneed));
-        HIP_TRY(c, hipMalloc(&t.W2, wneed));
+        HIP_TRY(c, dmalloc(c, &t.W1, wneed));
+        HIP_TRY(c, dmalloc(c, &t.W2, wneed));
         t.wbytes = wneed;
     }
     // per-orbit partials: whole job if the caller wants them, else one batch
     const size_t pneed = (size_t)(partials_out ? std::max<int64_t>(nwork, 1) : 2 * nbatch) * (size_t)t.ngrp;
     if (t.partials_cap < pneed) {
-        dfree(t.partials);
-        HIP_TRY(c, hipMalloc((void **)&t.partials, sizeof(double) * pneed));
+        dfree(c, t.partials);
+        HIP_TRY(c, dmalloc(c, &t.partials, sizeof(double) * pneed));
         t.partials_cap = pneed;
     }
     const size_t uneed = 2 * (size_t)nbatch * 3 * (size_t)(v * vR);
     if (t.u_cap < uneed) {
-        dfree(t.U);
-        HIP_TRY(c, hipMalloc((void **)&t.U, sizeof(double) * uneed));
+        dfree(c, t.U);
+        HIP_TRY(c, dmalloc(c, &t.U, sizeof(double) * uneed));
         t.u_cap = uneed;
     }
     HIP_TRY(c, hipMemsetAsync(t.F, 0, sizeof(double) * nall, c->stream));
@@ -890,7 +900,7 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
     // device buffers of this call, freed on every exit
     std::vector<void *> bufs;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
+        hipError_t e = dmalloc(c, p, bytes);
         if (e == hipSuccess) {
             bufs.push_back(*p);
             e = hipMemsetAsync(*p, 0, std::max<size_t>(bytes, 16), c->stream);
@@ -906,7 +916,7 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
         if (ws)
             (void)hipStreamSynchronize(ws);
         for (void *p : bufs)
-            (void)hipFree(p);
+            c->blocks.put(p);
         bufs.clear();
         for (int q = 0; q < 2; q++) {
             if (evW[q])
@@ -1214,9 +1224,7 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
         for (auto &u : outs) {
             he = launch_unpack(u.mode, u.A, u.B, out, (int)o, (int)v, vK, oK, vR, (int64_t)u.n, c->stream);
             if (he == hipSuccess)
-                he = hipMemcpyAsync(u.host, out, 8 * u.n, hipMemcpyDeviceToHost, c->stream);
-            if (he == hipSuccess)
-                he = hipStreamSynchronize(c->stream);
+                he = scess::copy_to_host(u.host, out, 8 * u.n, c->stream);
             if (he != hipSuccess) {
                 rc = hip_fail(c, he, "scess_t_backward: unpack");
                 break;
