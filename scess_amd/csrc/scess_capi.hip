@@ -899,10 +899,11 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
 
     // device buffers of this call, freed on every exit
     std::vector<void *> bufs;
-    auto alloc = [&](size_t bytes, void **p) -> hipError_t {
+    auto alloc = [&](size_t bytes, void **p, bool zero) -> hipError_t {
         hipError_t e = dmalloc(c, p, bytes);
-        if (e == hipSuccess) {
+        if (e == hipSuccess)
             bufs.push_back(*p);
+        if (e == hipSuccess && zero) {
             e = hipMemsetAsync(*p, 0, std::max<size_t>(bytes, 16), c->stream);
         }
         return e;
@@ -927,46 +928,110 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
         if (ws)
             (void)hipStreamDestroy(ws);
     };
-    // K splits of dT (v x v outputs, K = v^2) and dRn (v x o outputs, K = v^2): about 1024 work-groups per
-    // GEMM so that the long K loops overlap their memory latency across the chip (the terms of a triple
-    // then run together, up to six GEMMs per launch). SCESS_ADJ_SPLITS = PT,PR overrides (tuning).
-    const int64_t tilesT = ((v + 63) / 64) * ((v + 63) / 64), tilesR = ((v + 63) / 64) * ((o + 63) / 64);
-    int PT = (int)std::min<int64_t>(64, std::max<int64_t>(16, 1024 / tilesT));
-    int PR = (int)std::min<int64_t>(128, std::max<int64_t>(32, 1024 / tilesR));
-    if (const char *e = std::getenv("SCESS_ADJ_SPLITS")) {
-        int a = 0, b = 0;
-        if (std::sscanf(e, "%d,%d", &a, &b) == 2 && a >= 1 && a <= 256 && b >= 1 && b <= 256) {
-            PT = a;
-            PR = b;
-        }
-    }
-    double *dX, *dT, *dRn, *dTM, *dS, *dt1, *GW, *GV, *U, *dU, *dtv, *scr, *out;
+    double *dX, *dT, *dRn, *dTM, *dS, *dt1, *GW, *GV, *U, *dU, *dtv, *H, *scr, *out;
     void *W1[2], *W2[2];
-    // W of up to WB triples is built by one launch (2 buffers of WB x vR^3 within 4 GB per set)
-    const int64_t WB = std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)(4.0e9 / (2.0 * (double)wstride * accb))));
+    BackSeg *dsegs;
+    BackTarget *dtg;
+    const int64_t nwork = (int64_t)t.work.size();
+    const int64_t w_begin = nwork * c->shard / c->nshards, w_end = nwork * (c->shard + 1) / c->nshards;
+    // Triples per batch, each step of which is one launch: 8 for large v (W of one set at least), up to 128 within 256 MB
+    // of W per set for small v, where a batch of 8 leaves launches too short to fill the chip (o=10, v=75: 8 triples
+    // 17.2 ms, 31 triples 12.7 ms); fewer where a set of W passes 4 GB, and one at a time where memory does not hold the batch
+    const double wper = 2.0 * (double)wstride * accb;
+    int64_t WB = std::max<int64_t>(8, std::min<int64_t>(128, (int64_t)(256.0e6 / wper)));
+    WB = std::max<int64_t>(1, std::min<int64_t>(WB, (int64_t)(4.0e9 / wper)));
+    WB = std::max<int64_t>(1, std::min<int64_t>(WB, w_end - w_begin));
     hipError_t he = hipSuccess;
     const size_t nX = (size_t)(o * v * v * vK), nT = (size_t)(o * o * v * vK), nR = (size_t)(o * o * v * oK),
                  nTM = (size_t)(o * v * v * oK), nS = (size_t)(o * o * v * v), nt1 = (size_t)(o * vR),
-                 nG = (size_t)wstride, nscr = (size_t)kMaxGemmGroup * std::max<int64_t>(PT * v * v, PR * v * o);
+                 vv = (size_t)(v * v);
     // staging of each unpacked gradient before its download: the largest of ovvv (o v^3), ovoo (o^3 v),
     // ovov and t2 (o^2 v^2) and t1 (o v)
     const size_t nout = std::max<size_t>({(size_t)(o * v * v * v), (size_t)(o * v * o * o), (size_t)(o * o * v * v),
                                           (size_t)(o * v)});
-    if ((he = alloc(8 * nX, (void **)&dX)) != hipSuccess || (he = alloc(8 * nT, (void **)&dT)) != hipSuccess ||
-        (he = alloc(8 * nR, (void **)&dRn)) != hipSuccess || (he = alloc(8 * nTM, (void **)&dTM)) != hipSuccess ||
-        (he = alloc(8 * nS, (void **)&dS)) != hipSuccess || (he = alloc(8 * nt1, (void **)&dt1)) != hipSuccess ||
-        (he = alloc(8 * nG, (void **)&GW)) != hipSuccess || (he = alloc(8 * nG, (void **)&GV)) != hipSuccess ||
-        (he = alloc(8 * 3 * (size_t)(v * vR), (void **)&U)) != hipSuccess ||
-        (he = alloc(8 * 3 * (size_t)(v * v), (void **)&dU)) != hipSuccess ||
-        (he = alloc(8 * 3 * (size_t)v, (void **)&dtv)) != hipSuccess ||
-        (he = alloc(8 * nscr, (void **)&scr)) != hipSuccess || (he = alloc(8 * nout, (void **)&out)) != hipSuccess ||
-        (he = alloc(accb * (size_t)(WB * wstride), &W1[0])) != hipSuccess ||
-        (he = alloc(accb * (size_t)(WB * wstride), &W2[0])) != hipSuccess ||
-        (he = alloc(accb * (size_t)(WB * wstride), &W1[1])) != hipSuccess ||
-        (he = alloc(accb * (size_t)(WB * wstride), &W2[1])) != hipSuccess) {
+    BackArgs ba{};
+    ba.o8 = (int)round_up(o, 8);
+    ba.v8 = (int)round_up(v, 8);
+    BackTables tab;
+    std::vector<BackBatch> bb;
+    std::vector<int> ijk;  // the shard's triples in the order of the batches
+    int *dijk;
+    for (;; WB = 1) {
+        ba.splits = back_splits((int)WB, (int)o, (int)v);
+        tab.segs.clear();
+        tab.tg.clear();
+        bb.assign((size_t)((w_end - w_begin + WB - 1) / WB), BackBatch{});
+        ijk.clear();
+        const int64_t nsh = w_end - w_begin, step = back_spread((int)o, (int)v) ? (int64_t)bb.size() : 1;
+        for (int64_t first = 0; first < step; first++)
+            for (int64_t w = first; w < nsh; w += step)
+                ijk.insert(ijk.end(), t.work_ijk.begin() + 3 * (w_begin + w), t.work_ijk.begin() + 3 * (w_begin + w) + 3);
+        for (size_t b = 0; b < bb.size(); b++)
+            back_terms(ijk.data() + 3 * b * WB, (int)std::min<int64_t>(WB, nsh - (int64_t)b * WB), (int)o, tab, bb[b]);
+        const size_t n = (size_t)WB, nw = sizeof(double) * n;
+        const size_t nscr = 6 * n * (size_t)ba.splits * (size_t)(v * (ba.v8 + ba.o8));
+        struct {
+            size_t bytes;
+            void **p;
+            bool zero;
+        } all[] = {{8 * nX, (void **)&dX, true},
+                   {8 * nT, (void **)&dT, true},
+                   {8 * nR, (void **)&dRn, true},
+                   {8 * nTM, (void **)&dTM, true},
+                   {8 * nS, (void **)&dS, true},
+                   {8 * nt1, (void **)&dt1, true},
+                   {nw * (size_t)wstride, (void **)&GW, true},  // stays zero past v
+                   {nw * (size_t)wstride, (void **)&GV, false},
+                   {nw * 3 * (size_t)(v * vR), (void **)&U, true},
+                   {nw * 3 * vv, (void **)&dU, false},
+                   {nw * 3 * (size_t)v, (void **)&dtv, false},
+                   {nw * vv, (void **)&H, false},
+                   {8 * nscr, (void **)&scr, false},
+                   {8 * nout, (void **)&out, false},
+                   {accb * n * (size_t)wstride, &W1[0], true},
+                   {accb * n * (size_t)wstride, &W2[0], true},
+                   {accb * n * (size_t)wstride, &W1[1], true},
+                   {accb * n * (size_t)wstride, &W2[1], true},
+                   {sizeof(BackSeg) * tab.segs.size(), (void **)&dsegs, false},
+                   {sizeof(BackTarget) * tab.tg.size(), (void **)&dtg, false},
+                   {sizeof(int) * ijk.size(), (void **)&dijk, false}};
+        he = hipSuccess;
+        for (auto &x : all)
+            if (he == hipSuccess)
+                he = alloc(x.bytes, x.p, x.zero);
+        if (he == hipSuccess)
+            break;
         release();
-        return hip_fail(c, he, "scess_t_backward: device allocation");
+        if (he != hipErrorOutOfMemory || WB == 1)
+            return hip_fail(c, he, "scess_t_backward: device allocation");
+        (void)hipGetLastError();
     }
+    if (!tab.segs.empty()) {
+        he = hipMemcpyAsync(dsegs, tab.segs.data(), sizeof(BackSeg) * tab.segs.size(), hipMemcpyHostToDevice, c->stream);
+        if (he == hipSuccess)
+            he = hipMemcpyAsync(dtg, tab.tg.data(), sizeof(BackTarget) * tab.tg.size(), hipMemcpyHostToDevice, c->stream);
+        if (he == hipSuccess)
+            he = hipMemcpyAsync(dijk, ijk.data(), sizeof(int) * ijk.size(), hipMemcpyHostToDevice, c->stream);
+        if (he != hipSuccess) {
+            release();
+            return hip_fail(c, he, "scess_t_backward: tables");
+        }
+    }
+    ba.G = GW;
+    ba.gstride = wstride;
+    ba.o = (int)o;
+    ba.v = (int)v;
+    ba.vR = (int)vR;
+    ba.vK = vK;
+    ba.oK = oK;
+    ba.T = (const double *)o64.T;
+    ba.Rn = (const double *)o64.Rn;
+    ba.X = (const double *)o64.X;
+    ba.TM = (const double *)o64.TM;
+    ba.dX = dX;
+    ba.dTM = dTM;
+    ba.scr = scr;
+    ba.segs = dsegs;
     if ((he = hipStreamCreateWithFlags(&ws, hipStreamNonBlocking)) != hipSuccess) {
         ws = nullptr;
         release();
@@ -1006,206 +1071,57 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
     ea.ev = t.ev;
     ea.U = U;
 
-    static const int PERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
-    const int64_t pos_stride[3] = {vR * vR, vR, 1};
-    const double *X64 = (const double *)o64.X, *T64 = (const double *)o64.T, *Rn64 = (const double *)o64.Rn,
-                 *TM64 = (const double *)o64.TM;
     int rc = SCESS_OK;
     bool cancelled = false;
-    const int64_t nwork = (int64_t)t.work.size();
-    const int64_t w_begin = nwork * c->shard / c->nshards, w_end = nwork * (c->shard + 1) / c->nshards;
-    for (int64_t w = w_begin; w < w_end && rc == SCESS_OK; w++) {
-        if ((w & 7) == 0) {
-            if ((he = hipStreamSynchronize(c->stream)) != hipSuccess) {
-                rc = hip_fail(c, he, "scess_t_backward");
-                break;
-            }
-            if (c->should_stop && c->should_stop(c->user)) {
-                cancelled = true;
-                break;
-            }
+    const int64_t nbat = (int64_t)bb.size();
+    // W of a batch on the second stream, once the batch before the last has released its set
+    auto build = [&](int64_t b) {
+        const int64_t w0 = b * WB;
+        hipError_t e = hipSuccess;
+        if (b >= 2)
+            e = hipStreamWaitEvent(ws, evDone[b & 1], 0);
+        wa.ijk = dijk + 3 * w0;
+        wa.queue = t.queue + kWQueues * b;
+        wa.W1 = W1[b & 1];
+        wa.W2 = W2[b & 1];
+        if (e == hipSuccess)
+            e = launch_wbuild(prec, blk, wbuild_dma(), wa, (int)std::min<int64_t>(WB, w_end - w_begin - w0), ws);
+        if (e == hipSuccess)
+            e = hipEventRecord(evW[b & 1], ws);
+        return e;
+    };
+    for (int64_t b = 0; b < nbat && rc == SCESS_OK; b++) {
+        const int64_t w0 = b * WB, set = b & 1;
+        const int n = (int)std::min<int64_t>(WB, w_end - w_begin - w0);
+        // at most two batches in flight, so that cancellation is polled while the device works
+        if (b >= 2 && (he = hipEventSynchronize(evDone[set])) != hipSuccess) {
+            rc = hip_fail(c, he, "scess_t_backward");
+            break;
         }
-        const int occ[3] = {t.work_ijk[3 * w], t.work_ijk[3 * w + 1], t.work_ijk[3 * w + 2]};
-        const double deg = (occ[0] == occ[1] || occ[1] == occ[2]) ? 2.0 : 1.0;
-        const int *dijk = t.d_work_ijk + 3 * w;
-        const int64_t slot = (w - w_begin) % WB, batch = (w - w_begin) / WB, set = batch & 1;
-        if (slot == 0) {
-            // W of batch b + 1 on the second stream (W of batch 0 first), once batch b - 1 has released
-            // that set; batch b waits for its own W
-            auto build = [&](int64_t b) {
-                const int64_t w0 = w_begin + b * WB;
-                hipError_t e = hipSuccess;
-                if (b >= 2)
-                    e = hipStreamWaitEvent(ws, evDone[b & 1], 0);
-                wa.ijk = t.d_work_ijk + 3 * w0;
-                wa.queue = t.queue + kWQueues * b;
-                wa.W1 = W1[b & 1];
-                wa.W2 = W2[b & 1];
-                if (e == hipSuccess)
-                    e = launch_wbuild(prec, blk, wbuild_dma(), wa, (int)std::min<int64_t>(WB, w_end - w0), ws);
-                if (e == hipSuccess)
-                    e = hipEventRecord(evW[b & 1], ws);
-                return e;
-            };
-            if (batch == 0)
-                he = build(0);
-            if (he == hipSuccess && w + WB < w_end)
-                he = build(batch + 1);
-            if (he == hipSuccess)
-                he = hipStreamWaitEvent(c->stream, evW[set], 0);
+        if (c->should_stop && c->should_stop(c->user)) {
+            cancelled = true;
+            break;
         }
-        ea.ijk = dijk;
-        ea.W1 = (const char *)W1[set] + (size_t)slot * wstride * accb;
-        ea.W2 = occ[0] == occ[1] ? ea.W1 : (const char *)W2[set] + (size_t)slot * wstride * accb;
+        he = b == 0 ? build(0) : hipSuccess;
         if (he == hipSuccess)
-            he = launch_vpieces(t.S, dijk, (int)o, (int)v, (int)vR, U, 1, c->stream);
+            he = hipStreamWaitEvent(c->stream, evW[set], 0);
+        if (he == hipSuccess && b + 1 < nbat)
+            he = build(b + 1);
+        ea.ijk = dijk + 3 * w0;
+        ea.W1 = W1[set];
+        ea.W2 = W2[set];
+        if (he == hipSuccess)
+            he = launch_vpieces(t.S, ea.ijk, (int)o, (int)v, (int)vR, U, n, c->stream);
         // G_W entries with an index in [v, vR) are zero: the buffer starts zeroed and the G kernel writes
-        // exact zeros past v (the back-contraction GEMMs read them as K padding)
+        // exact zeros past v (the back-contractions read them as K padding)
         if (he == hipSuccess)
-            he = launch_adjoint_g(prec, ea, dE * 2.0 / deg, GW, GV, c->stream);
-        // With occ[0] == occ[1] (every triple with two equal indices, as evaluated) G is symmetric in its
-        // first two indices, and the permutation terms pair up: the term with the values 0 and 1 of its
-        // permutation exchanged (PERM rows 0-2, 1-3, 4-5) reads the same operands and writes the same
-        // output. Such a triple runs one term of each pair with alpha = 2 (half the GEMM work).
-        const bool twin = occ[0] == occ[1];
-        // dX[p][x][y][f] += sum_z G(x,y,z) T[r][q][z][f]: the two permutation terms with the same
-        // position for x (PERM rows 2m, 2m+1) write the same dX[p], so they run as one GEMM with
-        // two K segments (twin: pair 1 equals pair 0, and the two segments of pair 2 are equal)
-        // The GEMMs of each kind write disjoint slices (dX[p] for the three values of p, dT[r][q] and
-        // dRn[p][q] for six distinct pairs, dTM[r] for three values), so each kind runs as one group, and
-        // every output element still receives this triple's contribution once, in triple order.
-        GemmGroup grp{};
-        grp.n = 0;
-        for (int pr = 0; pr < 3 && he == hipSuccess; pr++) {
-            if (twin && pr == 1)
-                continue;
-            const int64_t p = occ[PERM[2 * pr][0]], sx = pos_stride[PERM[2 * pr][0]];
-            GemmArgs g{};
-            g.nseg = twin && pr == 2 ? 1 : 2;
-            g.M = (int)v;
-            g.N = (int)v;
-            g.alpha = twin ? 2.0 : 1.0;
-            g.splits = 1;
-            for (int h = 0; h < g.nseg; h++) {
-                const int sgm = 2 * pr + h;
-                const int64_t q = occ[PERM[sgm][1]], r = occ[PERM[sgm][2]];
-                const int64_t sy = pos_stride[PERM[sgm][1]], sz = pos_stride[PERM[sgm][2]];
-                GemmSeg &sg = g.seg[h];
-                sg.K1 = 1;
-                sg.K2 = (int)v;
-                // rows x batch y, or rows y batch x
-                sg.A = {GW, sx == 1 ? sx : sy, 0, sz, sx == 1 ? sy : sx, vR, true};
-                sg.B = {T64 + (r * o + q) * v * vK, 1, 0, vK, 0, vK, false};
-            }
-            g.C = dX + p * v * v * vK;
-            g.sCn = 1;
-            g.sCb = sx == 1 ? vK : v * vK;
-            g.sCm = sx == 1 ? v * vK : vK;
-            grp.g[grp.n++] = g;
-        }
+            he = launch_adjoint_g(prec, ea, dE, GW, GV, n, c->stream);
         if (he == hipSuccess)
-            he = launch_gemm_group(grp, (int)v, c->stream);
-        GemmGroup grpT{}, grpR{};
-        grpT.n = grpR.n = 0;
-        for (int sgm = 0; sgm < 6 && he == hipSuccess; sgm++) {
-            if (twin && (sgm == 2 || sgm == 3 || sgm == 5))
-                continue;  // the twins of terms 0, 1, 4
-            const double alpha = twin ? 2.0 : 1.0;
-            const int64_t p = occ[PERM[sgm][0]], q = occ[PERM[sgm][1]], r = occ[PERM[sgm][2]];
-            const int64_t sx = pos_stride[PERM[sgm][0]], sy = pos_stride[PERM[sgm][1]], sz = pos_stride[PERM[sgm][2]];
-            // dT[r][q][z][f] += sum_{x,y} G(x,y,z) X[p][x][y][f]
-            {
-                GemmArgs g{};
-                g.nseg = 1;
-                g.M = (int)v;
-                g.N = (int)v;
-                g.alpha = alpha;
-                g.splits = PT;
-                g.scratch = scr + (size_t)grpT.n * PT * v * v;
-                GemmSeg &sg = g.seg[0];
-                sg.K1 = (int)v;
-                sg.K2 = (int)v;
-                if (sx < sy) {  // inner K over x
-                    sg.A = {GW, sz, sy, sx, 0, vR, true};
-                    sg.B = {X64 + p * v * v * vK, 1, vK, v * vK, 0, vK, false};
-                } else {  // inner K over y
-                    sg.A = {GW, sz, sx, sy, 0, vR, true};
-                    sg.B = {X64 + p * v * v * vK, 1, v * vK, vK, 0, vK, false};
-                }
-                g.C = dT + (r * o + q) * v * vK;
-                g.sCm = vK;
-                g.sCn = 1;
-                grpT.g[grpT.n++] = g;
-            }
-            // dRn[p][q][x][m] += sum_{y,z} G(x,y,z) TM[r][y][z][m] (its own group; run after the dT group,
-            // so the two reuse one scratch area)
-            {
-                GemmArgs g{};
-                g.nseg = 1;
-                g.M = (int)v;
-                g.N = (int)o;
-                g.alpha = alpha;
-                g.splits = PR;
-                g.scratch = scr + (size_t)grpR.n * PR * v * o;
-                GemmSeg &sg = g.seg[0];
-                sg.K1 = (int)v;
-                sg.K2 = (int)v;
-                if (sy < sz) {  // inner K over y
-                    sg.A = {GW, sx, sz, sy, 0, vR, true};
-                    sg.B = {TM64 + r * v * v * oK, 1, oK, v * oK, 0, oK, false};
-                } else {  // inner K over z
-                    sg.A = {GW, sx, sy, sz, 0, vR, true};
-                    sg.B = {TM64 + r * v * v * oK, 1, v * oK, oK, 0, oK, false};
-                }
-                g.C = dRn + (p * o + q) * v * oK;
-                g.sCm = oK;
-                g.sCn = 1;
-                grpR.g[grpR.n++] = g;
-            }
-        }
+            he = launch_back(ba, dtg, bb[(size_t)b], dT, dRn, c->stream);
         if (he == hipSuccess)
-            he = launch_gemm_group(grpT, 1, c->stream);
+            he = launch_vback(GV, wstride, U, t.t1, ea.ijk, n, dtg + bb[(size_t)b].second.tg0, bb[(size_t)b].second.ntg, (int)o,
+                              (int)v, (int)vR, dU, dtv, H, dS, dt1, c->stream);
         if (he == hipSuccess)
-            he = launch_gemm_group(grpR, 1, c->stream);
-        // dTM[r][y][z][m] += sum_x Rn[p][q][x][m] G(x,y,z): the two terms with the same position for z
-        // write the same dTM[r]; one GEMM with two K segments each (rows z and batch y when z is the
-        // contiguous position of G, else rows y and batch z)
-        // (twin: the two segments of pair 0 are equal, and pair 2 equals pair 1)
-        static const int ZPAIR[3][2] = {{0, 2}, {1, 4}, {3, 5}};
-        grp.n = 0;
-        for (int pr = 0; pr < 3 && he == hipSuccess; pr++) {
-            if (twin && pr == 2)
-                continue;
-            const int64_t r = occ[PERM[ZPAIR[pr][0]][2]], sz = pos_stride[PERM[ZPAIR[pr][0]][2]];
-            GemmArgs g{};
-            g.nseg = twin && pr == 0 ? 1 : 2;
-            g.M = (int)v;
-            g.N = (int)o;
-            g.alpha = twin ? 2.0 : 1.0;
-            g.splits = 1;
-            for (int h = 0; h < g.nseg; h++) {
-                const int sgm = ZPAIR[pr][h];
-                const int64_t p = occ[PERM[sgm][0]], q = occ[PERM[sgm][1]];
-                const int64_t sx = pos_stride[PERM[sgm][0]], sy = pos_stride[PERM[sgm][1]];
-                GemmSeg &sg = g.seg[h];
-                sg.K1 = 1;
-                sg.K2 = (int)v;
-                sg.B = {Rn64 + (p * o + q) * v * oK, 1, 0, oK, 0, oK, false};
-                sg.A = sz == 1 ? GemmOp{GW, sz, 0, sx, sy, vR, true} : GemmOp{GW, sy, 0, sx, sz, vR, true};
-            }
-            g.C = dTM + r * v * v * oK;
-            g.sCn = 1;
-            g.sCb = sz == 1 ? v * oK : oK;
-            g.sCm = sz == 1 ? oK : v * oK;
-            grp.g[grp.n++] = g;
-        }
-        if (he == hipSuccess)
-            he = launch_gemm_group(grp, (int)v, c->stream);
-        if (he == hipSuccess)
-            he = launch_vback(GV, U, t.t1, occ[0], occ[1], occ[2], (int)o, (int)v, (int)vR, dU, dtv, scr, dS, dt1,
-                              c->stream);  // scr (the split-K scratch, >= v^2, free again here) holds H
-        // the last triple of a batch releases its W set
-        if (he == hipSuccess && (slot == WB - 1 || w == w_end - 1))
             he = hipEventRecord(evDone[set], c->stream);
         if (he != hipSuccess)
             rc = hip_fail(c, he, "scess_t_backward: kernel launch");

@@ -5,18 +5,20 @@
 // W is recomputed per ijk (the forward W-build), G is formed by an orbit kernel
 // like the forward epilogue, and the six permutation terms
 //   w(x,y,z; p,q,r) = sum_f X[p][x][y][f] T[r][q][z][f] + sum_m Rn[p][q][x][m] TM[r][y][z][m]
-// are back-contracted by one generic FP64 MFMA GEMM:
+// are back-contracted on the FP64 MFMAs (back_kernel):
 //   dX[p][x][y][f]  += sum_z     G(x,y,z) T[r][q][z][f]
 //   dT[r][q][z][f]  += sum_{x,y} G(x,y,z) X[p][x][y][f]
 //   dRn[p][q][x][m] += sum_{y,z} G(x,y,z) TM[r][y][z][m]
 //   dTM[r][y][z][m] += sum_x     Rn[p][q][x][m] G(x,y,z)
-// Occupied triples are processed one after another and every kernel writes each
-// output element from one thread in a fixed order (split-K partials are summed
-// in split order), so the gradients are deterministic.
-#include <type_traits>
+// Occupied triples are processed in batches and every kernel writes each output
+// element from one thread in a fixed order (partials are summed in order), so the
+// gradients are deterministic.
 #include "triples_internal.h"
 
+#include <algorithm>
 #include <cstdint>
+#include <type_traits>
+#include <vector>
 #include <cstdlib>
 
 namespace scess {
@@ -102,23 +104,28 @@ __device__ inline OrbitRowA orbit_row_a(const int *orbits, int orb, int tid) {
 
 constexpr int GK_THREADS = 384;
 
-// G_W and G_V (row-major [vR][vR][vR], FP64) of one occupied triple.
+// G_W and G_V (row-major [vR][vR][vR], FP64) of the occupied triple blockIdx.y, with the weight dE 2 / deg. Triples with
+// two equal indices come as i == j: their G_W is symmetric in its first two indices and the six terms of the
+// back-contractions pair up, so G_W is doubled and one term of each pair is left out (back_terms).
 template <typename AccT>
-__global__ __launch_bounds__(GK_THREADS) void adjoint_g_kernel(EpiArgs a, double wgt, double *GW, double *GV) {
+__global__ __launch_bounds__(GK_THREADS) void adjoint_g_kernel(EpiArgs a, double dE, double *GW, double *GV) {
     constexpr int EB = 8;
     constexpr int PY = 9, PX = EB * PY + 1, PB = EB * PX;
     __shared__ double Yl[6 * PB];
     __shared__ double Zl[6 * PB];
     const int tid = threadIdx.x;
     const int orb = blockIdx.x;
-    const int *q = a.ijk;
+    const int *q = a.ijk + 3 * blockIdx.y;
     const int i = q[0], j = q[1], k = q[2];
     const int v = a.v, vR = a.vR, nbR = a.vR >> 3;
     const int64_t vr = (int64_t)v * vR;
     const double eocc = a.e[i] + a.e[j] + a.e[k];
-    const double *U = a.U;
-    const AccT *W1b = (const AccT *)a.W1;
-    const AccT *W2b = (const AccT *)a.W2;
+    const double *U = a.U + blockIdx.y * 3 * vr;
+    const AccT *W1b = (const AccT *)a.W1 + blockIdx.y * a.wstride;
+    const AccT *W2b = i == j ? W1b : (const AccT *)a.W2 + blockIdx.y * a.wstride;
+    const double wgt = i == j ? dE : 2.0 * dE, wgtw = 2.0 * dE;
+    GW += blockIdx.y * a.wstride;
+    GV += blockIdx.y * a.wstride;
     const int ap = (tid >> 3) & 7, bp = tid & 7, d = tid >> 6;
 
     const OrbitRowA r = orbit_row_a<PB, PX, PY>(a.orbits, orb, tid);
@@ -160,6 +167,7 @@ __global__ __launch_bounds__(GK_THREADS) void adjoint_g_kernel(EpiArgs a, double
     if (rowok) {
         double *gw = GW + ((int64_t)r.ga * vR + r.gb) * vR + r.gc0;
         double *gv = GV + ((int64_t)r.ga * vR + r.gb) * vR + r.gc0;
+        double ow[EB], oz[EB];
 #pragma unroll
         for (int cp = 0; cp < EB; cp++) {
             double y3 = 0.0, z3 = 0.0;
@@ -169,435 +177,29 @@ __global__ __launch_bounds__(GK_THREADS) void adjoint_g_kernel(EpiArgs a, double
                 z3 = 4.0 * Z0[cp] + Zl[r.off[0] + cp * r.step[0]] + Zl[r.off[1] + cp * r.step[1]] -
                      2.0 * (Zl[r.off[2] + cp * r.step[2]] + Zl[r.off[3] + cp * r.step[3]] + Zl[r.off[4] + cp * r.step[4]]);
             }
-            gw[cp] = wgt * (y3 / D0[cp] + z3);
-            gv[cp] = wgt * z3;
+            ow[cp] = wgtw * (y3 / D0[cp] + z3);
+            oz[cp] = wgt * z3;
+        }
+#pragma unroll
+        for (int cp = 0; cp < EB; cp += 2) {
+            *(d2 *)(gw + cp) = d2{ow[cp], ow[cp + 1]};
+            *(d2 *)(gv + cp) = d2{oz[cp], oz[cp + 1]};
         }
     }
 }
 
-hipError_t launch_adjoint_g(int prec, const EpiArgs &a, double wgt, double *GW, double *GV, hipStream_t s) {
+hipError_t launch_adjoint_g(int prec, const EpiArgs &a, double dE, double *GW, double *GV, int nbatch, hipStream_t s) {
+    const dim3 grid((unsigned)a.norb, (unsigned)nbatch);
     if (prec == P64 || prec == PI8)  // both build W in FP64
-        hipLaunchKernelGGL(adjoint_g_kernel<double>, dim3((unsigned)a.norb), dim3(GK_THREADS), 0, s, a, wgt, GW, GV);
+        hipLaunchKernelGGL(adjoint_g_kernel<double>, grid, dim3(GK_THREADS), 0, s, a, dE, GW, GV);
     else
-        hipLaunchKernelGGL(adjoint_g_kernel<float>, dim3((unsigned)a.norb), dim3(GK_THREADS), 0, s, a, wgt, GW, GV);
+        hipLaunchKernelGGL(adjoint_g_kernel<float>, grid, dim3(GK_THREADS), 0, s, a, dE, GW, GV);
     return hipGetLastError();
 }
 
-// ------------------------------------------------------------ generic GEMM
-// C[beta][m][n] += alpha * sum_seg sum_{k1,k2} A(m, k1, k2) B(n, k1, k2), FP64 MFMA 16x16x4,
-// 64x64 tiles (2x2 waves of 2x2 blocks), K chunks of 16 along k2 staged through LDS.
-// With splits > 1 (no batch), split p handles a fixed contiguous range of the K chunks
-// and writes its partial tile to scratch[p]; gemm_reduce_kernel adds them in split order.
-// pitch 80: the four 16-lane groups of a fragment read land 32 banks apart (conflict-free halves)
-constexpr int GT = 64, GKC = 16, GPITCH = 80;
-
-// One operand's 64 rows x 16 k of chunk (k1, k2c): 4 elements per thread. Sixteen consecutive
-// lanes take 16 consecutive elements along the operand's contiguous dimension (k when the
-// operand is K-major, rows otherwise), so every load instruction reads 128-byte runs.
-struct TileLoad {
-    bool kinner;
-    __device__ TileLoad(const GemmOp &op) : kinner(op.s2 == 1 || (op.sr != 1 && (op.s2 < op.sr))) {}
-    __device__ void coords(int tid, int u, int &rr, int &kk) const {
-        if (kinner) {
-            rr = (tid >> 4) + 16 * u;
-            kk = tid & 15;
-        } else {
-            kk = tid >> 4;
-            rr = (tid & 15) + 16 * u;
-        }
-    }
-};
-
-__device__ inline void gemm_fetch(const GemmOp &op, const TileLoad &tl, int64_t base, int r0, int rext, int k1, int k2c,
-                                  int K2, double *reg, int tid) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        int rr, kk;
-        tl.coords(tid, u, rr, kk);
-        const int gr = r0 + rr, gk = k2c * GKC + kk;
-        reg[u] = gr < rext && gk < K2 ? op.base[base + (int64_t)gr * op.sr + (int64_t)k1 * op.s1 + (int64_t)gk * op.s2]
-                                      : 0.0;
-    }
-}
-
-__device__ inline void gemm_stash(const TileLoad &tl, const double *reg, double *lds, int tid) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        int rr, kk;
-        tl.coords(tid, u, rr, kk);
-        lds[kk * GPITCH + rr] = reg[u];
-    }
-}
-
-// Paired loads for operands with a contiguous dimension and even strides (16-byte aligned pairs):
-// MODE 1 rows contiguous (sr == 1), a pair is rows (2j, 2j + 1) at one k, 32 lanes per k row;
-// MODE 2 K contiguous (s2 == 1), a pair is k (2j, 2j + 1) of one row, 8 lanes per row. Two pairs
-// per thread; reg[2u], reg[2u + 1] hold pair u. Elements past rext / K2 are zero.
-template <int MODE> __device__ inline void pair_coords(int tid, int u, int &rr, int &kk) {
-    const int p = tid + 256 * u;
-    if constexpr (MODE == 1) {
-        kk = p >> 5;
-        rr = (p & 31) * 2;
-    } else {
-        rr = p >> 3;
-        kk = (p & 7) * 2;
-    }
-}
-
-template <int MODE>
-__device__ inline void gemm_fetch_pair(const GemmOp &op, int64_t base, int r0, int rext, int k1, int k2c, int K2,
-                                       double *reg, int tid) {
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        int rr, kk;
-        pair_coords<MODE>(tid, u, rr, kk);
-        const int gr = r0 + rr, gk = k2c * GKC + kk;
-        const bool full = MODE == 1 ? (gk < K2 && gr + 1 < rext) : (gr < rext && gk + 1 < K2);
-        const bool first = gr < rext && gk < K2;
-        const double *src = op.base + base + (int64_t)gr * op.sr + (int64_t)k1 * op.s1 + (int64_t)gk * op.s2;
-        if (full) {
-            const d2 x = *(const d2 *)src;
-            reg[2 * u] = x[0];
-            reg[2 * u + 1] = x[1];
-        } else {
-            reg[2 * u] = first ? src[0] : 0.0;
-            reg[2 * u + 1] = 0.0;
-        }
-    }
-}
-
-template <int MODE> __device__ inline void gemm_stash_pair(const double *reg, double *lds, int tid) {
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        int rr, kk;
-        pair_coords<MODE>(tid, u, rr, kk);
-        if constexpr (MODE == 1) {
-            *(d2 *)&lds[kk * GPITCH + rr] = d2{reg[2 * u], reg[2 * u + 1]};
-        } else {
-            lds[kk * GPITCH + rr] = reg[2 * u];
-            lds[(kk + 1) * GPITCH + rr] = reg[2 * u + 1];
-        }
-    }
-}
-
-// One operand of chunk (k1, k2c) in load mode MODE (0 element-wise, 1 / 2 paired)
-template <int MODE>
-__device__ inline void fetch_op(const GemmOp &op, int64_t base, int r0, int rext, int k1, int k2c, int K2, double *reg,
-                                int tid) {
-    if constexpr (MODE == 0)
-        gemm_fetch(op, TileLoad(op), base, r0, rext, k1, k2c, K2, reg, tid);
-    else
-        gemm_fetch_pair<MODE>(op, base, r0, rext, k1, k2c, K2, reg, tid);
-}
-template <int MODE> __device__ inline void stash_op(const GemmOp &op, const double *reg, double *lds, int tid) {
-    if constexpr (MODE == 0)
-        gemm_stash(TileLoad(op), reg, lds, tid);
-    else
-        gemm_stash_pair<MODE>(reg, lds, tid);
-}
-
-// A0, A1, B0, B1: load modes of A and B in segments 0 and 1
-template <int A0, int A1, int B0, int B1>
-__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-    // two LDS buffers; the global loads of chunk c + 1 are in flight while chunk c is multiplied
-    __shared__ __attribute__((aligned(16))) double As[2][GKC * GPITCH];
-    __shared__ __attribute__((aligned(16))) double Bs[2][GKC * GPITCH];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int ntn = (g.N + GT - 1) / GT;
-    // tiles of one (batch, split) on one XCD, so the tiles sharing an operand panel share its L2
-    const int nx = gridDim.x, ny = gridDim.y;
-    const int lin = xcd_remap(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z), nx * ny * gridDim.z);
-    const int bx = lin % nx, byz = lin / nx;
-    const int tm = bx / ntn, tn = bx - tm * ntn;
-    const int m0 = tm * GT, n0 = tn * GT;
-    const int beta = byz % ny, split = byz / ny;
-
-    // flat chunk index over the segments; this split takes a fixed contiguous range of it
-    // (segment values as scalars: a runtime-indexed local array would live in scratch memory)
-    const int nk20 = (g.seg[0].K2 + GKC - 1) / GKC, nk21 = g.nseg > 1 ? (g.seg[1].K2 + GKC - 1) / GKC : 1;
-    const int nch0 = g.seg[0].K1 * nk20, nch1 = g.nseg > 1 ? g.seg[1].K1 * nk21 : 0;
-    const int total = nch0 + nch1;
-    const int c_begin = (int)((int64_t)total * split / g.splits), c_end = (int)((int64_t)total * (split + 1) / g.splits);
-
-    d4 acc[2][2];
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++)
-            acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-    // MFMA blocks of this wave wholly past M or N are skipped (wave-uniform)
-    bool vm[2], vn[2];
-#pragma unroll
-    for (int x = 0; x < 2; x++) {
-        vm[x] = m0 + wm * 32 + x * 16 < g.M;
-        vn[x] = n0 + wn * 32 + x * 16 < g.N;
-    }
-
-    // two register sets: chunk c + 2 is loaded while chunk c is multiplied (c + 1 waits in the other)
-    double ra0[4], rb0[4], ra1[4], rb1[4];
-    auto fetch = [&](int ch, double *ra, double *rb) {
-        if (ch < nch0) {
-            const GemmSeg &sg = g.seg[0];
-            const int k1 = ch / nk20, k2c = ch - k1 * nk20;
-            fetch_op<A0>(sg.A, (int64_t)beta * sg.A.sb, m0, g.M, k1, k2c, sg.K2, ra, tid);
-            fetch_op<B0>(sg.B, (int64_t)beta * sg.B.sb, n0, g.N, k1, k2c, sg.K2, rb, tid);
-        } else {
-            const GemmSeg &sg = g.seg[1];
-            const int cl = ch - nch0, k1 = cl / nk21, k2c = cl - k1 * nk21;
-            fetch_op<A1>(sg.A, (int64_t)beta * sg.A.sb, m0, g.M, k1, k2c, sg.K2, ra, tid);
-            fetch_op<B1>(sg.B, (int64_t)beta * sg.B.sb, n0, g.N, k1, k2c, sg.K2, rb, tid);
-        }
-    };
-    int buf = 0;
-    auto step = [&](int ch, double *ra, double *rb) {
-        if (ch < nch0) {
-            stash_op<A0>(g.seg[0].A, ra, As[buf], tid);
-            stash_op<B0>(g.seg[0].B, rb, Bs[buf], tid);
-        } else {
-            stash_op<A1>(g.seg[1].A, ra, As[buf], tid);
-            stash_op<B1>(g.seg[1].B, rb, Bs[buf], tid);
-        }
-        __syncthreads();
-        if (ch + 2 < c_end)
-            fetch(ch + 2, ra, rb);
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int kk = t * 4 + (lane >> 4);
-            double af[2], bf[2];
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-                af[x] = As[buf][kk * GPITCH + wm * 32 + x * 16 + (lane & 15)];
-#pragma unroll
-            for (int y = 0; y < 2; y++)
-                bf[y] = Bs[buf][kk * GPITCH + wn * 32 + y * 16 + (lane & 15)];
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-                if (vm[x])
-#pragma unroll
-                    for (int y = 0; y < 2; y++)
-                        if (vn[y])
-                            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[x], bf[y], acc[x][y], 0, 0, 0);
-        }
-        buf ^= 1;
-    };
-    if (c_begin < c_end)
-        fetch(c_begin, ra0, rb0);
-    if (c_begin + 1 < c_end)
-        fetch(c_begin + 1, ra1, rb1);
-    for (int ch = c_begin; ch < c_end; ch += 2) {
-        step(ch, ra0, rb0);
-        if (ch + 1 < c_end)
-            step(ch + 1, ra1, rb1);
-    }
-
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++) {
-            const int n = n0 + wn * 32 + y * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 32 + x * 16 + (lane >> 4) + 4 * r;
-                if (m < g.M && n < g.N) {
-                    if (g.splits == 1) {
-                        double *cp = g.C + (int64_t)beta * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
-                        *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
-                    } else {
-                        g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
-                    }
-                }
-            }
-        }
-}
-
-// The same contraction for the layouts of the (T) back-contractions, with direct-to-LDS operand loads:
-// B has unit stride along n (rows of T2 and of the integral blocks), A (a gradient array G) unit stride
-// along m (AM = 0) or along k2 (AM = 1). A 16-deep chunk of a unit-stride-n (or m) operand is a [k][x]
-// tile of 16 rows of 64 doubles (32 sixteen-byte vectors, vector p of row k at slot p ^ 8 (k & 1)); of a
-// unit-stride-k operand a [m][k] tile of 64 rows of 16 doubles (8 vectors, vector p of row m at slot
-// p ^ ((m >> 1) & 7)). Both put the 16 lanes of every MFMA operand read on distinct banks. Loads go
-// global -> LDS (global_load_lds, 16 bytes per lane, 1 KiB per wave instruction) into a two-stage ring;
-// vectors past M or N are clamped into the padded rows (cext), B rows with k2 >= K2 to row K2 - 1 (A
-// reads zero there: kzero). Tiles, waves, MFMA blocks, splits and the store are those of gemm_kernel.
-constexpr int KN_TILE = 16 * 64;  // doubles per operand chunk (8 KiB)
-
-// source of the 16-byte vector that lane `lane` of wave load L (0..7) puts into an operand chunk;
-// mfold > 0 (A of a folded batch): tile row x is row x % mfold of batch entry x / mfold
-template <int MK, int W = 64>
-__device__ inline const double *kn_src(const GemmOp &op, int64_t base, int x0, int xext, int k1, int k2c, int K2, int L,
-                                       int lane, int mfold) {
-    if constexpr (MK) {  // [m][k] tile: wave load L covers rows 8 L .. 8 L + 7
-        const int mm = 8 * L + (lane >> 3), p = lane & 7;
-        const int lv = p ^ ((mm >> 1) & 7);
-        const int64_t k2 = min((int64_t)k2c * 16 + 2 * lv, op.cext - 2);
-        int m = min(x0 + mm, xext - 1);
-        if (mfold) {
-            const int b = m / mfold;
-            base += b * op.sb;
-            m -= b * mfold;
-        }
-        return op.base + base + (int64_t)m * op.sr + (int64_t)k1 * op.s1 + k2;
-    } else {  // [k][x] tile of W-double rows: wave load L covers rows 2 L, 2 L + 1 (W = 64) or row L (128)
-        const int kk = W == 64 ? 2 * L + (lane >> 5) : L, p = W == 64 ? lane & 31 : lane;
-        const int lv = p ^ ((kk & 1) << 3);
-        int64_t x;
-        if (mfold) {  // mfold is even, so the two rows of a vector lie in one batch entry
-            const int xf = min(x0 + 2 * lv, xext - 2), b = xf / mfold;
-            base += b * op.sb;
-            x = xf - b * mfold;
-        } else {
-            x = min((int64_t)x0 + 2 * lv, op.cext - 2);
-        }
-        const int k2 = op.kzero ? k2c * 16 + kk : min(k2c * 16 + kk, K2 - 1);
-        return op.base + base + (int64_t)k1 * op.s1 + (int64_t)k2 * op.s2 + x;
-    }
-}
-
-// element (x, k) of an operand chunk in LDS (x = row of A or B within the tile, k = 0..15; [k][x] tiles
-// with rows of W doubles)
-template <int MK, int W = 64> __device__ inline double kn_frag(const double *t, int x, int k) {
-    if constexpr (MK)
-        return t[x * 16 + (((k >> 1) ^ ((x >> 1) & 7)) << 1) + (k & 1)];
-    else
-        return t[k * W + (((x >> 1) ^ ((k & 1) << 3)) << 1) + (x & 1)];
-}
-
-// WIDE = 2: tiles of 64 rows by 128 columns (each wave 32 x 64, four B wave loads per chunk), twice the
-// MFMAs per barrier for 1.5x the staged bytes; two stages only.
-template <int AM0, int AM1, int NST, int WIDE>
-__global__ __launch_bounds__(256) void gemm_kn_kernel(GemmGroup gg) {
-    static_assert(NST == 2 || NST == 3, "stages");
-    static_assert(WIDE == 1 || (WIDE == 2 && NST == 2), "wide tiles: two stages");
-    constexpr int BW = 64 * WIDE, NBY = 2 * WIDE;  // tile columns; MFMA blocks per wave along n
-    __shared__ __attribute__((aligned(1024))) double lds[NST][KN_TILE + 16 * BW];  // [stage][A chunk, B chunk]
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int nx = gridDim.x, ny = gridDim.y;
-    const int lin = xcd_remap(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z), nx * ny * gridDim.z);
-    const int bx = lin % nx, byz = lin / nx;
-    const int beta = byz % ny, zz = byz / ny;
-    const int prob = zz % gg.n, split = zz / gg.n;
-    const GemmArgs &g = gg.g[prob];
-    const int ntn = (g.N + BW - 1) / BW;
-    const int tm = bx / ntn, tn = bx - tm * ntn;
-    const int m0 = tm * GT, n0 = tn * BW;
-
-    const int nk20 = (g.seg[0].K2 + 15) / 16, nk21 = g.nseg > 1 ? (g.seg[1].K2 + 15) / 16 : 1;
-    const int nch0 = g.seg[0].K1 * nk20, nch1 = g.nseg > 1 ? g.seg[1].K1 * nk21 : 0;
-    const int total = nch0 + nch1;
-    const int c_begin = (int)((int64_t)total * split / g.splits), c_end = (int)((int64_t)total * (split + 1) / g.splits);
-
-    d4 acc[2][NBY];
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < NBY; y++)
-            acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-    bool vm[2], vn[NBY];
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-        vm[x] = m0 + wm * 32 + x * 16 < g.M;
-#pragma unroll
-    for (int y = 0; y < NBY; y++)
-        vn[y] = n0 + wn * 32 * WIDE + y * 16 < g.N;
-
-    // wave loads 2 wave and 2 wave + 1 of the A chunk and 2 WIDE wave .. 2 WIDE wave + 2 WIDE - 1 of the
-    // B chunk are this wave's
-    auto issue_seg = [&](const GemmSeg &sg, auto amk, int cl, int nk2, int st) {
-        constexpr int MK = decltype(amk)::value;
-        const int k1 = cl / nk2, k2c = cl - k1 * nk2;
-        double *As = lds[st], *Bs = lds[st] + KN_TILE;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int L = 2 * wave + h;
-            const double *sa = kn_src<MK>(sg.A, (int64_t)beta * sg.A.sb, m0, g.M, k1, k2c, sg.K2, L, lane, g.mfold);
-            __builtin_amdgcn_global_load_lds((const void *)sa, (lds_void *)(As + L * 128), 16, 0, 0);
-        }
-#pragma unroll
-        for (int h = 0; h < 2 * WIDE; h++) {
-            const int L = 2 * WIDE * wave + h;
-            const double *sb = kn_src<0, BW>(sg.B, (int64_t)beta * sg.B.sb, n0, g.N, k1, k2c, sg.K2, L, lane, 0);
-            __builtin_amdgcn_global_load_lds((const void *)sb, (lds_void *)(Bs + L * 128), 16, 0, 0);
-        }
-    };
-    auto issue = [&](int ch, int st) {
-        if (ch < nch0)
-            issue_seg(g.seg[0], std::integral_constant<int, AM0>{}, ch, nk20, st);
-        else
-            issue_seg(g.seg[1], std::integral_constant<int, AM1>{}, ch - nch0, nk21, st);
-    };
-    auto compute = [&](int st, auto amk) {
-        constexpr int MK = decltype(amk)::value;
-        const double *As = lds[st], *Bs = lds[st] + KN_TILE;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int kk = t * 4 + (lane >> 4);
-            double af[2], bf[NBY];
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-                af[x] = kn_frag<MK>(As, wm * 32 + x * 16 + (lane & 15), kk);
-#pragma unroll
-            for (int y = 0; y < NBY; y++)
-                bf[y] = kn_frag<0, BW>(Bs, wn * 32 * WIDE + y * 16 + (lane & 15), kk);
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-                if (vm[x])
-#pragma unroll
-                    for (int y = 0; y < NBY; y++)
-                        if (vn[y])
-                            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[x], bf[y], acc[x][y], 0, 0, 0);
-        }
-    };
-#pragma unroll
-    for (int p = 0; p < NST - 1; p++)
-        if (c_begin + p < c_end)
-            issue(c_begin + p, p);
-    int st = 0;
-    for (int ch = c_begin; ch < c_end; ch++) {
-        // this wave's four loads per chunk: chunk ch has landed once only later chunks' are outstanding
-        if (NST > 2 && ch + 1 < c_end)
-            wait_vm<(NST > 2 ? 4 : 0)>();
-        else
-            wait_vm<0>();
-        __syncthreads();  // chunk ch is in LDS; the stage of chunk ch - 1 is free again
-        if (ch + NST - 1 < c_end)
-            issue(ch + NST - 1, st == 0 ? NST - 1 : st - 1);
-        if (ch < nch0)
-            compute(st, std::integral_constant<int, AM0>{});
-        else
-            compute(st, std::integral_constant<int, AM1>{});
-        st = st == NST - 1 ? 0 : st + 1;
-    }
-
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < NBY; y++) {
-            const int n = n0 + wn * 32 * WIDE + y * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 32 + x * 16 + (lane >> 4) + 4 * r;
-                if (m < g.M && n < g.N) {
-                    if (g.splits == 1) {
-                        int64_t row = (int64_t)beta * g.sCb + (int64_t)m * g.sCm;
-                        if (g.mfold) {  // row m of the folded batch: row m % mfold of entry m / mfold
-                            const int bq = m / g.mfold;
-                            row = (int64_t)bq * g.sCb + (int64_t)(m - bq * g.mfold) * g.sCm;
-                        }
-                        double *cp = g.C + row + (int64_t)n * g.sCn;
-                        *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
-                    } else {
-                        g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
-                    }
-                }
-            }
-        }
-}
-
-// (blockIdx.y: batch entry; only gemm_nt_kernel has more than one)
+// -------------------------------------------------------------------- GEMM
+// C[b][m][n] += alpha sum_seg sum_k1 sum_k2 A(m, k1, k2) B(n, k1, k2); with splits > 1, split p handles a fixed contiguous
+// range of the 16-deep K chunks and writes its partial to scratch[p]; gemm_reduce_kernel adds them in split order.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (int64_t)g.M * g.N)
@@ -619,32 +221,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     for (; p < g.splits; p++)
         s += src[(int64_t)p * mn];
     double *cp = g.C + (int64_t)blockIdx.y * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
-    *cp = g.ow ? g.alpha * s : *cp + g.alpha * s;
-}
-
-// gemm_reduce_kernel for problem blockIdx.y of a group
-__global__ __launch_bounds__(256) void gemm_reduce_group_kernel(GemmGroup gg) {
-    const GemmArgs &g = gg.g[blockIdx.y];
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)g.M * g.N)
-        return;
-    const int m = (int)(idx / g.N), n = (int)(idx - (int64_t)m * g.N);
-    const int64_t mn = (int64_t)g.M * g.N;
-    const double *src = g.scratch + idx;
-    double s = 0.0;
-    int p = 0;
-    for (; p + 8 <= g.splits; p += 8) {  // eight loads in flight, added in split order
-        double x[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            x[u] = src[(int64_t)(p + u) * mn];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            s += x[u];
-    }
-    for (; p < g.splits; p++)
-        s += src[(int64_t)p * mn];
-    double *cp = g.C + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
     *cp = g.ow ? g.alpha * s : *cp + g.alpha * s;
 }
 
@@ -1276,50 +852,6 @@ static int k_contiguous(const GemmArgs &g) {
     return r;
 }
 
-// Paired-load mode of one operand: 1 rows contiguous, 2 K contiguous (both with even strides and a
-// 16-byte aligned base), 0 otherwise
-static int pair_mode(const GemmOp &op) {
-    const bool even = !(op.s1 & 1) && !(op.sb & 1) && !(((uintptr_t)op.base) & 15);
-    if (even && op.sr == 1 && !(op.s2 & 1))
-        return 1;
-    if (even && op.s2 == 1 && !(op.sr & 1))
-        return 2;
-    return 0;
-}
-
-// Whether gemm_kn_kernel applies (FP64 products, B of unit stride in n, A of unit stride in m or in
-// k2, every stride and base even so that operand vectors are 16-byte aligned, padded extents known, A
-// zero past K2): 0 if not, else 1 + (segment 0's A unit-stride in k2) + 2 (segment 1's).
-// SCESS_GEMM_KN=0 keeps the register-staged kernel.
-static int kn_modes(const GemmArgs &g) {
-    if (g.prec != P64)
-        return 0;
-    if (const char *e = std::getenv("SCESS_GEMM_KN"))
-        if (std::atoi(e) == 0)
-            return 0;
-    auto even = [](const GemmOp &op) {
-        return !(op.sr & 1) || op.sr == 1 ? !(op.s1 & 1) && !(op.sb & 1) && !(((uintptr_t)op.base) & 15) : false;
-    };
-    int am = 1;
-    for (int q = 0; q < g.nseg; q++) {
-        const GemmOp &A = g.seg[q].A, &B = g.seg[q].B;
-        if (B.sr != 1 || (B.s2 & 1) || B.cext < 2 || (B.cext & 1) || !even(B) || g.seg[q].K2 < 1 || g.seg[q].K1 < 1)
-            return 0;
-        if (!A.kzero || A.cext < 2 || (A.cext & 1) || !even(A))
-            return 0;
-        if (A.sr == 1 && !(A.s2 & 1))
-            continue;  // [k][m] tile
-        if (A.s2 == 1 && !(A.sr & 1) && A.cext >= (g.seg[q].K2 + 15) / 16 * 16) {
-            am += q == 0 ? 1 : 2;  // [m][k] tile
-            continue;
-        }
-        return 0;
-    }
-    if (g.nseg == 1 && am == 2)
-        am = 4;  // segment 1 is not used: give it segment 0's mode
-    return am;
-}
-
 hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
     {  // the kernels index K chunks (16 deep) with 32-bit integers
         int64_t chunks = 0;
@@ -1328,76 +860,47 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
         if (chunks >= (int64_t)1 << 31 || g.nseg < 1 || g.nseg > 2)
             return hipErrorInvalidValue;
     }
-    if (const int kc = k_contiguous(g)) {
-        // FP64: 128 x 128 tiles; rows of a tile at lane offsets of 32 bits
-        const GemmSeg &s0 = g.seg[0];
-        const double far = 128.0 * 8.0 * (double)std::max(s0.A.sr, s0.B.sr);
-        if (g.prec == P64 && kc == 2 && g.nseg == 1 && s0.K2 >= 1 && s0.K1 >= 1 && g.M >= 1 && g.N >= 1 &&
-            s0.A.sr >= 0 && s0.B.sr >= 0 && far < 4294967296.0) {
-            const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
-            if (tiles > 0x7fffffff)
-                return hipErrorInvalidValue;
-            hipLaunchKernelGGL(gemm_nt_kernel, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256), 0, s,
-                               g);
-        } else {
-        // 64x64 tiles: for FP64 MFMA more resident work-groups beat larger register tiles
-        int blk = 2;
-        if (const char *e = std::getenv("SCESS_GEMM_BLK"))  // tuning override: 2 or 4 (FP64 only)
-            blk = std::atoi(e) == 4 && g.prec == P64 ? 4 : 2;
-        const int bm = 32 * blk;
-        const int nt = ((g.M + bm - 1) / bm) * ((g.N + bm - 1) / bm);
+    const int kc = k_contiguous(g);
+    if (!kc)  // the callers lay their operands out with K contiguous
+        return hipErrorInvalidValue;
+    // FP64: 128 x 128 tiles, unless rows of a tile are too far apart for lane offsets of 32 bits
+    const GemmSeg &s0 = g.seg[0];
+    const double far = 128.0 * 8.0 * (double)std::max(s0.A.sr, s0.B.sr);
+    if (g.prec == P64 && kc == 2 && g.nseg == 1 && s0.K2 >= 1 && s0.K1 >= 1 && g.M >= 1 && g.N >= 1 && s0.A.sr >= 0 &&
+        s0.B.sr >= 0 && far < 4294967296.0) {
+        const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+        if (tiles > 0x7fffffff)
+            return hipErrorInvalidValue;
+        hipLaunchKernelGGL(gemm_nt_kernel, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256), 0, s, g);
+    } else {
+        // 64 x 64 tiles
+        const int nt = ((g.M + 63) / 64) * ((g.N + 63) / 64);
         const dim3 grid((unsigned)nt, (unsigned)batch, (unsigned)g.splits);
-        // direct-to-LDS loads when the rows are 16-byte vectors and at least two elements long (the first
-        // vector of every row is then inside it); SCESS_GEMM_DMA=0 keeps the register-staged loads
-        bool dma = kc == 2 && blk == 2;
+        // direct-to-LDS loads when the rows are 16-byte vectors and at least two elements long (the first vector of every
+        // row is then inside it); SCESS_GEMM_DMA=0 keeps the register-staged loads of the other precisions (tuning)
+        bool dma = kc == 2 && g.M >= 1 && g.N >= 1;
         for (int q = 0; q < g.nseg; q++)
-            dma = dma && g.seg[q].K2 >= 2 && g.M >= 1 && g.N >= 1;
+            dma = dma && g.seg[q].K2 >= 2;
         if (const char *e = std::getenv("SCESS_GEMM_DMA"))
-            dma = dma && std::atoi(e) != 0;
-        // 64 x 128 tiles for the direct-to-LDS FP64 and pre-split BF16x3 products: twice the MFMAs per
-        // barrier for 1.5x the staged bytes (CCSD update at o=50, v=500: FP64 17.9 s against 19.5 s,
-        // BF16x3 6.66 s against 7.47 s with 64 x 64). SCESS_GEMM_WIDE=0 keeps 64 x 64 (tuning).
+            dma = dma && (g.prec == P64 || std::atoi(e) != 0);
+        const bool vec = kc == 2 && (g.prec != P64 || dma);
+        // 64 x 128 tiles for the direct-to-LDS pre-split BF16x3 products: twice the MFMAs per barrier for 1.5x the staged
+        // bytes (CCSD update at o=50, v=500: 6.66 s against 7.47 s with 64 x 64). SCESS_GEMM_WIDE=0 keeps 64 x 64 (tuning).
         const char *ew = std::getenv("SCESS_GEMM_WIDE");
-        const bool wide = dma && blk == 2 && (g.prec == P64 || g.prec == PB3S) && !(ew && std::atoi(ew) == 0);
-#define SCESS_KC(B, V, P, D)                                                                      \
-    if (blk == B && (kc == 2) == V && g.prec == P && dma == D) {                                  \
-        hipLaunchKernelGGL((gemm_kc_kernel<B, V, P, D, 1>), grid, dim3(256), 0, s, g);            \
+        const bool wide = dma && g.prec == PB3S && !(ew && std::atoi(ew) == 0);
+#define SCESS_KC(V, P, D)                                                                         \
+    if (vec == V && g.prec == P && dma == D) {                                                    \
+        hipLaunchKernelGGL((gemm_kc_kernel<2, V, P, D, 1>), grid, dim3(256), 0, s, g);            \
     } else
-        if (wide) {  // 64 x 128 tiles
+        if (wide) {
             const dim3 gw((unsigned)(((g.M + 63) / 64) * ((g.N + 127) / 128)), (unsigned)batch, (unsigned)g.splits);
-            if (g.prec == PB3S)
-                hipLaunchKernelGGL((gemm_kc_kernel<2, true, PB3S, true, 2>), gw, dim3(256), 0, s, g);
-            else
-                hipLaunchKernelGGL((gemm_kc_kernel<2, true, P64, true, 2>), gw, dim3(256), 0, s, g);
+            hipLaunchKernelGGL((gemm_kc_kernel<2, true, PB3S, true, 2>), gw, dim3(256), 0, s, g);
         } else
-        SCESS_KC(2, true, P64, true) SCESS_KC(2, true, P32, true) SCESS_KC(2, true, PB3, true)
-        SCESS_KC(2, true, PB3S, true) SCESS_KC(2, true, PB3S, false)
-        SCESS_KC(2, true, P64, false) SCESS_KC(2, false, P64, false) SCESS_KC(2, true, P32, false)
-        SCESS_KC(2, false, P32, false) SCESS_KC(2, true, PB3, false) SCESS_KC(2, false, PB3, false)
-        SCESS_KC(4, true, P64, false) SCESS_KC(4, false, P64, false)
+        SCESS_KC(true, P64, true) SCESS_KC(true, P32, true) SCESS_KC(true, PB3, true) SCESS_KC(true, PB3S, true)
+        SCESS_KC(true, PB3S, false) SCESS_KC(true, P32, false) SCESS_KC(true, PB3, false)
+        SCESS_KC(false, P64, false) SCESS_KC(false, P32, false) SCESS_KC(false, PB3, false)
         return hipErrorInvalidValue;
 #undef SCESS_KC
-        }
-    } else if (kn_modes(g)) {
-        GemmGroup gg;
-        gg.g[0] = g;
-        gg.n = 1;
-        return launch_gemm_group(gg, batch, s);
-    } else {
-        const int ntiles = ((g.M + GT - 1) / GT) * ((g.N + GT - 1) / GT);
-        const dim3 grid((unsigned)ntiles, (unsigned)batch, (unsigned)g.splits);
-        int a0 = pair_mode(g.seg[0].A), b0 = pair_mode(g.seg[0].B);
-        int a1 = g.nseg > 1 ? pair_mode(g.seg[1].A) : a0, b1 = g.nseg > 1 ? pair_mode(g.seg[1].B) : b0;
-        if (!a0 || !a1 || !b0 || !b1 || b0 != b1)
-            a0 = a1 = b0 = b1 = 0;  // element-wise loads for every operand
-#define SCESS_GP(A0, A1, B)                                                                       \
-    if (a0 == A0 && a1 == A1 && b0 == B) {                                                        \
-        hipLaunchKernelGGL((gemm_kernel<A0, A1, B, B>), grid, dim3(256), 0, s, g);                \
-    } else
-        SCESS_GP(1, 1, 1) SCESS_GP(1, 2, 1) SCESS_GP(2, 1, 1) SCESS_GP(2, 2, 1)
-        SCESS_GP(1, 1, 2) SCESS_GP(1, 2, 2) SCESS_GP(2, 1, 2) SCESS_GP(2, 2, 2)
-        hipLaunchKernelGGL((gemm_kernel<0, 0, 0, 0>), grid, dim3(256), 0, s, g);
-#undef SCESS_GP
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || g.splits == 1)
@@ -1407,108 +910,452 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
     return hipGetLastError();
 }
 
-static hipError_t launch_kn_group(const GemmGroup &gg0, int am, int batch, hipStream_t s) {
-    // A batch whose B operands do not depend on the batch index (the dX and dTM back-contractions) is
-    // folded into the rows: M' = M x batch rows of 64-row tiles leave one partly filled tile instead of
-    // one per batch entry (at v = 200 the fourth tile of every entry holds 8 rows). Needs M even (the
-    // two rows of a 16-byte A vector then share a batch entry) and one split.
-    GemmGroup gg = gg0;
-    const char *ef = std::getenv("SCESS_KN_FOLD");  // tuning override: 0 keeps one tile row set per entry
-    bool fold = batch > 1 && !(ef && std::atoi(ef) == 0);
-    for (int p = 0; p < gg.n && fold; p++) {
-        const GemmArgs &q = gg.g[p];
-        fold = q.splits == 1 && q.M % 2 == 0 && (int64_t)q.M * batch < ((int64_t)1 << 30);
-        for (int h = 0; h < q.nseg && fold; h++)
-            fold = q.seg[h].B.sb == 0;
+// -------------------------------------------------- back-contractions of a batch
+// With c one of the three positions of a triple's G and a, b the others, the six terms of all four gradients read G in
+// two ways only, each against two operands side by side as v8 + o8 columns (v, o rounded up to 8):
+//   rows (x_p, x_b), K = x_c:  dX[p][x_p][x_b][f] | dTM[p][x_b][x_p][m] += G (T[c][b][x_c][f] | Rn[c][b][x_c][m])
+//   rows x_c, K = (x_a, x_b):  dT[c][b][x_c][f]   | dRn[c][b][x_c][m]   += G (X[a][x_a][x_b][f] | TM[a][x_b][x_a][m])
+// (p, b, c and a, b, c stand for a position and its occupied index). The first kind runs over all triples of the batch
+// with the same p in one go: its output, the size of G, is read and written once per batch and p instead of once per
+// term. The second kind is split over ranges of the outer K index into partials, added in order by back_reduce_kernel.
+// A row group is 8 rows along the unit-stride position of G where that is a row (K otherwise). Position 2 may be p or b,
+// and all terms of one output tile need the same row order: the terms with p at position 2 make a launch of their own.
+//
+// One work-group makes a tile of up to 8 x 8 blocks of 16; the four waves own its rows in slabs, all columns each. The
+// loop is that of gemm_nt_kernel (look-ahead of one k-step, one barrier per 16 k, two work-groups per CU); a chunk of G is
+// a [m][k] tile (128-byte rows, vectors swizzled by kswz) where k has unit stride, else a [k][m] tile like B's [k][n],
+// with the pairs of odd k 16 elements apart from those of even k. Bound by the FP64 matrix pipes.
+// Gradients of a shard (190 triples) of o=20, v=200: 141 ms in back_kernel, 57 TFLOP/s of useful products (one GEMM group
+// per kind and triple before: 350 ms); o=10, v=75 (210 triples): 5.1 ms against 32 and 2520 fewer launches.
+constexpr int kBackOp = 16 * 128 * 8;  // bytes of an operand's chunk
+
+template <int RB, int CB> struct BackGemm {
+    const BackArgs &a;
+    char *lds;
+    int lane, wave;
+    // rows: groups of 8 with coordinates (X, Y); gx, gy of the four loads of a [m][k] chunk, lx, ly of a [k][m] one
+    int gx[4], gy[4], lx, ly;
+    int n;        // first of this lane's two columns
+    int block0;   // first row block of the wave's slab
+    bool rows2, second;  // second: the K = (x_a, x_b) kind; rows2: p at position 2
+    // next chunk to load
+    const BackSeg *sg;
+    int segs, k1, k1n, k2c, nk2;
+    bool mc;
+    const double *pa[4], *pb;
+    int64_t da, a1, b1, b2;  // advance of G per chunk and of G and B per outer k, B's per k
+
+    __device__ inline int64_t pos(int q) const { return q == 0 ? (int64_t)a.vR * a.vR : q == 1 ? a.vR : 1; }
+
+    __device__ inline void setup() {
+        // a scalar load: the wait of a vector load would be one for the chunks in flight, too
+        const auto *seg = (const __attribute__((address_space(4))) int *)(uintptr_t)sg;
+        const int slot = seg[0], code = seg[1];
+        const int64_t occ = seg[2], v = a.v;
+        const int P = code & 3, B = (code >> 2) & 3, C = code >> 4;
+        const double *G = a.G + slot * a.gstride;
+        int64_t sX, sY, sk;
+        const bool inv = n < a.v8;
+        k2c = 0;
+        if (!second) {
+            mc = C != 2;
+            sX = pos(rows2 ? B : P);
+            sY = pos(rows2 ? P : B);
+            sk = pos(C);
+            a1 = b1 = 0;
+            k1n = 1;
+            b2 = inv ? a.vK : a.oK;
+            pb = inv ? a.T + occ * v * a.vK + n : a.Rn + occ * v * a.oK + (n - a.v8);
+        } else {
+            // P: position of x_a; the inner K index is at position 2, or at 1 where that is the row
+            mc = C == 2;
+            const int in = mc ? 1 : 2;
+            const bool ina = P == in;
+            sX = 0;
+            sY = pos(C);
+            sk = pos(in);
+            a1 = pos(ina ? B : P);
+            const int64_t ba = inv ? v * a.vK : a.oK, bb = inv ? a.vK : v * a.oK;
+            b2 = ina ? ba : bb;
+            b1 = ina ? bb : ba;
+            pb = inv ? a.X + occ * v * v * a.vK + n : a.TM + occ * v * v * a.oK + (n - a.v8);
+            pb += k1 * b1;
+            G += k1 * a1;
+        }
+        if (mc) {
+            da = 16 * sk;
+#pragma unroll
+            for (int h = 0; h < 4; h++)
+                pa[h] = G + lx * sX + ly + (wave + 4 * h) * sk;
+        } else {
+            da = 16;
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                const int r = 8 * (wave + 4 * h) + (lane >> 3);
+                pa[h] = G + gx[h] * sX + (gy[h] + (lane >> 3)) * sY + 2 * ((lane & 7) ^ kswz(r & 15));
+            }
+        }
     }
-    if (fold) {
-        for (int p = 0; p < gg.n; p++) {
-            gg.g[p].mfold = gg.g[p].M;
-            gg.g[p].M *= batch;
+
+    // the next chunk into stage st: returns its k-steps, bit 3: a [k][m] chunk, bit 4: there is another
+    __device__ inline int issue(int st) {
+        char *base = lds + st * 2 * kBackOp;
+        const int left = a.v - 16 * k2c, ret = (min(left, 16) + 3) >> 2 | (mc ? 8 : 0);
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            const int u = wave + 4 * h;
+            __builtin_amdgcn_global_load_lds((const void *)pa[h], (lds_void *)(base + u * 1024), 16, 0, 0);
+            // k past v: the last row again, times zeros of G
+            __builtin_amdgcn_global_load_lds((const void *)(pb + (int64_t)min(16 * k2c + u, a.v - 1) * b2),
+                                             (lds_void *)(base + kBackOp + u * 1024), 16, 0, 0);
         }
-        batch = 1;
+#pragma unroll
+        for (int h = 0; h < 4; h++)
+            pa[h] += da;
+        if (++k2c < nk2)
+            return ret | 16;
+        k2c = 0;
+        if (++k1 < k1n) {
+#pragma unroll
+            for (int h = 0; h < 4; h++)
+                pa[h] += a1 - nk2 * da;
+            pb += b1;
+            return ret | 16;
+        }
+        if (--segs == 0)
+            return ret;
+        sg++;
+        k1 = 0;
+        setup();
+        return ret | 16;
     }
-    const GemmArgs &g = gg.g[0];
-    // am: 1 + (A of segment 0 unit-stride in k) + 2 (A of segment 1 unit-stride in k)
-    const char *e3 = std::getenv("SCESS_KN_STAGES");  // tuning override: 2 or 3 LDS stages
-    const char *ew = std::getenv("SCESS_KN_WIDE");    // tuning override: 1 for 64 x 128 tiles
-    const bool three = e3 && std::atoi(e3) == 3;
-    // 64 x 128 tiles where N spans more than one 64-wide tile: slower here (4.07 s per backward at o=20,
-    // v=200 against 3.70 s), as fewer resident work-groups cost these short-K GEMMs more than the MFMAs
-    // per barrier gain
-    const bool wide = !three && g.N > 64 && ew && std::atoi(ew) == 1;
-    const int ntiles = ((g.M + GT - 1) / GT) * ((g.N + (wide ? 2 * GT : GT) - 1) / (wide ? 2 * GT : GT));
-    const dim3 grid((unsigned)ntiles, (unsigned)batch, (unsigned)(g.splits * gg.n));
-    if (wide) {
-        switch (am) {
-        case 1: hipLaunchKernelGGL((gemm_kn_kernel<0, 0, 2, 2>), grid, dim3(256), 0, s, gg); break;
-        case 2: hipLaunchKernelGGL((gemm_kn_kernel<1, 0, 2, 2>), grid, dim3(256), 0, s, gg); break;
-        case 3: hipLaunchKernelGGL((gemm_kn_kernel<0, 1, 2, 2>), grid, dim3(256), 0, s, gg); break;
-        default: hipLaunchKernelGGL((gemm_kn_kernel<1, 1, 2, 2>), grid, dim3(256), 0, s, gg); break;
+
+    template <class Store> __device__ inline void run(Store &&store) {
+        d4 acc[RB][CB];
+        double fr[2][RB], fc[2][CB];
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = d4{};
+        const int lr = lane & 15, lq = lane >> 4;
+        uint32_t km[4], mk[RB], cn[2];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            km[t] = (block0 * 16 + lr) * 128 + ((2 * t + (lq >> 1)) ^ kswz(lr)) * 16 + (lq & 1) * 8;
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+            mk[x] = lq * 1024 + lr * 8 + ((block0 + x) ^ (lq & 1)) * 128;
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+            cn[y] = kBackOp + lq * 1024 + lr * 8 + (y ^ (lq & 1)) * 128;
+        lds_char *q;
+        auto read = [&](auto tc, int buf, int flags) {
+            constexpr int t = decltype(tc)::value;
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+                fr[buf][x] = *(lds_double *)(q + (flags & 8 ? mk[x] + t * 4096 : km[t] + x * 2048));
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[buf][y] = *(lds_double *)(q + cn[y & 1] + (y & ~1) * 128 + t * 4096);
+        };
+        auto row = [&](int buf, int x) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[buf][x], fc[buf][y], acc[x][y], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int cur, nxt = 0;
+        auto step = [&](int buf, auto tc) {
+            row(buf, 0);
+            read(tc, buf ^ 1, cur);
+#pragma unroll
+            for (int x = 1; x < RB; x++)
+                row(buf, x);
+        };
+        auto move = [&]() {
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+                fr[1][x] = fr[0][x];
+#pragma unroll
+            for (int y = 0; y < CB; y++)
+                fc[1][y] = fc[0][y];
+        };
+        using std::integral_constant;
+        setup();
+        cur = issue(0);
+        if (cur & 16)
+            nxt = issue(1);
+        wait_vm_lgkm0();
+        __syncthreads();
+        q = (lds_char *)lds;
+        read(integral_constant<int, 0>{}, 0, cur);
+        for (int st = 0;; st ^= 1) {
+            const int steps = cur & 7;
+            if (steps >= 2) {
+                step(0, integral_constant<int, 1>{});
+                if (steps >= 3) {
+                    step(1, integral_constant<int, 2>{});
+                    if (steps == 4)
+                        step(0, integral_constant<int, 3>{});
+                    else
+                        move();
+                }
+            } else {
+                move();
+            }
+            const bool more = cur & 16;
+            if (more) {
+                wait_vm_lgkm0();
+                __syncthreads();
+            }
+            row(1, 0);
+            if (more) {
+                q = (lds_char *)lds + (st ^ 1) * 2 * kBackOp;
+                read(integral_constant<int, 0>{}, 0, nxt);
+            }
+            cur = nxt;
+            if (more && (nxt & 16))
+                nxt = issue(st);
+#pragma unroll
+            for (int x = 1; x < RB; x++)
+                row(1, x);
+            if (!more)
+                break;
         }
-    } else if (three) {
-        switch (am) {
-        case 1: hipLaunchKernelGGL((gemm_kn_kernel<0, 0, 3, 1>), grid, dim3(256), 0, s, gg); break;
-        case 2: hipLaunchKernelGGL((gemm_kn_kernel<1, 0, 3, 1>), grid, dim3(256), 0, s, gg); break;
-        case 3: hipLaunchKernelGGL((gemm_kn_kernel<0, 1, 3, 1>), grid, dim3(256), 0, s, gg); break;
-        default: hipLaunchKernelGGL((gemm_kn_kernel<1, 1, 3, 1>), grid, dim3(256), 0, s, gg); break;
-        }
+        store(acc);
+    }
+};
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void back_kernel(BackArgs a) {
+    __shared__ __attribute__((aligned(1024))) char lds[4 * kBackOp];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nc = a.v8 + a.o8, nbn = (nc + 15) >> 4, ntn = (nbn + 7) >> 3;
+    const bool second = (int)blockIdx.x >= a.blocks1;
+    // Blocks b, b + 8, ... run on one XCD. First kind: the column tiles of a row tile there, one after another (they share
+    // its rows of G); second kind: all tiles of one K range.
+    int tm, tn, nbm, ngy, ngrp, seg0, segs, k10 = 0, k1n = 1, id = 0, part = 0;
+    if (!second) {
+        const int t = (int)blockIdx.x / a.per, l = (int)blockIdx.x - t * a.per, slot = l >> 3;
+        const BackTarget tg = a.tg[t];
+        id = tg.id;
+        seg0 = tg.seg0;
+        segs = tg.nseg;
+        ngy = a.v8 >> 3;
+        ngrp = a.v * ngy;
+        nbm = (ngrp + 1) >> 1;
+        tm = slot / ntn * 8 + (l & 7);
+        tn = slot % ntn;
     } else {
-        switch (am) {
-        case 1: hipLaunchKernelGGL((gemm_kn_kernel<0, 0, 2, 1>), grid, dim3(256), 0, s, gg); break;
-        case 2: hipLaunchKernelGGL((gemm_kn_kernel<1, 0, 2, 1>), grid, dim3(256), 0, s, gg); break;
-        case 3: hipLaunchKernelGGL((gemm_kn_kernel<0, 1, 2, 1>), grid, dim3(256), 0, s, gg); break;
-        default: hipLaunchKernelGGL((gemm_kn_kernel<1, 1, 2, 1>), grid, dim3(256), 0, s, gg); break;
-        }
+        ngy = ngrp = a.v8 >> 3;
+        nbm = (ngrp + 1) >> 1;
+        const int tiles = ((nbm + 7) >> 3) * ntn, l = (int)blockIdx.x - a.blocks1, slot = l >> 3, t = slot % tiles;
+        part = slot / tiles * 8 + (l & 7);
+        if (part >= a.nseg2 * a.splits)
+            return;
+        tm = t / ntn;
+        tn = t % ntn;
+        seg0 = a.seg2 + part / a.splits;
+        segs = 1;
+        const int sp = part % a.splits;
+        k10 = (int)((int64_t)a.v * sp / a.splits);
+        k1n = (int)((int64_t)a.v * (sp + 1) / a.splits);
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || g.splits == 1)
-        return e;
-    const int64_t n = (int64_t)g.M * g.N;
-    hipLaunchKernelGGL(gemm_reduce_group_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)gg.n), dim3(256), 0, s,
-                       gg);
-    return hipGetLastError();
+    const int ntm = (nbm + 7) >> 3;
+    if (tm >= ntm)
+        return;
+    const int am = (int)((int64_t)tm * nbm / ntm), rb = (int)((int64_t)(tm + 1) * nbm / ntm) - am;
+    const int an = (int)((int64_t)tn * nbn / ntn), cb = (int)((int64_t)(tn + 1) * nbn / ntn) - an;
+    const int slab = (wave + (blockIdx.x >> 3)) & 3;  // the uneven slabs of neighbouring tiles on different SIMDs
+    const int sb0 = slab * rb >> 2, nr = ((slab + 1) * rb >> 2) - sb0;
+    auto go = [&](auto rbc, auto cbc) {
+        constexpr int RB = decltype(rbc)::value, CB = decltype(cbc)::value;
+        BackGemm<RB, CB> w{a, lds};
+        w.lane = lane;
+        w.wave = wave;
+        w.second = second;
+        w.rows2 = a.rows2;
+        w.block0 = nr > 0 ? sb0 : 0;
+        // column pair at slot `lane` of the rows of odd or even k (those of this wave), past the end: the last pair
+        const int pair = lane ^ ((wave & 1) << 3);
+        w.n = min(16 * an + 2 * pair, nc - 2);
+        {
+            const int g = min(2 * am + (pair >> 2), ngrp - 1);
+            w.lx = g / ngy;
+            w.ly = (g - w.lx * ngy) * 8 + ((2 * pair) & 7);
+        }
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            const int g = min(2 * am + wave + 4 * h, ngrp - 1);
+            w.gx[h] = g / ngy;
+            w.gy[h] = (g - w.gx[h] * ngy) * 8;
+        }
+        w.sg = a.segs + seg0;
+        w.segs = segs;
+        w.k1 = k10;
+        w.k1n = k1n;
+        w.nk2 = (a.v + 15) >> 4;
+        w.run([&](d4 (&acc)[RB][CB]) {
+            if (nr == 0)  // ran for its loads and barriers
+                return;
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // keeps the store addresses from being formed, and held, before the loop
+            const int lr = ln & 15, lq = ln >> 4;
+            const int n0 = 16 * an + lr;
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    // row lq + 4 r of the block: group 2 x + (r >> 1)
+                    const int g = 2 * (am + sb0 + x) + (r >> 1);
+                    const int X = g / ngy, Y = (g - X * ngy) * 8 + lq + 4 * (r & 1);
+                    if (g >= ngrp || Y >= a.v)
+                        continue;
+                    double *c0, *c1;
+                    if (second) {
+                        c0 = c1 = a.scr + ((int64_t)part * a.v + Y) * nc + n0;
+                    } else {
+                        const int64_t xp = a.rows2 ? Y : X, xb = a.rows2 ? X : Y;
+                        c0 = a.dX + ((id * (int64_t)a.v + xp) * a.v + xb) * a.vK + n0;
+                        c1 = a.dTM + ((id * (int64_t)a.v + xb) * a.v + xp) * a.oK + (n0 - a.v8);
+                    }
+                    // the old values of the row in flight together
+                    double old[CB];
+#pragma unroll
+                    for (int y = 0; y < CB; y++) {
+                        const int n = n0 + 16 * y;
+                        old[y] = 0.0;
+                        if (!second && (n < a.v8 ? n < a.v : n - a.v8 < a.o))
+                            old[y] = (n < a.v8 ? c0 : c1)[16 * y];
+                    }
+#pragma unroll
+                    for (int y = 0; y < CB; y++) {
+                        const int n = n0 + 16 * y;
+                        if (n < a.v8 ? n < a.v : n - a.v8 < a.o)
+                            (n < a.v8 ? c0 : c1)[16 * y] = old[y] + acc[x][y][r];
+                    }
+                }
+        });
+    };
+    using std::integral_constant;
+    auto cols = [&](auto rbc) {
+        switch (cb) {
+        case 8: go(rbc, integral_constant<int, 8>{}); break;
+        case 7: go(rbc, integral_constant<int, 7>{}); break;
+        case 6: go(rbc, integral_constant<int, 6>{}); break;
+        case 5: go(rbc, integral_constant<int, 5>{}); break;
+        case 4: go(rbc, integral_constant<int, 4>{}); break;
+        case 3: go(rbc, integral_constant<int, 3>{}); break;
+        case 2: go(rbc, integral_constant<int, 2>{}); break;
+        default: go(rbc, integral_constant<int, 1>{}); break;
+        }
+    };
+    if (nr == 2)
+        cols(integral_constant<int, 2>{});
+    else
+        cols(integral_constant<int, 1>{});
 }
 
-hipError_t launch_gemm_group(const GemmGroup &gg, int batch, hipStream_t s) {
-    if (gg.n < 1 || gg.n > kMaxGemmGroup)
-        return hipErrorInvalidValue;
-    const GemmArgs &g0 = gg.g[0];
-    for (int p = 1; p < gg.n; p++)  // one shape per group
-        if (gg.g[p].M != g0.M || gg.g[p].N != g0.N || gg.g[p].splits != g0.splits)
-            return hipErrorInvalidValue;
-    for (int p = 0; p < gg.n; p++) {
-        int64_t chunks = 0;  // the kernels index K chunks (16 deep) with 32-bit integers
-        for (int q = 0; q < gg.g[p].nseg; q++)
-            chunks += (int64_t)gg.g[p].seg[q].K1 * ((gg.g[p].seg[q].K2 + 15) / 16);
-        if (chunks >= (int64_t)1 << 31 || gg.g[p].nseg < 1 || gg.g[p].nseg > 2)
-            return hipErrorInvalidValue;
+// dT, dRn of target blockIdx.y += the partials of its segments, in order
+__global__ __launch_bounds__(256) void back_reduce_kernel(BackArgs a, const BackTarget *tg, double *dT, double *dRn) {
+    const int nc = a.v8 + a.o8;
+    const int idx = blockIdx.x * 256 + threadIdx.x, m = idx / nc, n = idx - m * nc;
+    if (m >= a.v || (n < a.v8 ? n >= a.v : n - a.v8 >= a.o))
+        return;
+    const BackTarget t = tg[blockIdx.y];
+    const int64_t step = (int64_t)a.v * nc;
+    const double *p = a.scr + (int64_t)(t.seg0 - a.seg2) * a.splits * step + idx;
+    double s = 0.0;
+    int q = 0;
+    for (; q + 8 <= t.nseg * a.splits; q += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            x[u] = p[(q + u) * step];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            s += x[u];
     }
-    // one launch per operand layout class (problems keep their relative order; outputs are disjoint)
-    bool done[kMaxGemmGroup] = {};
-    for (int p = 0; p < gg.n; p++) {
-        if (done[p])
-            continue;
-        const int am = kn_modes(gg.g[p]);
-        if (!am) {
-            hipError_t e = launch_gemm(gg.g[p], batch, s);  // not a direct-to-LDS layout
-            if (e != hipSuccess)
-                return e;
-            done[p] = true;
-            continue;
+    for (; q < t.nseg * a.splits; q++)
+        s += p[q * step];
+    double *c = n < a.v8 ? dT + ((int64_t)t.id * a.v + m) * a.vK + n : dRn + ((int64_t)t.id * a.v + m) * a.oK + n - a.v8;
+    *c += s;
+}
+
+// The terms of triples work[0..n) (occupied indices, 3 each) as segments and targets
+void back_terms(const int *ijk, int n, int o, BackTables &t, BackBatch &b) {
+    // positions (P, B, C) of the six terms; with i == j (positions 0 and 1 alike) terms 4, 1, 3 equal 0, 2, 5
+    static const int TERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 2, 0}, {2, 0, 1}, {1, 0, 2}, {2, 1, 0}};
+    static const bool TWIN[6] = {true, false, true, false, false, true};
+    struct Entry {
+        int id;
+        BackSeg s;
+    };
+    std::vector<Entry> e[3];  // first kind with p at position 0 or 1, first kind with p at position 2, second kind
+    for (int w = 0; w < n; w++) {
+        const int *q = ijk + 3 * w;
+        for (int m = 0; m < 6; m++) {
+            if (q[0] == q[1] && !TWIN[m])
+                continue;
+            const int P = TERM[m][0], B = TERM[m][1], C = TERM[m][2];
+            const int code = P | B << 2 | C << 4;
+            e[P == 2].push_back({q[P], {w, code, q[C] * o + q[B]}});
+            e[2].push_back({q[C] * o + q[B], {w, code, q[P]}});
         }
-        GemmGroup sub;
-        sub.n = 0;
-        for (int q = p; q < gg.n; q++)
-            if (!done[q] && kn_modes(gg.g[q]) == am) {
-                sub.g[sub.n++] = gg.g[q];
-                done[q] = true;
-            }
-        hipError_t e = launch_kn_group(sub, am, batch, s);
-        if (e != hipSuccess)
-            return e;
     }
-    return hipSuccess;
+    BackRange *out[3] = {&b.rows, &b.rows2, &b.second};
+    for (int k = 0; k < 3; k++) {
+        std::stable_sort(e[k].begin(), e[k].end(), [](const Entry &x, const Entry &y) { return x.id < y.id; });
+        out[k]->tg0 = (int)t.tg.size();
+        out[k]->seg0 = (int)t.segs.size();
+        for (const Entry &x : e[k]) {
+            if ((int)t.tg.size() == out[k]->tg0 || t.tg.back().id != x.id)
+                t.tg.push_back({x.id, (int)t.segs.size(), 0});
+            t.tg.back().nseg++;
+            t.segs.push_back(x.s);
+        }
+        out[k]->ntg = (int)t.tg.size() - out[k]->tg0;
+        out[k]->nseg = (int)t.segs.size() - out[k]->seg0;
+        if (k < 2)  // the longest first
+            std::stable_sort(t.tg.begin() + out[k]->tg0, t.tg.end(),
+                             [](const BackTarget &x, const BackTarget &y) { return x.nseg > y.nseg; });
+    }
+}
+
+static int round8(int n) { return (n + 7) / 8 * 8; }
+static int back_cols(int o, int v) { return ((round8(v) + round8(o) + 15) / 16 + 7) / 8; }  // column tiles
+// Blocks of a target of the first kind: row tiles in eights (one per XCD) times column tiles
+static int back_blocks(int o, int v) {
+    const int64_t nbm = ((int64_t)v * (round8(v) / 8) + 1) / 2, ntm = (nbm + 7) / 8;
+    return (int)((ntm + 7) / 8 * 8 * back_cols(o, v));
+}
+// Tiles of a term of the second kind
+static int back_tiles(int o, int v) { return ((v + 15) / 16 + 7) / 8 * back_cols(o, v); }
+
+// K ranges of a term of the second kind: 3072 work-groups (six rounds of the chip) from n triples, at most v
+// One round of the chip (o=10, v=75, 48 tiles: 12.7 ms spread, 13.0 not; o=20, v=200, 640 tiles: no difference)
+bool back_spread(int o, int v) { return back_blocks(o, v) < 512; }
+
+int back_splits(int n, int o, int v) { return std::max(1, std::min(v, 3072 / (6 * n * back_tiles(o, v)))); }
+
+hipError_t launch_back(const BackArgs &a0, const BackTarget *tg, const BackBatch &b, double *dT, double *dRn, hipStream_t s) {
+    BackArgs a = a0;
+    const int nc = a.v8 + a.o8, tiles2 = back_tiles(a.o, a.v);
+    a.per = back_blocks(a.o, a.v);
+    a.tg = tg + b.rows.tg0;
+    a.blocks1 = b.rows.ntg * a.per;
+    a.seg2 = b.second.seg0;
+    a.nseg2 = b.second.nseg;
+    const int blocks2 = (a.nseg2 * a.splits + 7) / 8 * 8 * tiles2;
+    hipLaunchKernelGGL(back_kernel, dim3((unsigned)(a.blocks1 + blocks2)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(back_reduce_kernel, dim3((unsigned)(((int64_t)a.v * nc + 255) / 256), (unsigned)b.second.ntg), dim3(256),
+                       0, s, a, tg + b.second.tg0, dT, dRn);
+    a.rows2 = 1;
+    a.tg = tg + b.rows2.tg0;
+    a.blocks1 = b.rows2.ntg * a.per;
+    hipLaunchKernelGGL(back_kernel, dim3((unsigned)a.blocks1), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------- V backward
@@ -1533,12 +1380,18 @@ template <typename F> __device__ inline void nsum8(int n, F f, double &s, double
 
 // dU (w = 0, 1, 2) and H[a][c] = sum_b G_V[a][b][c] U0[a][b] (w = 3, into H), one thread per output
 // element; the threads of a wave take consecutive y, so every G_V read but dU0's is coalesced
-__global__ __launch_bounds__(256) void vback_du_kernel(const double *GV, const double *t1, const double *U, int i,
-                                                        int j, int k, int v, int vR, double *dU, double *H) {
+__global__ __launch_bounds__(256) void vback_du_kernel(const double *GV, int64_t gstride, const double *t1,
+                                                        const double *U, const int *ijk, int v, int vR, double *dU,
+                                                        double *H) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t vv = (int64_t)v * v;
     if (idx >= 4 * vv)
         return;
+    const int i = ijk[3 * blockIdx.y], j = ijk[3 * blockIdx.y + 1], k = ijk[3 * blockIdx.y + 2];
+    GV += blockIdx.y * gstride;
+    U += (int64_t)blockIdx.y * 3 * v * vR;
+    dU += blockIdx.y * 3 * vv;
+    H += blockIdx.y * vv;
     const int w = (int)(idx / vv);
     const int64_t xy = idx - w * vv;
     const int x = (int)(xy / v), y = (int)(xy - (int64_t)x * v);
@@ -1563,9 +1416,13 @@ __global__ __launch_bounds__(256) void vback_du_kernel(const double *GV, const d
     dU[idx] = s + c;
 }
 
-__global__ __launch_bounds__(256) void vback_dt_kernel(const double *GV, const double *U, const double *H, int v, int vR,
-                                                        double *dt) {
+__global__ __launch_bounds__(256) void vback_dt_kernel(const double *GV, int64_t gstride, const double *U,
+                                                        const double *H, int v, int vR, double *dt) {
     __shared__ double rs[256], rc[256];
+    GV += blockIdx.y * gstride;
+    U += (int64_t)blockIdx.y * 3 * v * vR;
+    H += (int64_t)blockIdx.y * v * v;
+    dt += (int64_t)blockIdx.y * 3 * v;
     const int w = blockIdx.x / v, x = blockIdx.x - w * v;
     const int64_t R2 = (int64_t)vR * vR, vr = (int64_t)v * vR;
     const int64_t n = w == 0 ? v : (int64_t)v * v;
@@ -1614,39 +1471,56 @@ __global__ __launch_bounds__(256) void vback_dt_kernel(const double *GV, const d
         dt[blockIdx.x] = rs[0] + rc[0];
 }
 
-// dS[p][q][x][y] = d/d(px|qy): the six updates dS[pq_u] += 1/2 dU[u / 2] (transposed for odd u), in u
-// order, and the three dt1 row updates (k from dt[0..v), j from dt[v..2v), i from dt[2v..3v)), in order.
-// Targets may coincide (two equal occupied indices); each thread owns one (x, y) of every target, so the
-// updates of one element stay in that order and no two threads touch the same element.
+// dS[p][q][x][y] = d/d(px|qy): of each triple in order the six updates dS[pq_u] += 1/2 dU[u / 2] (transposed for odd u),
+// in u order, for the pair p o + q of target blockIdx.y; past the targets the row dt1[blockIdx.y - ntg] with a triple's k
+// from dt[0..v), j from dt[v..2v), i from dt[2v..3v). One thread per output element, read and written once.
 __global__ __launch_bounds__(256) void vback_acc_kernel(double *dS, double *dt1, const double *dU, const double *dt,
-                                                         int i, int j, int k, int o, int v, int vR) {
+                                                         const int *ijk, int n, const BackTarget *tg, int ntg, int o, int v,
+                                                         int vR) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t vv = (int64_t)v * v;
-    if (idx < vv) {
-        const int x = (int)(idx / v), y = (int)(idx - (int64_t)x * v);
-        const int pq[6][2] = {{i, j}, {j, i}, {i, k}, {k, i}, {j, k}, {k, j}};
+    double s = 0.0;
+    if ((int)blockIdx.y >= ntg) {
+        const int p = (int)blockIdx.y - ntg;
+        if (idx >= v)
+            return;
+        double *out = dt1 + (int64_t)p * vR + idx;
+        s = *out;
+        for (int b = 0; b < n; b++)
 #pragma unroll
-        for (int u = 0; u < 6; u++) {
-            const double *src = dU + (u / 2) * vv;
-            dS[((int64_t)pq[u][0] * o + pq[u][1]) * vv + idx] += 0.5 * ((u & 1) ? src[(int64_t)y * v + x] : src[idx]);
-        }
+            for (int u = 0; u < 3; u++)
+                if (ijk[3 * b + 2 - u] == p)
+                    s += dt[((int64_t)3 * b + u) * v + idx];
+        *out = s;
+        return;
     }
-    if (idx < v) {
-        const int rows[3] = {k, j, i};
+    if (idx >= vv)
+        return;
+    const int pq = tg[blockIdx.y].id, p = pq / o, q = pq - p * o;
+    const int64_t x = idx / v, y = idx - x * v;
+    double *out = dS + pq * vv + idx;
+    s = *out;
+    for (int b = 0; b < n; b++) {
+        const int i = ijk[3 * b], j = ijk[3 * b + 1], k = ijk[3 * b + 2];
+        const int P[6] = {i, j, i, k, j, k}, Q[6] = {j, i, k, i, k, j};
 #pragma unroll
-        for (int u = 0; u < 3; u++)
-            dt1[(int64_t)rows[u] * vR + idx] += dt[(int64_t)u * v + idx];
+        for (int u = 0; u < 6; u++)
+            if (P[u] == p && Q[u] == q)
+                s += 0.5 * dU[(int64_t)(3 * b + u / 2) * vv + (u & 1 ? y * v + x : idx)];
     }
+    *out = s;
 }
 
-hipError_t launch_vback(const double *GV, const double *U, const double *t1, int i, int j, int k, int o, int v, int vR,
-                        double *dU, double *dt, double *H, double *dS, double *dt1, hipStream_t s) {
+hipError_t launch_vback(const double *GV, int64_t gstride, const double *U, const double *t1, const int *ijk, int n,
+                        const BackTarget *tg, int ntg, int o, int v, int vR, double *dU, double *dt, double *H, double *dS,
+                        double *dt1, hipStream_t s) {
     const int64_t vv = (int64_t)v * v;
-    hipLaunchKernelGGL(vback_du_kernel, dim3((unsigned)((4 * vv + 255) / 256)), dim3(256), 0, s, GV, t1, U, i, j, k, v,
-                       vR, dU, H);
-    hipLaunchKernelGGL(vback_dt_kernel, dim3((unsigned)(3 * v)), dim3(256), 0, s, GV, U, H, v, vR, dt);
-    hipLaunchKernelGGL(vback_acc_kernel, dim3((unsigned)((std::max<int64_t>(vv, v) + 255) / 256)), dim3(256), 0, s, dS,
-                       dt1, dU, dt, i, j, k, o, v, vR);
+    hipLaunchKernelGGL(vback_du_kernel, dim3((unsigned)((4 * vv + 255) / 256), (unsigned)n), dim3(256), 0, s, GV, gstride,
+                       t1, U, ijk, v, vR, dU, H);
+    hipLaunchKernelGGL(vback_dt_kernel, dim3((unsigned)(3 * v), (unsigned)n), dim3(256), 0, s, GV, gstride, U, H, v, vR,
+                       dt);
+    hipLaunchKernelGGL(vback_acc_kernel, dim3((unsigned)((std::max<int64_t>(vv, v) + 255) / 256), (unsigned)(ntg + o)),
+                       dim3(256), 0, s, dS, dt1, dU, dt, ijk, n, tg, ntg, o, v, vR);
     return hipGetLastError();
 }
 

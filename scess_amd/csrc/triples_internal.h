@@ -149,22 +149,17 @@ hipError_t launch_reduce_energy(const double *F, const int *ijk_all, int nall, d
 hipError_t launch_fill_zero(double *p, int64_t n, hipStream_t s);
 
 // ----------------------------------------------------------------- adjoint
-// FP64 operand of the generic GEMM: element (r, k1, k2) of batch b at
+// FP64 operand of the GEMM (s2 == 1): element (r, k1, k2) of batch b at
 // base + b*sb + r*sr + k1*s1 + k2*s2.
 struct GemmOp {
     const double *base;
     int64_t sr, s1, s2, sb;
-    // Elements readable along the unit-stride dimension from index 0 (the padded row length of the
-    // array; 0 = unknown), and whether entries with k2 in [K2, K2 rounded up to 16) read as zero. With
-    // these known, the back-contraction GEMMs use direct-to-LDS loads (gemm_kn_kernel).
-    int64_t cext;
-    bool kzero;
 };
 struct GemmSeg {
     GemmOp A, B;  // A rows m, B rows n
     int K1, K2;   // K = K1 x K2, K2 the inner (chunked) extent
 };
-// C[b][m][n] += alpha sum_seg sum_k A(m,k) B(n,k); splits > 1 (batch 1) sums K-range partials in order.
+// C[b][m][n] += alpha sum_seg sum_k A(m,k) B(n,k); splits > 1 sums K-range partials in order (batch 1 but for gemm_nt_kernel).
 struct GemmArgs {
     GemmSeg seg[2];
     int nseg;
@@ -173,33 +168,63 @@ struct GemmArgs {
     int64_t sCm, sCn, sCb;
     double alpha;
     int splits;
-    double *scratch;  // splits * M * N (times the batch for K-contiguous FP64 operands)
+    double *scratch;  // splits * M * N * batch
     int ow;           // C[b][m][n] is overwritten, not added to
-    // products in P64 (default), P32 or PB3 on the K-contiguous path; FP64 inputs are rounded (split
+    // products in P64 (default), P32 or PB3; FP64 inputs are rounded (split
     // into hi + lo bf16 for PB3) in registers, each 16-deep K chunk is summed on the MFMA in FP32
-    // and added to FP64 accumulators. Other layouts always use FP64.
+    // and added to FP64 accumulators.
     int prec;
-    // Set by launch_gemm_group only (gemm_kn_kernel): > 0 when the batch is folded into the rows, M
-    // then being mfold x batch and row m' of A and C row m' % mfold of batch entry m' / mfold.
-    int mfold;
 };
 hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s);
-// Up to kMaxGemmGroup GEMMs of one shape (M, N, batch, splits) writing disjoint outputs, launched
-// together (direct-to-LDS kernel: grid z = split x problem; grouped by operand layout) or, where that
-// kernel does not apply, one after another in the given order. Each problem's splits > 1 needs its own
-// scratch. The sums are those of launch_gemm on each problem.
-constexpr int kMaxGemmGroup = 6;
-struct GemmGroup {
-    GemmArgs g[kMaxGemmGroup];
-    int n;
+// G_W, G_V ([vR]^3 row-major, FP64, wstride apart) of nbatch occupied triples; W in a.W1/W2, V pieces in a.U, weights
+// dE 2 / deg. G_W of triples with i == j is doubled (see back_terms).
+hipError_t launch_adjoint_g(int prec, const EpiArgs &a, double dE, double *GW, double *GV, int nbatch, hipStream_t s);
+// Back-contractions of a batch of triples: each term (one G, read with K at one position) is a segment, the segments of
+// one output a target.
+struct BackSeg {
+    int slot, code;  // triple of the batch; positions P | B << 2 | C << 4
+    int x;           // first kind: c o + b (T, Rn); second kind: a (X, TM)
 };
-hipError_t launch_gemm_group(const GemmGroup &gg, int batch, hipStream_t s);
-// G_W, G_V ([vR]^3 row-major, FP64) of the single occupied triple a.ijk; W in a.W1/W2, V pieces in a.U
-hipError_t launch_adjoint_g(int prec, const EpiArgs &a, double wgt, double *GW, double *GV, hipStream_t s);
-// V backward of one occupied triple into dS [o][o][v][v] and dt1 [o][vR]; dU (3 v^2), dt (3 v) and H (v^2)
-// are scratch
-hipError_t launch_vback(const double *GV, const double *U, const double *t1, int i, int j, int k, int o, int v, int vR,
-                        double *dU, double *dt, double *H, double *dS, double *dt1, hipStream_t s);
+struct BackTarget {
+    int id, seg0, nseg;  // first kind: p; second kind: c o + b
+};
+struct BackTables {
+    std::vector<BackSeg> segs;
+    std::vector<BackTarget> tg;
+};
+struct BackRange {
+    int tg0, ntg, seg0, nseg;
+};
+struct BackBatch {
+    BackRange rows, rows2, second;  // first kind with p at position 0 or 1, with p at position 2; second kind
+};
+struct BackArgs {
+    const double *G;  // [vR]^3 per triple, zero past v
+    int64_t gstride;
+    int o, v, o8, v8, vR;  // v8, o8: rounded up to 8
+    int64_t vK, oK;
+    const double *T, *Rn, *X, *TM;  // packed FP64 operands
+    double *dX, *dTM, *scr;
+    const BackSeg *segs;
+    int splits;
+    // set by launch_back
+    const BackTarget *tg;
+    int per, blocks1, seg2, nseg2, rows2;
+};
+// Appends the terms of n triples (3 indices each, i == j where two are equal) to the tables
+void back_terms(const int *ijk, int n, int o, BackTables &t, BackBatch &b);
+// K ranges of a term of the second kind; scr holds 6 n splits v (v8 + o8) doubles
+int back_splits(int n, int o, int v);
+// dX, dTM (in a), dT and dRn += the terms of one batch; tg: the device copy of the tables' targets
+hipError_t launch_back(const BackArgs &a, const BackTarget *tg, const BackBatch &b, double *dT, double *dRn, hipStream_t s);
+// True where a target has too few tiles to fill the chip: batches of triples from all over the list then have many
+// targets of few terms, batches of neighbours (the same i, often j) one with most of the terms
+bool back_spread(int o, int v);
+// V backward of n triples, in order, into dS [o][o][v][v] and dt1 [o][vR]; tg: the batch's targets of the second kind (all
+// pairs of its triples); dU (3 v^2 n), dt (3 v n) and H (v^2 n) are scratch
+hipError_t launch_vback(const double *GV, int64_t gstride, const double *U, const double *t1, const int *ijk, int n,
+                        const BackTarget *tg, int ntg, int o, int v, int vR, double *dU, double *dt, double *H, double *dS,
+                        double *dt1, hipStream_t s);
 // ColMajor gradients: mode 0 ovvv <- dX, 1 ovoo <- -dRn, 2 ovov <- dS, 3 t2 <- dT + dTM, 4 t1 <- dt1
 hipError_t launch_unpack(int mode, const double *A, const double *B, double *out, int o, int v, int64_t vK, int64_t oK,
                          int64_t vR, int64_t n, hipStream_t s);
