@@ -1279,13 +1279,14 @@ __global__ __launch_bounds__(F == 4 ? 512 : 256, (F == 1 || (F == 2 && S == 5)) 
 // step, F = 1 / 2 / 4): S = 5 5.49 / 5.25 / 5.48, S = 6 6.42 / 12.4 / 6.97, S = 7 8.62 / 14.2 / -.
 int i8_fixed_per_group(int slices) { return slices == 5 ? 2 : 1; }
 
-// MFMA blocks per wave edge, from timing sweeps at v = 300: 2 (64x64 work-group tiles) for FP64
-// and FP32; 4 for BF16x3, whose three MFMAs per product need the larger register tile to keep
-// LDS reads per MFMA low.
+// MFMA blocks per wave edge, from timing sweeps: 2 (64x64 work-group tiles) for FP64 and FP32; 4 for BF16x3 where 64-wide
+// tiles need a fourth per edge: its three MFMAs per product leave it bound by the traffic of the operands, which halves
+// with the larger tile, but two 128-wide tiles pad v <= 192 too far (E(T), 2 / 4 blocks, ms: o=12, v=160 22.7 / 26.7, v=192
+// 37.3 / 38.6; 1/8 of o=16, v=200 16.9 / 13.0, v=224 21.5 / 15.6; 1/16 of o=16, v=239 12.9 / 10.0).
 int wbuild_tile(int prec, int v) {
     if (prec == PI8 || prec == P64)
         return 2;
-    if (prec == PB3 && v >= 240)
+    if (prec == PB3 && v > 192)
         return 4;
     if (v > 32)
         return 2;
