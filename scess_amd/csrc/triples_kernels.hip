@@ -233,11 +233,6 @@ hipError_t launch_pack(int mode, int prec, const double *src, void *dst, int o, 
 
 // ----------------------------------------------------------------- W build
 template <int PREC> struct Tr;
-template <> struct Tr<P64> {
-    using Acc = double;
-    using AccV = d4;
-    static constexpr int RB = 128;  // bytes of one K chunk of a row (16 doubles)
-};
 template <> struct Tr<P32> {
     using Acc = float;
     using AccV = f4;
@@ -403,28 +398,7 @@ __global__ __launch_bounds__(256) void wbuild_kernel(WBuildArgs a) {
     auto compute = [&](int buf) {
         const char *As = lds[buf];
         const char *Bs = As + BM * PITCH;
-        if constexpr (PREC == P64) {
-            double af[BLK][4], bf[BLK][4];
-#pragma unroll
-            for (int b = 0; b < BLK; b++) {
-                const double *pa = (const double *)(As + (wm * BLK * 16 + b * 16 + lr) * PITCH + lq * 32);
-                const double *pb = (const double *)(Bs + (wn * BLK * 16 + b * 16 + lr) * PITCH + lq * 32);
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    af[b][t] = pa[t];
-                    bf[b][t] = pb[t];
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int x = 0; x < BLK; x++)
-                    if (vr[x])
-#pragma unroll
-                        for (int y = 0; y < BLK; y++)
-                            if (vc[y])
-                                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[x][t], bf[y][t], acc[x][y], 0, 0, 0);
-        } else if constexpr (PREC == P32) {
+        if constexpr (PREC == P32) {
             f4 af[BLK], bf[BLK];
 #pragma unroll
             for (int b = 0; b < BLK; b++) {
@@ -497,7 +471,7 @@ __global__ __launch_bounds__(256) void wbuild_kernel(WBuildArgs a) {
             const int col = c0 + wn * BLK * 16 + y * 16 + lr;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = r0 + wm * BLK * 16 + x * 16 + (PREC == P64 ? lq + 4 * r : 4 * lq + r);
+                const int row = r0 + wm * BLK * 16 + x * 16 + 4 * lq + r;
                 if (row < v && col < v)
                     W[fbase + ((int64_t)(row >> 3) * nbR + (col >> 3)) * 512 + (row & 7) * 8 + (col & 7)] = acc[x][y][r];
             }
@@ -622,26 +596,7 @@ __global__ __launch_bounds__(256) void wbuild_dma_kernel(WBuildArgs a) {
     auto compute = [&](int st) {
         const char *As = lds[st];
         const char *Bs = As + OPB;
-        if constexpr (PREC == P64) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {  // two k-pairs per 16-byte vector: half the fragment registers
-                d2 af[BLK], bf[BLK];
-#pragma unroll
-                for (int b = 0; b < BLK; b++) {
-                    af[b] = *(const d2 *)frag(As, wm * BLK * 16 + b * 16 + lr, 2 * lq + h);
-                    bf[b] = *(const d2 *)frag(Bs, wn * BLK * 16 + b * 16 + lr, 2 * lq + h);
-                }
-#pragma unroll
-                for (int t = 0; t < 2; t++)
-#pragma unroll
-                    for (int x = 0; x < BLK; x++)
-                        if (vr[x])
-#pragma unroll
-                            for (int y = 0; y < BLK; y++)
-                                if (vc[y])
-                                    acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[x][t], bf[y][t], acc[x][y], 0, 0, 0);
-            }
-        } else if constexpr (PREC == P32) {
+        if constexpr (PREC == P32) {
             f4 af[BLK], bf[BLK];
 #pragma unroll
             for (int b = 0; b < BLK; b++) {
@@ -709,7 +664,7 @@ __global__ __launch_bounds__(256) void wbuild_dma_kernel(WBuildArgs a) {
             const int col = c0 + wn * BLK * 16 + y * 16 + lr;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = r0 + wm * BLK * 16 + x * 16 + (PREC == P64 ? lq + 4 * r : 4 * lq + r);
+                const int row = r0 + wm * BLK * 16 + x * 16 + 4 * lq + r;
                 if (row < v && col < v)
                     W[fbase + ((int64_t)(row >> 3) * nbR + (col >> 3)) * 512 + (row & 7) * 8 + (col & 7)] = acc[x][y][r];
             }
