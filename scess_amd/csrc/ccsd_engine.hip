@@ -59,7 +59,7 @@ struct PermWalk {
 // outputs: walking several consecutive outputs per thread saves index divisions but spreads every
 // store instruction over 32-byte strides (FP64 update at o=50, v=500: 1.33 s of permutes against 0.70 s).
 __global__ __launch_bounds__(256) void permute_kernel(PermArgs a) {
-    const int64_t lin = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t lin = element_id();
     if (lin >= a.n)
         return;
     PermWalk w;
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void permute_split_kernel(PermArgs a, int64_t 
     // one element per thread: the lanes of a wave read consecutive k of a row (walking eight k per
     // thread and storing 16-byte vectors spread each load over 64-byte strides: 0.74 s against 0.63 s
     // of split permutes per BF16x3 update at o=50, v=500)
-    const int64_t lin = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t lin = element_id();
     if (lin >= nrows * Kp)
         return;
     const int64_t row = lin / Kp, k = lin - row * Kp;
@@ -426,7 +426,7 @@ void Engine::permute(const std::string &li, const double *in, const std::vector<
         return;
     a.row = row == pitch ? 0 : row;
     a.pitch = pitch;
-    hipLaunchKernelGGL(permute_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(permute_kernel, element_grid(a.n), dim3(256), 0, stream, a);
     check(hipGetLastError(), "permute");
 }
 
@@ -438,7 +438,7 @@ DTensor Engine::permute_split(const std::string &li, const double *in, const std
     const int64_t Kp = (K + 31) / 32 * 32, nrows = a.n / K;
     DTensor out = alloc({nrows, Kp / 2});  // Kp bf16 pairs per row = Kp / 2 eight-byte slots
     if (nrows > 0) {
-        hipLaunchKernelGGL(permute_split_kernel, dim3((unsigned)((nrows * Kp + 255) / 256)), dim3(256), 0, stream, a,
+        hipLaunchKernelGGL(permute_split_kernel, element_grid(nrows * Kp), dim3(256), 0, stream, a,
                            K, Kp, (uint16_t *)out.p, nrows);
         check(hipGetLastError(), "permute_split");
     }

@@ -1529,7 +1529,7 @@ hipError_t launch_vback(const double *GV, int64_t gstride, const double *U, cons
 __global__ __launch_bounds__(256) void unpack_kernel(int mode, const double *A, const double *B, double *out, int o_,
                                                      int v_, int64_t vK, int64_t oK, int64_t vR) {
     const int64_t o = o_, v = v_;
-    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t gid = element_id();
     int64_t n = 0;
     switch (mode) {
     case 0: n = o * v * v * v; break;  // ovvv(p,x,y,f) = dX[p][x][y][f]
@@ -1568,7 +1568,7 @@ __global__ __launch_bounds__(256) void unpack_kernel(int mode, const double *A, 
 
 hipError_t launch_unpack(int mode, const double *A, const double *B, double *out, int o, int v, int64_t vK, int64_t oK,
                          int64_t vR, int64_t n, hipStream_t s) {
-    hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, mode, A, B, out, o, v, vK, oK,
+    hipLaunchKernelGGL(unpack_kernel, element_grid(n), dim3(256), 0, s, mode, A, B, out, o, v, vK, oK,
                        vR);
     return hipGetLastError();
 }

@@ -37,6 +37,16 @@ template <int N> __device__ inline void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// n elements, one per thread of work-groups of 256, as a two-dimensional grid and their number in it: a dimension of a
+// launch holds fewer than 2^32 threads, and (px|yf) at o=50, v=500 has 6.25e9 elements
+inline dim3 element_grid(int64_t n) {
+    const int64_t blocks = (n + 255) / 256, x = blocks < (1 << 23) ? blocks : 1 << 23;
+    return dim3((unsigned)x, (unsigned)((blocks + x - 1) / x));
+}
+__device__ inline int64_t element_id() {
+    return ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+}
+
 // s_waitcnt vmcnt(0) lgkmcnt(0)
 __device__ inline void wait_vm_lgkm0() { __builtin_amdgcn_s_waitcnt(7 << 4); }
 typedef __attribute__((address_space(3))) char lds_char;

@@ -118,7 +118,7 @@ __device__ inline double pack_value(int mode, const double *__restrict__ src, in
 template <int PREC>
 __global__ void pack_kernel(int mode, const double *__restrict__ src, void *__restrict__ dst, int o_, int v_,
                             int64_t kpad, int64_t nrows) {
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t gid = element_id();
     if (gid >= nrows * kpad)
         return;
     const int64_t row = gid / kpad, k = gid - row * kpad;
@@ -142,7 +142,7 @@ __global__ void pack_kernel(int mode, const double *__restrict__ src, void *__re
 // d = ((N + 128) mod 256) - 128 in [-128, 127] and N = (N - d) / 256, all exact in int64.
 __global__ void pack_i8_kernel(int mode, const double *__restrict__ src, int8_t *__restrict__ dst, int o_, int v_,
                                int64_t kpad, int gran, double scale, int S, int64_t nrows) {
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t gid = element_id();
     if (gid >= nrows * kpad)
         return;
     const int64_t row = gid / kpad, k = gid - row * kpad;
@@ -176,7 +176,7 @@ hipError_t launch_pack_i8(int mode, const double *src, void *dst, int o, int v, 
     const int64_t blocks = (nrows * kpad + 255) / 256;
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pack_i8_kernel, dim3((unsigned)blocks), dim3(256), 0, s, mode, src, (int8_t *)dst, o, v,
+    hipLaunchKernelGGL(pack_i8_kernel, element_grid(nrows * kpad), dim3(256), 0, s, mode, src, (int8_t *)dst, o, v,
                        kpad, gran, scale, slices, nrows);
     return hipGetLastError();
 }
@@ -223,11 +223,11 @@ hipError_t launch_pack(int mode, int prec, const double *src, void *dst, int o, 
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidValue;
     if (prec == P64)
-        hipLaunchKernelGGL(pack_kernel<P64>, dim3((unsigned)blocks), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
+        hipLaunchKernelGGL(pack_kernel<P64>, element_grid(n), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
     else if (prec == P32)
-        hipLaunchKernelGGL(pack_kernel<P32>, dim3((unsigned)blocks), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
+        hipLaunchKernelGGL(pack_kernel<P32>, element_grid(n), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
     else
-        hipLaunchKernelGGL(pack_kernel<PB3>, dim3((unsigned)blocks), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
+        hipLaunchKernelGGL(pack_kernel<PB3>, element_grid(n), dim3(256), 0, s, mode, src, dst, o, v, kpad, nrows);
     return hipGetLastError();
 }
 
