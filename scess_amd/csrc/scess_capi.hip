@@ -538,18 +538,21 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     // the XCD-ordered work-groups give each of the 8 XCDs whole triples (measured: the FP64 W-build at
     // o=50, v=500 is 27% faster than with one triple per launch, at the same HBM bytes per triple);
     // fewer when the W sets (2 arrays x 2 sets x nbatch x vR^3) exceed a quarter of the free device memory.
-    // FP64: 16 against 8 (o=20, v=200 0.549 s against 0.560 s: fewer half-empty ends of launches); for small v
-    // as many as make 8 rounds of the W-build's items over its 512 work-groups, within 1 GiB of W
+    // FP64: 16 against 8 (o=20, v=200 0.549 s against 0.560 s: fewer half-empty ends of launches). For small v a launch
+    // of 16 leaves the chip nearly empty, so it takes as many triples as make 8 rounds of the FP64 W-build's items over
+    // its 512 work-groups, within 1 GiB of W (other modes where that is twice as many or more: o=24, v=19, 16 or 8
+    // against 819 triples, FP32 6.95 / 1.25 ms, BF16x3 7.32 / 1.16, int8 15.8 / 1.94; o=10, v=100, 40 and 23: 6.44 / 5.94,
+    // 3.80 / 3.50, 6.28 / 5.98; int8 at v=180 would lose, 16.7 / 18.0 with 16)
     int64_t nbatch = c->nbatch_req;
     if (nbatch <= 0) {
         const double per = 4.0 * (double)wstride * (double)accb;
         size_t fr = 0, tot = 0;
         const double budget = hipMemGetInfo(&fr, &tot) == hipSuccess ? 0.25 * (double)fr : 4.0e9;
         nbatch = prec == PI8 ? 8 : 16;
-        if (prec == P64) {
-            const int64_t nt = (v + 63) / 64, items = (v + 3) / 4 * nt * nt;
-            nbatch = std::max<int64_t>(16, std::min<int64_t>(8 * 512 / items, (int64_t)(1073741824.0 / per)));
-        }
+        const int64_t nt = (v + 63) / 64, items = (v + 3) / 4 * nt * nt;
+        const int64_t small = std::min<int64_t>(8 * 512 / items, (int64_t)(1073741824.0 / per));
+        if (small >= (prec == P64 ? 1 : 2) * nbatch)
+            nbatch = small;
         while (nbatch > 1 && nbatch * per > budget)
             nbatch /= 2;
     }
