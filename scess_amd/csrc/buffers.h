@@ -19,6 +19,18 @@ public:
     hipError_t get(void **p, size_t bytes, hipStream_t s);
     void put(void *p);  // null is allowed
     void flush();
+    // p to at least `need` elements, without its contents; after an error p is null and cap 0
+    template <class T> hipError_t grow(T *&p, size_t &cap, size_t need, hipStream_t s) {
+        if (need <= cap)
+            return hipSuccess;
+        put((void *)p);
+        p = nullptr;
+        cap = 0;
+        const hipError_t e = get((void **)&p, sizeof(T) * need, s);
+        if (e == hipSuccess)
+            cap = need;
+        return e;
+    }
 
 private:
     struct Block {

@@ -572,17 +572,9 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     }
     // per-orbit partials: whole job if the caller wants them, else one batch
     const size_t pneed = (size_t)(partials_out ? std::max<int64_t>(nwork, 1) : 2 * nbatch) * (size_t)t.ngrp;
-    if (t.partials_cap < pneed) {
-        dfree(c, t.partials);
-        HIP_TRY(c, dmalloc(c, &t.partials, sizeof(double) * pneed));
-        t.partials_cap = pneed;
-    }
+    HIP_TRY(c, c->blocks.grow(t.partials, t.partials_cap, pneed, c->stream));
     const size_t uneed = 2 * (size_t)nbatch * 3 * (size_t)(v * vR);
-    if (t.u_cap < uneed) {
-        dfree(c, t.U);
-        HIP_TRY(c, dmalloc(c, &t.U, sizeof(double) * uneed));
-        t.u_cap = uneed;
-    }
+    HIP_TRY(c, c->blocks.grow(t.U, t.u_cap, uneed, c->stream));
     HIP_TRY(c, hipMemsetAsync(t.F, 0, sizeof(double) * nall, c->stream));
     HIP_TRY(c, hipMemsetAsync(t.queue, 0, sizeof(int) * kWQueues * ((nshare + nbatch - 1) / nbatch), c->stream));
     const size_t wset = (size_t)nbatch * (size_t)wstride * accb;  // bytes of one set of W1 (or W2)

@@ -1,0 +1,89 @@
+// Host-only check of the device block cache (scess_amd/csrc/buffers.cpp) over a simulated device: the HIP calls that
+// buffers.cpp makes are defined here. Memory is a count of bytes with a limit; a freed block returns to it when its stream
+// is next waited for. Run by tests/test_buffers_cpu.py with the name of one check.
+#include "buffers.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+namespace {
+
+struct Device {
+    size_t limit = (size_t)1 << 40, held = 0;  // bytes that can be handed out, and are (freed ones until the next wait)
+    std::map<void *, size_t> live, freed;      // by address: nothing is behind it
+    size_t next = 4096;
+} dev;
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMallocAsync(void **p, size_t bytes, hipStream_t) {
+    if (dev.held + bytes > dev.limit)
+        return hipErrorOutOfMemory;
+    *p = (void *)dev.next;
+    dev.next += (bytes + 4095) / 4096 * 4096;
+    dev.held += bytes;
+    dev.live[*p] = bytes;
+    return hipSuccess;
+}
+hipError_t hipFreeAsync(void *p, hipStream_t) {
+    const auto it = dev.live.find(p);
+    if (it == dev.live.end())
+        return hipErrorInvalidValue;
+    dev.freed.insert(*it);
+    dev.live.erase(it);
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+    for (auto &f : dev.freed)
+        dev.held -= f.second;
+    dev.freed.clear();
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipHostMalloc(void **, size_t, unsigned int) { return hipErrorOutOfMemory; }
+hipError_t hipHostFree(void *) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *, unsigned) { return hipErrorUnknown; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipErrorUnknown; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t) { return hipErrorUnknown; }
+}
+
+#define REQUIRE(x)                                             \
+    do {                                                       \
+        if (!(x)) {                                            \
+            std::printf("line %d: %s is false\n", __LINE__, #x); \
+            std::exit(1);                                      \
+        }                                                      \
+    } while (0)
+
+static hipStream_t stream() { return (hipStream_t)16; }
+
+// A growth that fails leaves a null pointer of no capacity, so the next call does not use it; a smaller need then works
+static void grow() {
+    dev.limit = 1 << 20;
+    scess::BlockCache c;
+    double *p = nullptr;
+    size_t cap = 0;
+    REQUIRE(c.grow(p, cap, 1000, stream()) == hipSuccess && p && cap == 1000);
+    double *const first = p;
+    REQUIRE(c.grow(p, cap, 500, stream()) == hipSuccess && p == first && cap == 1000);
+    REQUIRE(c.grow(p, cap, 1 << 20, stream()) == hipErrorOutOfMemory);
+    REQUIRE(!p && cap == 0);
+    REQUIRE(c.grow(p, cap, 1000, stream()) == hipSuccess && p && cap == 1000);
+    c.put(p);
+}
+
+int main(int argc, char **argv) {
+    const std::map<std::string, void (*)()> checks = {{"grow", grow}};
+    const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
+    if (it == checks.end())
+        return 2;
+    it->second();
+    std::printf("ok\n");
+    return 0;
+}
