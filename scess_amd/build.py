@@ -17,6 +17,7 @@ LIB = os.path.join(HERE, "libscess_gpu.so")
 CLI = os.path.join(HERE, "scess_cc")
 CPP_CHECK = os.path.join(ROOT, "tests", "cpp", "triples_function_check")
 BUF_CHECK = os.path.join(ROOT, "tests", "cpp", "buffers_check")
+GEMM_CHECK = os.path.join(ROOT, "tests", "cpp", "gemm_check")
 SO_CHECK = os.path.join(ROOT, "tests", "cpp", "spin_orbital_check")
 SOURCES = ["triples_kernels.hip", "triples_adjoint.hip", "ccsd_engine.hip", "scess_capi.hip", "buffers.cpp", "cc_api.cpp",
            "scf_host.cpp", "spin_orbital_cc.cpp", "regression.cpp"]
@@ -66,6 +67,10 @@ def build(verbose: bool = False) -> str:
     _run(["g++", "-O2", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "include"), "-o", CPP_CHECK + ".tmp",
           CPP_CHECK + ".cpp", "-L", HERE, "-lscess_gpu", "-Wl,-rpath,$ORIGIN/../../scess_amd"])
     os.replace(CPP_CHECK + ".tmp", CPP_CHECK)
+    # check of the GEMM launcher of the CCSD engine, run on the GPU by tests/test_gemm_gpu.py
+    _run([hipcc(), *HIP_FLAGS, "-I", CSRC, "-o", GEMM_CHECK + ".tmp", GEMM_CHECK + ".hip", "-L", HERE, "-lscess_gpu",
+          "-Wl,-rpath,$ORIGIN/../../scess_amd"])
+    os.replace(GEMM_CHECK + ".tmp", GEMM_CHECK)
     # host-only check of buffers.cpp over a simulated device (tests/test_buffers_cpu.py)
     _run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__", "-isystem",
           "/opt/rocm/include", "-I", CSRC, "-o", BUF_CHECK + ".tmp", BUF_CHECK + ".cpp", os.path.join(CSRC, "buffers.cpp"),

@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
                         double *cp = g.C + (int64_t)beta * g.sCb + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
                         *cp = g.ow ? g.alpha * acc[x][y][r] : *cp + g.alpha * acc[x][y][r];
                     } else {
-                        g.scratch[((int64_t)split * g.M + m) * g.N + n] = acc[x][y][r];
+                        g.scratch[(((int64_t)split * ny + beta) * g.M + m) * g.N + n] = acc[x][y][r];
                     }
                 }
             }

@@ -169,7 +169,7 @@ struct GemmSeg {
     GemmOp A, B;  // A rows m, B rows n
     int K1, K2;   // K = K1 x K2, K2 the inner (chunked) extent
 };
-// C[b][m][n] += alpha sum_seg sum_k A(m,k) B(n,k); splits > 1 sums K-range partials in order (batch 1 but for gemm_nt_kernel).
+// C[b][m][n] += alpha sum_seg sum_k A(m,k) B(n,k); splits > 1 sums K-range partials in order.
 struct GemmArgs {
     GemmSeg seg[2];
     int nseg;
