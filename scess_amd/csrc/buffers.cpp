@@ -34,10 +34,9 @@ hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
         return hipSuccess;
     }
     hipError_t e = hipMallocAsync(p, bytes, s);
-    if (e == hipErrorOutOfMemory && !free_.empty()) {  // the kept blocks may be what is missing
+    if (e == hipErrorOutOfMemory) {  // what is missing may be kept here, or freed but still with the runtime's pool
         (void)hipGetLastError();
-        flush();
-        (void)hipStreamSynchronize(s);
+        trim(s);
         e = hipMallocAsync(p, bytes, s);
     }
     if (e == hipSuccess)
@@ -70,6 +69,16 @@ void BlockCache::flush() {
         (void)hipFreeAsync(b.p, b.s);
     free_.clear();
     cached_ = 0;
+}
+
+void BlockCache::trim(hipStream_t s) {
+    flush();
+    (void)hipStreamSynchronize(s);
+    int device = 0;
+    hipMemPool_t pool;
+    if (hipGetDevice(&device) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess)
+        (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
 }
 
 // ------------------------------------------------------------------- copies

@@ -19,6 +19,7 @@ public:
     hipError_t get(void **p, size_t bytes, hipStream_t s);
     void put(void *p);  // null is allowed
     void flush();
+    void trim(hipStream_t s);  // waits for s (the stream of the blocks), and everything free goes back to the device
     // p to at least `need` elements, without its contents; after an error p is null and cap 0
     template <class T> hipError_t grow(T *&p, size_t &cap, size_t need, hipStream_t s) {
         if (need <= cap)

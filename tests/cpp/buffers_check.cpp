@@ -1,6 +1,6 @@
 // Host-only check of the device block cache (scess_amd/csrc/buffers.cpp) over a simulated device: the HIP calls that
-// buffers.cpp makes are defined here. Memory is a count of bytes with a limit; a freed block returns to it when its stream
-// is next waited for. Run by tests/test_buffers_cpu.py with the name of one check.
+// buffers.cpp makes are defined here. Memory is a count of bytes with a limit; a freed block goes to the pool when its
+// stream is next waited for, and back to the device when the pool is trimmed. Run by tests/test_buffers_cpu.py with the name of one check.
 #include "buffers.h"
 
 #include <cstdio>
@@ -12,8 +12,8 @@
 namespace {
 
 struct Device {
-    size_t limit = (size_t)1 << 40, held = 0;  // bytes that can be handed out, and are (freed ones until the next wait)
-    std::map<void *, size_t> live, freed;      // by address: nothing is behind it
+    size_t limit = (size_t)1 << 40, held = 0, pool = 0;  // bytes of the device, taken from it, and of these in the pool
+    std::map<void *, size_t> live, freed;                // by address: nothing is behind it
     size_t next = 4096;
 } dev;
 
@@ -39,8 +39,21 @@ hipError_t hipFreeAsync(void *p, hipStream_t) {
 }
 hipError_t hipStreamSynchronize(hipStream_t) {
     for (auto &f : dev.freed)
-        dev.held -= f.second;
+        dev.pool += f.second;
     dev.freed.clear();
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d) {
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *p, int) {
+    *p = nullptr;
+    return hipSuccess;
+}
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) {
+    dev.held -= dev.pool;
+    dev.pool = 0;
     return hipSuccess;
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
@@ -78,8 +91,26 @@ static void grow() {
     c.put(p);
 }
 
+// A block past the cache's bound goes back to the runtime, which may still hold it when a larger one is asked for
+static void freed_block_in_pool() {
+    const size_t gib = (size_t)1 << 30;
+    dev.limit = 20 * gib;
+    scess::BlockCache c;
+    void *p = nullptr, *q = nullptr;
+    REQUIRE(c.get(&p, 8 * gib, stream()) == hipSuccess);
+    c.put(p);  // nothing is kept of it
+    REQUIRE(c.get(&q, 16 * gib, stream()) == hipSuccess && q);
+    c.put(q);
+    // kept blocks make room, too
+    REQUIRE(c.get(&p, 5 * gib, stream()) == hipSuccess);
+    c.put(p);
+    REQUIRE(c.get(&q, 18 * gib, stream()) == hipSuccess && q);
+    c.put(q);
+    REQUIRE(c.get(&q, 21 * gib, stream()) == hipErrorOutOfMemory && !q);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, void (*)()> checks = {{"grow", grow}};
+    const std::map<std::string, void (*)()> checks = {{"grow", grow}, {"freed_block_in_pool", freed_block_in_pool}};
     const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end())
         return 2;
