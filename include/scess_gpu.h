@@ -97,6 +97,11 @@ int scess_create(scess_ctx **ctx, int device);
 void scess_destroy(scess_ctx *ctx);
 const char *scess_last_error(const scess_ctx *ctx);
 int scess_set_should_stop(scess_ctx *ctx, int (*should_stop)(void *), void *user);
+/* A context keeps up to 6 GiB of device memory that its calls have freed, for the next ones. It goes back to the
+ * device here, at scess_destroy, and when a context of the process runs out of memory on the same GPU; for
+ * programs that share the GPU with other users of its memory. Inputs stay resident (no counterpart in the
+ * reference). */
+int scess_trim(scess_ctx *ctx);
 /* Occupied-triple batch size (0 = automatic). */
 int scess_set_batch(scess_ctx *ctx, int64_t nbatch);
 

@@ -10,9 +10,36 @@
 namespace scess {
 
 // ------------------------------------------------------------------- blocks
-hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
-    bytes = (std::max<size_t>(bytes, 16) + 255) / 256 * 256;
-    *p = nullptr;
+namespace {
+
+// The caches of the process; left alone at its end
+std::mutex g_caches_mu;
+std::vector<BlockCache *> &g_caches = *new std::vector<BlockCache *>;
+
+// What was freed on the runtime's side goes back to the device
+void trim_pool(int device) {
+    hipMemPool_t pool;
+    if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess)
+        (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+}
+
+}  // namespace
+
+BlockCache::BlockCache() {
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    g_caches.push_back(this);
+}
+
+BlockCache::~BlockCache() {
+    flush();
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    g_caches.erase(std::find(g_caches.begin(), g_caches.end(), this));
+}
+
+// A block of this cache, or one of the runtime
+hipError_t BlockCache::take(void **p, size_t bytes, hipStream_t s) {
+    std::lock_guard<std::mutex> lk(m_);
     try {  // put() must not have to allocate
         used_.reserve(used_.size() + 1);
         free_.reserve(free_.size() + used_.size() + 1);
@@ -33,12 +60,9 @@ hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
         *p = used_.back().p;
         return hipSuccess;
     }
-    hipError_t e = hipMallocAsync(p, bytes, s);
-    if (e == hipErrorOutOfMemory) {  // what is missing may be kept here, or freed but still with the runtime's pool
-        (void)hipGetLastError();
-        trim(s);
-        e = hipMallocAsync(p, bytes, s);
-    }
+    if (device_ < 0)
+        (void)hipGetDevice(&device_);
+    const hipError_t e = hipMallocAsync(p, bytes, s);
     if (e == hipSuccess)
         used_.push_back({*p, bytes, s});
     else
@@ -46,9 +70,24 @@ hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
     return e;
 }
 
+hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
+    bytes = (std::max<size_t>(bytes, 16) + 255) / 256 * 256;
+    *p = nullptr;
+    hipError_t e = take(p, bytes, s);
+    if (e == hipErrorOutOfMemory) {
+        // what is missing may be kept here or by another context, or freed but still with the runtime's pool
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(s);
+        trim_all(device_);
+        e = take(p, bytes, s);
+    }
+    return e;
+}
+
 void BlockCache::put(void *p) {
     if (!p)
         return;
+    std::lock_guard<std::mutex> lk(m_);
     for (size_t i = used_.size(); i-- > 0;)
         if (used_[i].p == p) {
             const Block b = used_[i];
@@ -65,20 +104,36 @@ void BlockCache::put(void *p) {
 }
 
 void BlockCache::flush() {
+    std::lock_guard<std::mutex> lk(m_);
     for (const Block &b : free_)
         (void)hipFreeAsync(b.p, b.s);
     free_.clear();
     cached_ = 0;
 }
 
-void BlockCache::trim(hipStream_t s) {
-    flush();
-    (void)hipStreamSynchronize(s);
-    int device = 0;
-    hipMemPool_t pool;
-    if (hipGetDevice(&device) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess)
-        (void)hipMemPoolTrimTo(pool, 0);
-    (void)hipGetLastError();
+// The lock is held to the end: a context flushes its cache before its stream goes, and so waits for a thread that is here
+void BlockCache::trim(int device) {
+    std::lock_guard<std::mutex> lk(m_);
+    if (device_ < 0 || (device >= 0 && device != device_))
+        return;
+    hipStream_t last = nullptr;
+    for (const Block &b : free_) {
+        (void)hipFreeAsync(b.p, b.s);
+        if (last && b.s != last)
+            (void)hipStreamSynchronize(last);
+        last = b.s;
+    }
+    if (last)
+        (void)hipStreamSynchronize(last);
+    free_.clear();
+    cached_ = 0;
+    trim_pool(device_);
+}
+
+void BlockCache::trim_all(int device) {
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    for (BlockCache *c : g_caches)
+        c->trim(device);
 }
 
 // ------------------------------------------------------------------- copies

@@ -4,22 +4,28 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <mutex>
 #include <vector>
 
 namespace scess {
 
 // Device memory of one context: freed blocks are kept, up to kMaxCached bytes in all, and handed out again; the rest goes
-// back to the runtime, and everything at the end of the context. Stream ordered: a block is reused by work on the same
-// stream (or ordered after it). A call's dozens of allocations otherwise cost more than its kernels for small systems,
-// and the mapping of freshly allocated memory some milliseconds per GiB for large ones.
+// back to the runtime, and everything at the end of the context, on trim(), and where a context of the process finds the
+// device full. Stream ordered: a block is reused by work on the same stream (or ordered after it). A call's dozens of
+// allocations otherwise cost more than its kernels for small systems, and the mapping of freshly allocated memory some
+// milliseconds per GiB for large ones. Used by the context's thread; other threads only free kept blocks (trim_all).
 class BlockCache {
 public:
     static constexpr size_t kMaxCached = (size_t)6 << 30;
-    ~BlockCache() { flush(); }
+    BlockCache();
+    ~BlockCache();
+    BlockCache(const BlockCache &) = delete;
+    BlockCache &operator=(const BlockCache &) = delete;
     hipError_t get(void **p, size_t bytes, hipStream_t s);
     void put(void *p);  // null is allowed
-    void flush();
-    void trim(hipStream_t s);  // waits for s (the stream of the blocks), and everything free goes back to the device
+    void flush();       // the kept blocks go back to the runtime, in the order of their streams
+    // The kept blocks go back to the device, once the work that used them is done; not those of another device than `device`
+    void trim(int device = -1);
     // p to at least `need` elements, without its contents; after an error p is null and cap 0
     template <class T> hipError_t grow(T *&p, size_t &cap, size_t need, hipStream_t s) {
         if (need <= cap)
@@ -39,8 +45,12 @@ private:
         size_t bytes;
         hipStream_t s;
     };
+    hipError_t take(void **p, size_t bytes, hipStream_t s);
+    static void trim_all(int device);  // the kept blocks of every context on the device
+    std::mutex m_;
     std::vector<Block> free_, used_;
     size_t cached_ = 0;
+    int device_ = -1;  // of the blocks; -1 before the first
 };
 
 // Copies of any size between pageable host memory and the device, ordered on stream s as hipMemcpyAsync would be. Large

@@ -215,6 +215,14 @@ void scess_destroy(scess_ctx *c) {
     delete c;
 }
 
+int scess_trim(scess_ctx *c) {
+    if (!c)
+        return SCESS_ERR_ARG;
+    HIP_TRY(c, hipSetDevice(c->device));
+    c->blocks.trim();
+    return SCESS_OK;
+}
+
 const char *scess_last_error(const scess_ctx *c) { return c ? c->err.c_str() : "null context"; }
 
 int scess_set_should_stop(scess_ctx *c, int (*fn)(void *), void *user) {

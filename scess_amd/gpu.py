@@ -95,6 +95,8 @@ def load(path: str = LIB_PATH):
     lib.scess_last_error.restype = c.c_char_p
     lib.scess_set_should_stop.argtypes = [c.c_void_p, STOP_FN, c.c_void_p]
     lib.scess_set_should_stop.restype = c.c_int
+    lib.scess_trim.argtypes = [c.c_void_p]
+    lib.scess_trim.restype = c.c_int
     lib.scess_set_batch.argtypes = [c.c_void_p, c.c_int64]
     lib.scess_set_batch.restype = c.c_int
     lib.scess_t_set_inputs.argtypes = [c.c_void_p, c.POINTER(TIn), c.c_int]
@@ -182,6 +184,10 @@ class Context:
 
     def set_batch(self, n: int):
         self.check(self.lib.scess_set_batch(self.h, int(n)))
+
+    def trim(self):
+        """Gives back the device memory kept for later calls (inputs stay resident)."""
+        self.check(self.lib.scess_trim(self.h))
 
     def set_should_stop(self, fn):
         """fn() -> bool, polled between batches of occupied triples."""

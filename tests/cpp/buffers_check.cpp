@@ -74,7 +74,7 @@ hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream
         }                                                      \
     } while (0)
 
-static hipStream_t stream() { return (hipStream_t)16; }
+static hipStream_t stream(int n = 1) { return (hipStream_t)(size_t)(16 * n); }
 
 // A growth that fails leaves a null pointer of no capacity, so the next call does not use it; a smaller need then works
 static void grow() {
@@ -109,8 +109,31 @@ static void freed_block_in_pool() {
     REQUIRE(c.get(&q, 21 * gib, stream()) == hipErrorOutOfMemory && !q);
 }
 
+// Blocks that one context keeps make room for another, and trim() gives them back
+static void other_contexts() {
+    const size_t gib = (size_t)1 << 30;
+    dev.limit = 10 * gib;
+    scess::BlockCache a, b;
+    void *p = nullptr, *q = nullptr, *r = nullptr;
+    REQUIRE(a.get(&p, 5 * gib, stream(1)) == hipSuccess && a.get(&r, gib, stream(1)) == hipSuccess);
+    a.put(p);
+    REQUIRE(b.get(&q, 8 * gib, stream(2)) == hipSuccess && q);
+    REQUIRE(dev.live.count(r) == 1 && dev.live.size() == 2);  // what is in use stays
+    b.put(q);
+    REQUIRE(a.get(&p, gib, stream(1)) == hipSuccess);
+    a.put(p);
+    a.put(r);
+    REQUIRE(dev.held >= 2 * gib);
+    a.trim();
+    REQUIRE(dev.held == 0 && dev.live.empty());
+    a.trim();
+    REQUIRE(a.get(&p, gib, stream(1)) == hipSuccess && p);
+    a.put(p);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, void (*)()> checks = {{"grow", grow}, {"freed_block_in_pool", freed_block_in_pool}};
+    const std::map<std::string, void (*)()> checks = {{"grow", grow}, {"freed_block_in_pool", freed_block_in_pool},
+                                                               {"other_contexts", other_contexts}};
     const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end())
         return 2;

@@ -10,7 +10,7 @@ CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "buffers
 
 
 @pytest.mark.skipif(not os.path.exists(CHECK), reason="check not built")
-@pytest.mark.parametrize("name", ["grow", "freed_block_in_pool"])
+@pytest.mark.parametrize("name", ["grow", "freed_block_in_pool", "other_contexts"])
 def test_buffers_on_a_simulated_device(name):
     r = subprocess.run([CHECK, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
