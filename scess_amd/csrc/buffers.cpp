@@ -313,8 +313,17 @@ static hipError_t ring_copy(Ring &r, char *h, char *d, size_t bytes, hipStream_t
     return e;
 }
 
+// Pinned and managed host memory is copied directly (the ring would only add a copy), and device memory has to be
+static bool pageable(const void *h) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, h) == hipSuccess)
+        return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
 hipError_t copy_to_host(void *h, const void *d, size_t bytes, hipStream_t s) {
-    if (bytes >= kLarge) {
+    if (bytes >= kLarge && pageable(h)) {
         if (const std::shared_ptr<Ring> r = ring()) {
             std::unique_lock<std::mutex> lk(r->use, std::try_to_lock);  // in use by another thread: the plain way
             if (lk.owns_lock() && r->ready(bytes))
@@ -326,7 +335,7 @@ hipError_t copy_to_host(void *h, const void *d, size_t bytes, hipStream_t s) {
 }
 
 hipError_t copy_to_device(void *d, const void *h, size_t bytes, hipStream_t s) {
-    if (bytes >= kLarge) {
+    if (bytes >= kLarge && pageable(h)) {
         if (const std::shared_ptr<Ring> r = ring()) {
             std::unique_lock<std::mutex> lk(r->use, std::try_to_lock);  // in use by another thread: the plain way
             if (lk.owns_lock() && r->ready(bytes))

@@ -53,11 +53,11 @@ private:
     int device_ = -1;  // of the blocks; -1 before the first
 };
 
-// Copies of any size between pageable host memory and the device, ordered on stream s as hipMemcpyAsync would be. Large
-// ones go through a ring of pinned chunks shared by the process, filled or emptied by a few threads: one thread's
-// memcpy (and its page faults in a new array) runs at 5-13 GB/s, the link at 50 (gradients of o=20, v=200 to the host,
-// 1.6 GB: 100 ms -> 30; transform of 58 functions, 91 MB each way: 14.7 -> 9.6). copy_to_host returns when the data is
-// there; copy_to_device when `h` has been read.
+// Copies of any size between host memory and the device, ordered on stream s as hipMemcpyAsync would be. Large ones of
+// pageable memory go through a ring of pinned chunks shared by the process, filled or emptied by a few threads: one
+// thread's memcpy (and its page faults in a new array) runs at 5-13 GB/s, the link at 50 (gradients of o=20, v=200 to the
+// host, 1.6 GB: 100 ms -> 30; transform of 58 functions, 91 MB each way: 14.7 -> 9.6). copy_to_host returns when the data
+// is there; copy_to_device when a pageable `h` has been read.
 hipError_t copy_to_host(void *h, const void *d, size_t bytes, hipStream_t s);
 hipError_t copy_to_device(void *d, const void *h, size_t bytes, hipStream_t s);
 // The ring and its threads exist while a context does
