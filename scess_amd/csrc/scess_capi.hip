@@ -770,11 +770,13 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
         }
         stats->flops_algorithmic = 2.0 * (double)o * o * o * (double)v * v * v * (double)(o + v) *
                                    (ordered_all > 0.0 ? ordered / ordered_all : 1.0);
-        // rows and columns as the kernels issue them: MFMA blocks of 16 (blocks wholly past v skipped);
-        // the int8-digit kernel computes every 32-row block of its 64 x 64 tiles
+        // as the kernels issue them: rows and columns in MFMA blocks of 16 (blocks wholly past v skipped; the int8-digit
+        // kernel computes every 32-row block of its 64 x 64 tiles), K padded to whole chunks. FP64: only the k-steps (4 k)
+        // of a chunk that exist, and the four fixed indices of a group also where some are past v.
         const double rows = (double)round_up(v, prec == PI8 ? 64 : 16);
-        stats->flops_executed = ((double)nshare - 0.5 * (double)ndeg) * 2.0 * (double)v * rows * rows *
-                                (6.0 * (double)op.vK + 6.0 * (double)op.oK);
+        const double fixed = (double)(prec == P64 ? round_up(v, 4) : v);
+        const double depth = prec == P64 ? (double)(round_up(v, 4) + round_up(o, 4)) : (double)(op.vK + op.oK);
+        stats->flops_executed = ((double)nshare - 0.5 * (double)ndeg) * 2.0 * fixed * rows * rows * 6.0 * depth;
     }
     destroy_events();
     return rc;
