@@ -184,7 +184,8 @@ typedef struct scess_ccsd_result {
 typedef void (*scess_ccsd_log)(void *user, int iteration, double e_corr, double dE, double rms);
 
 int scess_ccsd_set_inputs(scess_ctx *ctx, const scess_ccsd_in *in);
-/* One Jacobi update t <- R(t)/D (UpdateAmplitudes, RCCSD.cpp:101-237); t1 (i,a), t2 (i,j,a,b) ColMajor. */
+/* One Jacobi update t <- R(t)/D (UpdateAmplitudes, RCCSD.cpp:101-237); t1 (i,a), t2 (i,j,a,b) ColMajor. With chol_vv
+ * a t2 with t_ij^ab = t_ji^ba, as every CCSD iterate has, takes a shorter form of the ladder; it need not have it. */
 int scess_ccsd_update(scess_ctx *ctx, const double *t1, const double *t2, double *t1_new, double *t2_new);
 /* E = sum (2<ij|ab> - <ij|ba>) tau_ij^ab (+ F12 coupling) (RCCSD.cpp:85-98). */
 int scess_ccsd_energy(scess_ctx *ctx, const double *t1, const double *t2, double *e_corr);

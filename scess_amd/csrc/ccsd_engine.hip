@@ -182,6 +182,44 @@ __global__ __launch_bounds__(256) void ladder_scatter_kernel(const double *rp, c
     }
 }
 
+// out[0] = max |t_ij^ab - t_ji^ba|, out[1] = max |t_ij^ab| as bit patterns (which order as the values, NaN above all); both
+// zero before. One work-group per (32 x 32 tile of a, b; pair i >= j); bound by one read of t.
+constexpr int kPairRow = 65535;  // pairs along y of the grid, the rest along z
+__global__ __launch_bounds__(256) void pair_asymmetry_kernel(const double *t, int o, int v, int nt, unsigned long long *out) {
+    __shared__ double ji[32][33];
+    __shared__ unsigned long long best[2];
+    const int pair = blockIdx.y + kPairRow * blockIdx.z;
+    if (pair >= tri(o))
+        return;
+    int i, j;
+    tile_pair(pair, i, j);
+    const int ta = blockIdx.x / nt, tb = blockIdx.x - ta * nt, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const double *x = t + ((int64_t)i * o + j) * v * v, *y = t + ((int64_t)j * o + i) * v * v;
+    if (threadIdx.x < 2)
+        best[threadIdx.x] = 0;
+    for (int r = ty; r < 32; r += 8) {
+        const int b = tb * 32 + r, a = ta * 32 + tx;
+        ji[r][tx] = a < v && b < v ? y[(int64_t)b * v + a] : 0.0;
+    }
+    __syncthreads();
+    unsigned long long d = 0, m = 0;
+    auto bits = [](double z) { return (unsigned long long)__double_as_longlong(fabs(z)); };
+    for (int r = ty; r < 32; r += 8) {
+        const int a = ta * 32 + r, b = tb * 32 + tx;
+        if (a < v && b < v) {
+            const double p = x[(int64_t)a * v + b], q = ji[tx][r];
+            d = max(d, bits(p - q));
+            m = max(m, max(bits(p), bits(q)));
+        }
+    }
+    atomicMax(&best[0], d);
+    atomicMax(&best[1], m);
+    __syncthreads();
+    if (threadIdx.x < 2 &&
+        best[threadIdx.x] > __hip_atomic_load(&out[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&out[threadIdx.x], best[threadIdx.x]);
+}
+
 // A whole einsum of a small system in one launch, straight from the operands: G lanes per output element, lane g
 // summing k = g, g + G, ... (then a fixed xor tree). The operand offsets of up to KT values of the summed index are
 // decomposed once per work-group into LDS. Bound by launches, not by the chip: the CCSD of a water-sized molecule is
@@ -760,6 +798,12 @@ double Engine::dot(const double *x, const double *y, int64_t n) {
 Engine::~Engine() {
     if (dotbuf)
         (void)hipFree(dotbuf);
+    if (asym)
+        (void)hipFree(asym);
+    if (asym_host)
+        (void)hipHostFree(asym_host);
+    if (asym_done)
+        (void)hipEventDestroy(asym_done);
 }
 
 // ------------------------------------------------------------- CCSD update
@@ -773,6 +817,29 @@ void CcsdState::make_tau(Engine &E, const DTensor &t1, const DTensor &t2, DTenso
 static void plus_transpose_add(Engine &E, DTensor &R, const DTensor &X, double alpha) {
     E.permute("ijab", X.p, X.dims, "ijab", R.p, R.dims, alpha, 1.0);
     E.permute("jiba", X.p, X.dims, "ijab", R.p, R.dims, alpha, 1.0);
+}
+
+void Engine::pair_check(const DTensor &t) {
+    const int64_t o = t.dims[0], v = t.dims[2], nt = (v + 31) / 32, np = o * (o + 1) / 2;
+    if (!asym_host) {
+        check(hipMalloc((void **)&asym, 16), "hipMalloc (symmetry of t2)");
+        check(hipEventCreateWithFlags(&asym_done, hipEventDisableTiming), "hipEventCreate");
+        check(hipHostMalloc((void **)&asym_host, 16, hipHostMallocDefault), "hipHostMalloc (symmetry of t2)");
+    }
+    check(hipMemsetAsync(asym, 0, 16, stream), "memset (symmetry of t2)");
+    const dim3 grid((unsigned)(nt * nt), (unsigned)std::min<int64_t>(np, kPairRow), (unsigned)((np + kPairRow - 1) / kPairRow));
+    hipLaunchKernelGGL(pair_asymmetry_kernel, grid, dim3(256), 0, stream, t.p, (int)o, (int)v, (int)nt, asym);
+    check(hipGetLastError(), "symmetry of t2");
+    check(hipMemcpyAsync(asym_host, asym, 16, hipMemcpyDeviceToHost, stream), "copy (symmetry of t2)");
+    check(hipEventRecord(asym_done, stream), "hipEventRecord");
+}
+
+bool Engine::pair_symmetric() {
+    check(hipEventSynchronize(asym_done), "symmetry of t2");
+    // well above what rounding leaves in the amplitudes of an update (o=5, v=24 to o=16, v=157: 2e-16, FP32 2e-8, BF16x3 5e-8
+    // of the largest), below the error of the products themselves
+    const double tol = prec == P64 ? 1e-11 : prec == P32 ? 1e-6 : 1e-5;
+    return asym_host[0] <= tol * asym_host[1];
 }
 
 // Particle-particle ladder sum_cd (ac|bd) tau_ij^cd from the Cholesky factor, (a,b) tiles of TAB x TAB
@@ -929,8 +996,10 @@ void CcsdState::ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R) {
     }
 }
 
-void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
+void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2, const bool *symmetric) {
     const int64_t O = o, Vv = v;
+    if (!vvvv_phys.p && !symmetric)
+        E.pair_check(t2);  // read where the ladder comes
     DTensor tau = E.alloc({O, O, Vv, Vv});
     make_tau(E, t1, t2, tau);
     DTensor Foo = E.alloc({O, O}), Fvv = E.alloc({Vv, Vv}), Fov = E.alloc({O, Vv});
@@ -1003,15 +1072,20 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2) {
         E.einsum("kcbd,ka->abcd", ovvv, &t1, Wvvvv, -1.0, 1.0);
         E.einsum("abcd,ijcd->ijab", Wvvvv, &tau, t2n, 1.0, 1.0);
     } else {
-        if (E.prec == P64 && O * (O + 1) / 2 <= 65535)  // (pairs are a grid dimension)
+        const bool sym = symmetric ? *symmetric : E.pair_symmetric();  // tau_ij^cd = tau_ji^dc
+        if (sym && E.prec == P64 && O * (O + 1) / 2 <= 65535)  // (pairs are a grid dimension)
             ladder_symmetric(E, tau, t2n);
-        else  // (its rounding is kept: packing would split and round other values)
+        else  // (the other precisions keep their rounding: packing would split and round other values)
             ladder_from_factor(E, tau, t2n);
         DTensor Z = E.alloc({O, Vv, O, O});  // Z[k][a][i][j] = sum_cd (kd|ac) tau_ij^cd
         E.einsum("kdac,ijcd->kaij", ovvv, &tau, Z, 1.0, 0.0);
         E.einsum("kaij,kb->ijab", Z, &t1, t2n, -1.0, 1.0);
-        // sum_cd (kc|bd) tau_ij^cd = Z[k][b][j][i] (tau_ij^cd = tau_ji^dc)
-        E.einsum("kbji,ka->ijab", Z, &t1, t2n, -1.0, 1.0);
+        if (sym) {  // sum_cd (kc|bd) tau_ij^cd = Z[k][b][j][i]
+            E.einsum("kbji,ka->ijab", Z, &t1, t2n, -1.0, 1.0);
+        } else {
+            E.einsum("kcbd,ijcd->kbij", ovvv, &tau, Z, 1.0, 0.0);
+            E.einsum("kbij,ka->ijab", Z, &t1, t2n, -1.0, 1.0);
+        }
     }
     {
         DTensor X = E.alloc({O, O, Vv, Vv});

@@ -53,6 +53,15 @@ struct Engine {
     // out[q] = dot(x, y[q]) for q < m <= kMaxDots, one launch and one copy
     static constexpr int kMaxDots = 8;
     void dots(const double *x, const double *const *y, int m, int64_t n, double *out);
+    // Whether t (i, j, a, b) has t_ij^ab = t_ji^ba within the rounding of precision `prec`: pair_check() starts the
+    // comparison, pair_symmetric() waits for it
+    void pair_check(const DTensor &t);
+    bool pair_symmetric();
+
+private:
+    unsigned long long *asym = nullptr;  // device
+    double *asym_host = nullptr;         // pinned: max |t_ij^ab - t_ji^ba|, max |t_ij^ab|
+    hipEvent_t asym_done = nullptr;
 };
 
 // Resident integral blocks of SolveRCCSD_DIIS (src/Quantum/CC/RCCSD.cpp:31-44), row-major with
@@ -65,7 +74,8 @@ struct CcsdState {
     void make_tau(Engine &E, const DTensor &t1, const DTensor &t2, DTensor &tau);
     void ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R);
     void ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R);
-    void update(Engine &E, DTensor &t1, DTensor &t2);  // one Jacobi update (UpdateAmplitudes)
+    // One Jacobi update (UpdateAmplitudes); symmetric: whether t_ij^ab = t_ji^ba is known to hold or not, null to find out
+    void update(Engine &E, DTensor &t1, DTensor &t2, const bool *symmetric = nullptr);
     double energy(Engine &E, const DTensor &t1, const DTensor &t2);
 };
 

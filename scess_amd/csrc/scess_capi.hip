@@ -1428,6 +1428,13 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
             scess::DTensor z1 = E.alloc({o, v}, true);
             HIP_TRY(c, scess::ccsd_jacobi(z1.p, t2.p, S.e.p, (int)o, (int)v, c->stream));
         }
+        // an update keeps t_ij^ab = t_ji^ba, which the driver need not have
+        bool symmetric = true;
+        if (!S.vvvv_phys.p) {
+            const PrecScope ps(E, c->ccsd_prec);
+            E.pair_check(t2);
+            symmetric = E.pair_symmetric();
+        }
         std::vector<scess::DTensor> amps, errs;
         double dotB[MAX_DIIS_VECS][MAX_DIIS_VECS] = {};  // products of the error vectors
         double E_last = 1.7976931348623157e308;
@@ -1442,7 +1449,7 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
             HIP_TRY(c, hipMemcpyAsync(prev.p, t1.p, 8 * n1, hipMemcpyDeviceToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(prev.p + n1, t2.p, 8 * n2, hipMemcpyDeviceToDevice, c->stream));
             const PrecScope ps(E, c->ccsd_prec);
-            S.update(E, t1, t2);
+            S.update(E, t1, t2, &symmetric);
             HIP_TRY(c, hipMemcpyAsync(upd.p, t1.p, 8 * n1, hipMemcpyDeviceToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(upd.p + n1, t2.p, 8 * n2, hipMemcpyDeviceToDevice, c->stream));
             E.axpby(change.p, upd.p, prev.p, 1.0, -1.0, nt);
