@@ -555,9 +555,12 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
     };
     const int64_t nb = prod(Lb), M = prod(Lm), N = prod(Ln), K = prod(Lk);
     // Small FP64 contractions in one launch (contract_kernel). The line is where its products at some 0.5 TFLOP/s
-    // cost what the GEMM path's extra launches do (about 40 us): 1 << 24 products.
-    if (prec == P64 && nb * M * N * std::max<int64_t>(K, 1) <= (int64_t)1 << 24 && A.size() < (int64_t)1 << 31 &&
-        B->size() < (int64_t)1 << 31) {
+    // cost what the GEMM path's extra launches do (about 40 us): 1 << 24 products. A longer sum than 16384 over few outputs
+    // (Foo: o^2 of o v^2) fills only a few work-groups, where the GEMM splits it over the chip: an update at o=1, v=200 takes
+    // 24.7 ms without that bound and 24.1 with it, o=2, v=150 9.0 / 8.6, o=10, v=100 6.2 / 6.0 (4096: 6.0, 65536: 6.0 but 9.0
+    // at o=2, v=150; 1024 costs o=5, v=100 4.0 ms against 3.8).
+    if (prec == P64 && K <= 16384 && nb * M * N * std::max<int64_t>(K, 1) <= (int64_t)1 << 24 &&
+        A.size() < (int64_t)1 << 31 && B->size() < (int64_t)1 << 31) {
         contract(la, A, lb, *B, lc, Lk, C, alpha, beta);
         return;
     }
