@@ -36,3 +36,10 @@ def _check(o, v, seed):
 @pytest.mark.parametrize("o,v", [(2, 90), (2, 91)])
 def test_long_sums(o, v):
     _check(o, v, v)
+
+
+# Z = sum_cd (kd|ac) tau_ij^cd: (kd|ac) read in place as a batch over k with the sum over d, c split (96), permuted because
+# its rows are too few per k (94) or not 16-byte aligned (97)
+@pytest.mark.parametrize("o,v", [(4, 94), (4, 96), (4, 97)])
+def test_operands_in_place(o, v):
+    _check(o, v, v)
