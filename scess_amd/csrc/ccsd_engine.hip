@@ -616,16 +616,15 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
             if (!direct)
                 X = alloc({mo, mi, n});
             GemmArgs g{};
-            g.nseg = 1;
             g.M = (int)mi;
             g.N = (int)n;
             g.alpha = direct ? alpha : 1.0;
             g.ow = !direct || beta == 0.0;
             g.splits = 1;
-            g.seg[0].K1 = (int)k1;
-            g.seg[0].K2 = (int)k2;
-            g.seg[0].A = {T.p, k2, mi * k2, 1, k1 * mi * k2};
-            g.seg[0].B = {p2, K, k2, 1, 0};
+            g.seg.K1 = (int)k1;
+            g.seg.K2 = (int)k2;
+            g.seg.A = {T.p, k2, mi * k2, 1, k1 * mi * k2};
+            g.seg.B = {p2, K, k2, 1, 0};
             g.C = direct ? C.p : X.p;
             g.sCm = n;
             g.sCn = 1;
@@ -694,16 +693,15 @@ void Engine::einsum(const std::string &spec, const DTensor &A, const DTensor *B,
     }
     if (M > 0 && N > 0 && K > 0) {
         GemmArgs g{};
-        g.nseg = 1;
         g.M = (int)M;
         g.N = (int)N;
         g.alpha = direct ? alpha : 1.0;
         g.ow = !direct || beta == 0.0;
         g.splits = 1;
-        g.seg[0].K1 = 1;
-        g.seg[0].K2 = (int)(split ? Ks : K);
-        g.seg[0].A = {pA, Ks, 0, 1, M * Ks};
-        g.seg[0].B = {pB, Ks, 0, 1, N * Ks};
+        g.seg.K1 = 1;
+        g.seg.K2 = (int)(split ? Ks : K);
+        g.seg.A = {pA, Ks, 0, 1, M * Ks};
+        g.seg.B = {pB, Ks, 0, 1, N * Ks};
         g.C = direct ? C.p : Cp.p;
         g.sCm = N;
         g.sCn = 1;
@@ -869,20 +867,19 @@ void CcsdState::ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R) {
             const int64_t tb = std::min(TAB, v - b0);
             // I[(a,c)][(b,d)] = sum_P L[a][c][P] L[b][d][P]
             GemmArgs g{};
-            g.nseg = 1;
             g.M = (int)(ta * v);
             g.N = (int)(tb * v);
             g.alpha = 1.0;
             g.splits = 1;
-            g.seg[0].K1 = 1;
+            g.seg.K1 = 1;
             if (split) {
-                g.seg[0].K2 = (int)Ps;
-                g.seg[0].A = {Ls.p + a0 * v * Ps, Ps, 0, 1, 0};
-                g.seg[0].B = {Ls.p + b0 * v * Ps, Ps, 0, 1, 0};
+                g.seg.K2 = (int)Ps;
+                g.seg.A = {Ls.p + a0 * v * Ps, Ps, 0, 1, 0};
+                g.seg.B = {Ls.p + b0 * v * Ps, Ps, 0, 1, 0};
             } else {
-                g.seg[0].K2 = (int)nP;
-                g.seg[0].A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};  // rows (a, c), K = P contiguous
-                g.seg[0].B = {Lvv.p + b0 * v * nP, nP, 0, 1, 0};
+                g.seg.K2 = (int)nP;
+                g.seg.A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};  // rows (a, c), K = P contiguous
+                g.seg.B = {Lvv.p + b0 * v * nP, nP, 0, 1, 0};
             }
             g.ow = 1;
             g.C = I.p;
@@ -893,22 +890,21 @@ void CcsdState::ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R) {
             check(launch_gemm(g, 1, E.stream), "ladder integrals");
             // R[i][j][a][b] += sum_{c,d} I[a][c][b][d] tau[i][j][c][d]; batch a, rows b, K = (c, d)
             GemmArgs h{};
-            h.nseg = 1;
             h.M = (int)tb;
             h.N = (int)(o * o);
             h.alpha = 1.0;
             h.splits = 1;
-            h.seg[0].K1 = (int)v;
+            h.seg.K1 = (int)v;
             DTensor Is;
             if (split) {  // I of this tile in pre-split rows (a, c, b), K = d
                 Is = E.permute_split("acbd", I.p, {ta, v, tb, v}, "acbd", {ta, v, tb, v}, v);
-                h.seg[0].K2 = (int)Vs;
-                h.seg[0].A = {Is.p, Vs, tb * Vs, 1, v * tb * Vs};
-                h.seg[0].B = {taus.p, v * Vs, Vs, 1, 0};
+                h.seg.K2 = (int)Vs;
+                h.seg.A = {Is.p, Vs, tb * Vs, 1, v * tb * Vs};
+                h.seg.B = {taus.p, v * Vs, Vs, 1, 0};
             } else {
-                h.seg[0].K2 = (int)v;
-                h.seg[0].A = {I.p, v, tb * v, 1, v * tb * v};
-                h.seg[0].B = {tau.p, v * v, v, 1, 0};
+                h.seg.K2 = (int)v;
+                h.seg.A = {I.p, v, tb * v, 1, v * tb * v};
+                h.seg.B = {tau.p, v * v, v, 1, 0};
             }
             h.prec = split ? PB3S : E.prec;
             h.C = R.p + a0 * v + b0;
@@ -944,15 +940,14 @@ void CcsdState::ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R) {
         const int64_t ta = std::min(TA, v - a0), nb = a0 + ta, rows = ta * nb;
         // I[(a,c)][(b,d)] = sum_P L[a][c][P] L[b][d][P], b < a0 + ta
         GemmArgs g{};
-        g.nseg = 1;
         g.M = (int)(ta * v);
         g.N = (int)(nb * v);
         g.alpha = 1.0;
         g.splits = 1;
-        g.seg[0].K1 = 1;
-        g.seg[0].K2 = (int)nP;
-        g.seg[0].A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};
-        g.seg[0].B = {Lvv.p, nP, 0, 1, 0};
+        g.seg.K1 = 1;
+        g.seg.K2 = (int)nP;
+        g.seg.A = {Lvv.p + a0 * v * nP, nP, 0, 1, 0};
+        g.seg.B = {Lvv.p, nP, 0, 1, 0};
         g.C = I.p;
         g.sCm = nb * v;
         g.sCn = 1;
@@ -965,15 +960,14 @@ void CcsdState::ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R) {
             if (K < 1 || N < 1)
                 return;
             GemmArgs h{};
-            h.nseg = 1;
             h.M = (int)rows;
             h.N = (int)N;
             h.alpha = 1.0;
             h.splits = 1;
-            h.seg[0].K1 = 1;
-            h.seg[0].K2 = (int)K;
-            h.seg[0].A = {S.p, ld, 0, 1, 0};
-            h.seg[0].B = {T.p, ld, 0, 1, 0};
+            h.seg.K1 = 1;
+            h.seg.K2 = (int)K;
+            h.seg.A = {S.p, ld, 0, 1, 0};
+            h.seg.B = {T.p, ld, 0, 1, 0};
             h.C = out.p;
             h.sCm = N;
             h.sCn = 1;

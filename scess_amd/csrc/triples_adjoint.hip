@@ -198,7 +198,7 @@ hipError_t launch_adjoint_g(int prec, const EpiArgs &a, double dE, double *GW, d
 }
 
 // -------------------------------------------------------------------- GEMM
-// C[b][m][n] += alpha sum_seg sum_k1 sum_k2 A(m, k1, k2) B(n, k1, k2); with splits > 1, split p handles a fixed contiguous
+// C[b][m][n] += alpha sum_k1 sum_k2 A(m, k1, k2) B(n, k1, k2); with splits > 1, split p handles a fixed contiguous
 // range of the 16-deep K chunks and writes its partial to scratch[p]; gemm_reduce_kernel adds them in split order.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs g) {
 }
 
 // ------------------------------------------- GEMM with K-contiguous operands
-// The same contraction when every segment has A.s2 == B.s2 == 1 (the inner K index is the
+// The same contraction when A.s2 == B.s2 == 1 (the inner K index is the
 // contiguous one, as the einsum engine lays its operands out) and even strides: rows are read as
 // 16-byte vectors (two doubles of K), staged through registers into a double-buffered LDS ring
 // with the rows' vectors XOR-permuted (conflict-free 16-lane fragment reads), and each of the 2x2
@@ -273,10 +273,8 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
     const int m0 = tm * BM, n0 = tn * BN;
     const int beta = byz % ny, split = byz / ny;
 
-    // segment values as scalars: a runtime-indexed local array would live in scratch memory
-    const int nk20 = (g.seg[0].K2 + 15) / 16, nk21 = g.nseg > 1 ? (g.seg[1].K2 + 15) / 16 : 1;
-    const int nch0 = g.seg[0].K1 * nk20, nch1 = g.nseg > 1 ? g.seg[1].K1 * nk21 : 0;
-    const int total = nch0 + nch1;
+    const GemmSeg &sg = g.seg;
+    const int nk = (sg.K2 + 15) / 16, total = sg.K1 * nk;
     const int c_begin = (int)((int64_t)total * split / g.splits), c_end = (int)((int64_t)total * (split + 1) / g.splits);
 
     d4 acc[BLK][BLKN];
@@ -297,10 +295,7 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
     // thread t loads vectors q = t + 256 u (u < NV) of the BM x 8 vector tile: row q / 8, vector q % 8
     d2v ra[NV], rb[NV];
     auto fetch = [&](int ch) {
-        const bool s0 = ch < nch0;
-        const int cl = s0 ? ch : ch - nch0, nk = s0 ? nk20 : nk21;
-        const GemmSeg &sg = s0 ? g.seg[0] : g.seg[1];
-        const int k1 = cl / nk, k0 = (cl - k1 * nk) * 16;
+        const int k1 = ch / nk, k0 = (ch - k1 * nk) * 16;
         const double *pa = sg.A.base + (int64_t)beta * sg.A.sb + (int64_t)k1 * sg.A.s1;
         const double *pb = sg.B.base + (int64_t)beta * sg.B.sb + (int64_t)k1 * sg.B.s1;
 #pragma unroll
@@ -492,62 +487,51 @@ __global__ __launch_bounds__(256) void gemm_kc_kernel(GemmArgs g) {
             larow[u] = r;
             lak[u] = 2 * ((qq & 7) ^ kswz(r));
         }
-        auto chunk_pos = [&](int ch, const GemmSeg *&sg, int &k1, int &k0) {
-            const bool s0 = ch < nch0;
-            const int cl = s0 ? ch : ch - nch0, nk = s0 ? nk20 : nk21;
-            sg = s0 ? &g.seg[0] : &g.seg[1];
-            k1 = cl / nk;
-            k0 = (cl - k1 * nk) * 16;
-        };
         auto issue = [&](int ch, int st) {
-            const GemmSeg *sg;
-            int k1, k0;
-            chunk_pos(ch, sg, k1, k0);
-            const double *pa = sg->A.base + (int64_t)beta * sg->A.sb + (int64_t)k1 * sg->A.s1;
-            const double *pb = sg->B.base + (int64_t)beta * sg->B.sb + (int64_t)k1 * sg->B.s1;
+            const int k1 = ch / nk, k0 = (ch - k1 * nk) * 16;
+            const double *pa = sg.A.base + (int64_t)beta * sg.A.sb + (int64_t)k1 * sg.A.s1;
+            const double *pb = sg.B.base + (int64_t)beta * sg.B.sb + (int64_t)k1 * sg.B.s1;
             char *base = lds[st];
 #pragma unroll
             for (int u = 0; u < NIW; u++) {
-                const int k = k0 + lak[u], kk = k + 1 < sg->K2 ? k : 0;  // inside the row, else its first vector
+                const int k = k0 + lak[u], kk = k + 1 < sg.K2 ? k : 0;  // inside the row, else its first vector
                 const int gm = min(m0 + larow[u], g.M - 1);
-                __builtin_amdgcn_global_load_lds((const void *)(pa + (int64_t)gm * sg->A.sr + kk),
+                __builtin_amdgcn_global_load_lds((const void *)(pa + (int64_t)gm * sg.A.sr + kk),
                                                  (lds_void *)(base + (wave * NIW + u) * 1024), 16, 0, 0);
             }
 #pragma unroll
             for (int u = 0; u < NIWB; u++) {
-                const int k = k0 + lk[u], kk = k + 1 < sg->K2 ? k : 0;
+                const int k = k0 + lk[u], kk = k + 1 < sg.K2 ? k : 0;
                 const int gn = min(n0 + lrow[u], g.N - 1);
-                __builtin_amdgcn_global_load_lds((const void *)(pb + (int64_t)gn * sg->B.sr + kk),
+                __builtin_amdgcn_global_load_lds((const void *)(pb + (int64_t)gn * sg.B.sr + kk),
                                                  (lds_void *)(base + OPB + (wave * NIWB + u) * 1024), 16, 0, 0);
             }
         };
         // after the chunk has landed: the vectors reaching past K2 get (x[k], 0) or (0, 0)
         auto fixup = [&](int ch, int st) {
-            const GemmSeg *sg;
-            int k1, k0;
-            chunk_pos(ch, sg, k1, k0);
-            if (k0 + 16 <= sg->K2)
+            const int k1 = ch / nk, k0 = (ch - k1 * nk) * 16;
+            if (k0 + 16 <= sg.K2)
                 return false;
-            const double *pa = sg->A.base + (int64_t)beta * sg->A.sb + (int64_t)k1 * sg->A.s1;
-            const double *pb = sg->B.base + (int64_t)beta * sg->B.sb + (int64_t)k1 * sg->B.s1;
+            const double *pa = sg.A.base + (int64_t)beta * sg.A.sb + (int64_t)k1 * sg.A.s1;
+            const double *pb = sg.B.base + (int64_t)beta * sg.B.sb + (int64_t)k1 * sg.B.s1;
             char *base = lds[st];
 #pragma unroll
             for (int u = 0; u < NIW; u++) {
                 const int k = k0 + lak[u];
-                if (k + 1 < sg->K2)
+                if (k + 1 < sg.K2)
                     continue;
                 const int gm = min(m0 + larow[u], g.M - 1);
                 *(d2v *)(base + (wave * NIW + u) * 1024 + lane * 16) =
-                    d2v{k < sg->K2 ? pa[(int64_t)gm * sg->A.sr + k] : 0.0, 0.0};
+                    d2v{k < sg.K2 ? pa[(int64_t)gm * sg.A.sr + k] : 0.0, 0.0};
             }
 #pragma unroll
             for (int u = 0; u < NIWB; u++) {
                 const int k = k0 + lk[u];
-                if (k + 1 < sg->K2)
+                if (k + 1 < sg.K2)
                     continue;
                 const int gn = min(n0 + lrow[u], g.N - 1);
                 *(d2v *)(base + OPB + (wave * NIWB + u) * 1024 + lane * 16) =
-                    d2v{k < sg->K2 ? pb[(int64_t)gn * sg->B.sr + k] : 0.0, 0.0};
+                    d2v{k < sg.K2 ? pb[(int64_t)gn * sg.B.sr + k] : 0.0, 0.0};
             }
             return true;  // wave-uniform: every lane of the block sees the same chunk
         };
@@ -621,7 +605,7 @@ template <int RB, int CB> struct GemmNT {
     // offsets of its vectors were clamped into the row)
     __device__ inline int issue(int st) {
         char *base = lds + st * 2 * OPB;
-        const int rem = k2c == nk2 - 1 ? g.seg[0].K2 - 16 * k2c : 16;
+        const int rem = k2c == nk2 - 1 ? g.seg.K2 - 16 * k2c : 16;
         const int last = (rem - 1) & ~1;  // first k of the last vector of the row
 #pragma unroll
         for (int h = 0; h < 4; h++) {
@@ -638,8 +622,8 @@ template <int RB, int CB> struct GemmNT {
         pb += 16;
         if (++k2c == nk2) {
             k2c = 0;
-            pa += g.seg[0].A.s1 - 16 * nk2;
-            pb += g.seg[0].B.s1 - 16 * nk2;
+            pa += g.seg.A.s1 - 16 * nk2;
+            pb += g.seg.B.s1 - 16 * nk2;
         }
         left--;
         return (rem + 3) >> 2 | (rem & 3 ? 8 : 0);
@@ -691,7 +675,7 @@ template <int RB, int CB> struct GemmNT {
                 fc[1][y] = fc[0][y];
         };
         using std::integral_constant;
-        const int lq = lane >> 4, keep = g.seg[0].K2 & 3;
+        const int lq = lane >> 4, keep = g.seg.K2 & 3;
         wait_vm_lgkm0();
         __syncthreads();
         tiles(0);
@@ -776,7 +760,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int am = (int)((int64_t)tm * nbm / ntm), an = (int)((int64_t)tn * nbn / ntn);
     const int rb = (int)((int64_t)(tm + 1) * nbm / ntm) - am, cb = (int)((int64_t)(tn + 1) * nbn / ntn) - an;
     const int quad = wave ^ (lin & 3);  // the uneven quadrants of neighbouring tiles on different SIMDs
-    const int nk2 = (g.seg[0].K2 + 15) >> 4, total = g.seg[0].K1 * nk2;
+    const int nk2 = (g.seg.K2 + 15) >> 4, total = g.seg.K1 * nk2;
     const int c_begin = (int)((int64_t)total * split / g.splits), c_end = (int)((int64_t)total * (split + 1) / g.splits);
     const int k1 = c_begin / nk2, k2c = c_begin - k1 * nk2;
     const int nr = (rb + 1 - (quad >> 1)) >> 1, nc = (cb + 1 - (quad & 1)) >> 1;  // blocks of this wave's quadrant
@@ -797,7 +781,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         w.k2c = k2c;
         w.nk2 = nk2;
         w.left = c_end - c_begin;
-        const GemmOp &A = g.seg[0].A, &B = g.seg[0].B;
+        const GemmOp &A = g.seg.A, &B = g.seg.B;
         w.pa = A.base + (int64_t)beta * A.sb + (int64_t)k1 * A.s1 + 16 * k2c + (int64_t)w.m0 * A.sr;
         w.pb = B.base + (int64_t)beta * B.sb + (int64_t)k1 * B.s1 + 16 * k2c + (int64_t)w.n0 * B.sr;
         const int lr = lane & 15, lq = lane >> 4;
@@ -839,34 +823,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // 0: not K-contiguous; 1: K-contiguous; 2: K-contiguous with 16-byte aligned rows (vector loads)
 static int k_contiguous(const GemmArgs &g) {
     int r = 2;
-    for (int s = 0; s < g.nseg; s++) {
-        const GemmSeg &sg = g.seg[s];
-        const GemmOp *ops[2] = {&sg.A, &sg.B};
-        for (const GemmOp *op : ops) {
-            if (op->s2 != 1)
-                return 0;
-            if ((op->sr & 1) || (op->s1 & 1) || (op->sb & 1) || (((uintptr_t)op->base) & 15))
-                r = 1;
-        }
+    for (const GemmOp *op : {&g.seg.A, &g.seg.B}) {
+        if (op->s2 != 1)
+            return 0;
+        if ((op->sr & 1) || (op->s1 & 1) || (op->sb & 1) || (((uintptr_t)op->base) & 15))
+            r = 1;
     }
     return r;
 }
 
 hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
     {  // the kernels index K chunks (16 deep) with 32-bit integers
-        int64_t chunks = 0;
-        for (int q = 0; q < g.nseg; q++)
-            chunks += (int64_t)g.seg[q].K1 * ((g.seg[q].K2 + 15) / 16);
-        if (chunks >= (int64_t)1 << 31 || g.nseg < 1 || g.nseg > 2)
+        if ((int64_t)g.seg.K1 * ((g.seg.K2 + 15) / 16) >= (int64_t)1 << 31)
             return hipErrorInvalidValue;
     }
     const int kc = k_contiguous(g);
     if (!kc)  // the callers lay their operands out with K contiguous
         return hipErrorInvalidValue;
     // FP64: 128 x 128 tiles, unless rows of a tile are too far apart for lane offsets of 32 bits
-    const GemmSeg &s0 = g.seg[0];
+    const GemmSeg &s0 = g.seg;
     const double far = 128.0 * 8.0 * (double)std::max(s0.A.sr, s0.B.sr);
-    if (g.prec == P64 && kc == 2 && g.nseg == 1 && s0.K2 >= 1 && s0.K1 >= 1 && g.M >= 1 && g.N >= 1 && s0.A.sr >= 0 &&
+    if (g.prec == P64 && kc == 2 && s0.K2 >= 1 && s0.K1 >= 1 && g.M >= 1 && g.N >= 1 && s0.A.sr >= 0 &&
         s0.B.sr >= 0 && far < 4294967296.0) {
         const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
         if (tiles > 0x7fffffff)
@@ -878,9 +855,7 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
         const dim3 grid((unsigned)nt, (unsigned)batch, (unsigned)g.splits);
         // direct-to-LDS loads when the rows are 16-byte vectors and at least two elements long (the first vector of every
         // row is then inside it); SCESS_GEMM_DMA=0 keeps the register-staged loads of the other precisions (tuning)
-        bool dma = kc == 2 && g.M >= 1 && g.N >= 1;
-        for (int q = 0; q < g.nseg; q++)
-            dma = dma && g.seg[q].K2 >= 2;
+        bool dma = kc == 2 && g.M >= 1 && g.N >= 1 && g.seg.K2 >= 2;
         if (const char *e = std::getenv("SCESS_GEMM_DMA"))
             dma = dma && (g.prec == P64 || std::atoi(e) != 0);
         const bool vec = kc == 2 && (g.prec != P64 || dma);

@@ -169,10 +169,9 @@ struct GemmSeg {
     GemmOp A, B;  // A rows m, B rows n
     int K1, K2;   // K = K1 x K2, K2 the inner (chunked) extent
 };
-// C[b][m][n] += alpha sum_seg sum_k A(m,k) B(n,k); splits > 1 sums K-range partials in order.
+// C[b][m][n] += alpha sum_k A(m,k) B(n,k); splits > 1 sums K-range partials in order.
 struct GemmArgs {
-    GemmSeg seg[2];
-    int nseg;
+    GemmSeg seg;
     int M, N;
     double *C;
     int64_t sCm, sCn, sCb;

@@ -38,18 +38,17 @@ static bool check(int prec, int batch, int splits, int M, int N, int K1, int K2,
         for (auto &y : *x)
             y = draw();
     GemmArgs g{};
-    g.nseg = 1;
     g.M = M;
     g.N = N;
     g.alpha = -0.5;
     g.splits = splits;
     g.prec = prec;
-    g.seg[0].K1 = K1;
-    g.seg[0].K2 = K2;
+    g.seg.K1 = K1;
+    g.seg.K2 = K2;
     double *dA = device(A), *dB = device(B), *dC = device(C);
     double *scratch = device(std::vector<double>((size_t)splits * batch * M * N, NAN));
-    g.seg[0].A = {dA, (int64_t)K1 * pitch, pitch, 1, ra};
-    g.seg[0].B = {dB, (int64_t)K1 * pitch, pitch, 1, rb};
+    g.seg.A = {dA, (int64_t)K1 * pitch, pitch, 1, ra};
+    g.seg.B = {dB, (int64_t)K1 * pitch, pitch, 1, rb};
     g.C = dC;
     g.sCm = N;
     g.sCn = 1;
