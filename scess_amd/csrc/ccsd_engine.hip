@@ -182,42 +182,45 @@ __global__ __launch_bounds__(256) void ladder_scatter_kernel(const double *rp, c
     }
 }
 
-// out[0] = max |t_ij^ab - t_ji^ba|, out[1] = max |t_ij^ab| as bit patterns (which order as the values, NaN above all); both
-// zero before. One work-group per (32 x 32 tile of a, b; pair i >= j); bound by one read of t.
-constexpr int kPairRow = 65535;  // pairs along y of the grid, the rest along z
+// out[2 b] = max |t_ij^ab - t_ji^ba|, out[2 b + 1] = max |t_ij^ab| over the work of block b, as bit patterns (which order as
+// the values, NaN above all); the (32 x 32 tile of a, b; pair i >= j) go round the blocks. Bound by one read of t; out is
+// pinned host memory, so that a small system pays for one launch and no copy.
+constexpr int kAsymBlocks = 1024;
 __global__ __launch_bounds__(256) void pair_asymmetry_kernel(const double *t, int o, int v, int nt, unsigned long long *out) {
     __shared__ double ji[32][33];
     __shared__ unsigned long long best[2];
-    const int pair = blockIdx.y + kPairRow * blockIdx.z;
-    if (pair >= tri(o))
-        return;
-    int i, j;
-    tile_pair(pair, i, j);
-    const int ta = blockIdx.x / nt, tb = blockIdx.x - ta * nt, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const double *x = t + ((int64_t)i * o + j) * v * v, *y = t + ((int64_t)j * o + i) * v * v;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     if (threadIdx.x < 2)
         best[threadIdx.x] = 0;
-    for (int r = ty; r < 32; r += 8) {
-        const int b = tb * 32 + r, a = ta * 32 + tx;
-        ji[r][tx] = a < v && b < v ? y[(int64_t)b * v + a] : 0.0;
-    }
-    __syncthreads();
     unsigned long long d = 0, m = 0;
     auto bits = [](double z) { return (unsigned long long)__double_as_longlong(fabs(z)); };
-    for (int r = ty; r < 32; r += 8) {
-        const int a = ta * 32 + r, b = tb * 32 + tx;
-        if (a < v && b < v) {
-            const double p = x[(int64_t)a * v + b], q = ji[tx][r];
-            d = max(d, bits(p - q));
-            m = max(m, max(bits(p), bits(q)));
+    const int64_t tiles = (int64_t)nt * nt, items = tri(o) * tiles;
+    for (int64_t w = blockIdx.x; w < items; w += gridDim.x) {
+        const int pair = (int)(w / tiles), tile = (int)(w - pair * tiles), ta = tile / nt, tb = tile - ta * nt;
+        int i, j;
+        tile_pair(pair, i, j);
+        const double *x = t + ((int64_t)i * o + j) * v * v, *y = t + ((int64_t)j * o + i) * v * v;
+        for (int r = ty; r < 32; r += 8) {
+            const int b = tb * 32 + r, a = ta * 32 + tx;
+            ji[r][tx] = a < v && b < v ? y[(int64_t)b * v + a] : 0.0;
         }
+        __syncthreads();
+        for (int r = ty; r < 32; r += 8) {
+            const int a = ta * 32 + r, b = tb * 32 + tx;
+            if (a < v && b < v) {
+                const double p = x[(int64_t)a * v + b], q = ji[tx][r];
+                d = max(d, bits(p - q));
+                m = max(m, max(bits(p), bits(q)));
+            }
+        }
+        __syncthreads();
     }
+    __syncthreads();
     atomicMax(&best[0], d);
     atomicMax(&best[1], m);
     __syncthreads();
-    if (threadIdx.x < 2 &&
-        best[threadIdx.x] > __hip_atomic_load(&out[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&out[threadIdx.x], best[threadIdx.x]);
+    if (threadIdx.x < 2)
+        out[2 * blockIdx.x + threadIdx.x] = best[threadIdx.x];
 }
 
 // A whole einsum of a small system in one launch, straight from the operands: G lanes per output element, lane g
@@ -800,9 +803,7 @@ Engine::~Engine() {
     if (dotbuf)
         (void)hipFree(dotbuf);
     if (asym)
-        (void)hipFree(asym);
-    if (asym_host)
-        (void)hipHostFree(asym_host);
+        (void)hipHostFree(asym);
     if (asym_done)
         (void)hipEventDestroy(asym_done);
 }
@@ -821,17 +822,15 @@ static void plus_transpose_add(Engine &E, DTensor &R, const DTensor &X, double a
 }
 
 void Engine::pair_check(const DTensor &t) {
-    const int64_t o = t.dims[0], v = t.dims[2], nt = (v + 31) / 32, np = o * (o + 1) / 2;
-    if (!asym_host) {
-        check(hipMalloc((void **)&asym, 16), "hipMalloc (symmetry of t2)");
+    const int64_t o = t.dims[0], v = t.dims[2], nt = (v + 31) / 32;
+    if (!asym) {
         check(hipEventCreateWithFlags(&asym_done, hipEventDisableTiming), "hipEventCreate");
-        check(hipHostMalloc((void **)&asym_host, 16, hipHostMallocDefault), "hipHostMalloc (symmetry of t2)");
+        check(hipHostMalloc((void **)&asym, sizeof(double) * 2 * kAsymBlocks, hipHostMallocDefault), "hipHostMalloc");
     }
-    check(hipMemsetAsync(asym, 0, 16, stream), "memset (symmetry of t2)");
-    const dim3 grid((unsigned)(nt * nt), (unsigned)std::min<int64_t>(np, kPairRow), (unsigned)((np + kPairRow - 1) / kPairRow));
-    hipLaunchKernelGGL(pair_asymmetry_kernel, grid, dim3(256), 0, stream, t.p, (int)o, (int)v, (int)nt, asym);
+    asym_blocks = (int)std::min<int64_t>(o * (o + 1) / 2 * nt * nt, kAsymBlocks);
+    hipLaunchKernelGGL(pair_asymmetry_kernel, dim3((unsigned)asym_blocks), dim3(256), 0, stream, t.p, (int)o, (int)v, (int)nt,
+                       (unsigned long long *)asym);
     check(hipGetLastError(), "symmetry of t2");
-    check(hipMemcpyAsync(asym_host, asym, 16, hipMemcpyDeviceToHost, stream), "copy (symmetry of t2)");
     check(hipEventRecord(asym_done, stream), "hipEventRecord");
 }
 
@@ -840,7 +839,12 @@ bool Engine::pair_symmetric() {
     // well above what rounding leaves in the amplitudes of an update (o=5, v=24 to o=16, v=157: 2e-16, FP32 2e-8, BF16x3 5e-8
     // of the largest), below the error of the products themselves
     const double tol = prec == P64 ? 1e-11 : prec == P32 ? 1e-6 : 1e-5;
-    return asym_host[0] <= tol * asym_host[1];
+    double d = 0.0, m = 0.0;
+    for (int b = 0; b < asym_blocks; b++) {
+        d = asym[2 * b] <= d ? d : asym[2 * b];  // NaN is kept
+        m = std::max(m, asym[2 * b + 1]);
+    }
+    return d <= tol * m;
 }
 
 // Particle-particle ladder sum_cd (ac|bd) tau_ij^cd from the Cholesky factor, (a,b) tiles of TAB x TAB

@@ -59,8 +59,8 @@ struct Engine {
     bool pair_symmetric();
 
 private:
-    unsigned long long *asym = nullptr;  // device
-    double *asym_host = nullptr;         // pinned: max |t_ij^ab - t_ji^ba|, max |t_ij^ab|
+    double *asym = nullptr;  // pinned: max |t_ij^ab - t_ji^ba| and max |t_ij^ab| of each block of the comparison
+    int asym_blocks = 0;
     hipEvent_t asym_done = nullptr;
 };
 
