@@ -57,7 +57,7 @@ struct PermWalk {
 
 // One output per thread, so that the lanes of a wave store (and, with beta != 0, load) consecutive
 // outputs: walking several consecutive outputs per thread saves index divisions but spreads every
-// store instruction over 32-byte strides (FP64 update at o=50, v=500: 1.33 s of permutes against 0.70 s).
+// store instruction over 32-byte strides (a CCSD update spent about twice the time in permutes).
 __global__ __launch_bounds__(256) void permute_kernel(PermArgs a) {
     const int64_t lin = element_id();
     if (lin >= a.n)
@@ -81,9 +81,8 @@ __device__ inline uint16_t bf16_rn(float f) {
 // one thread per group of 8 k of one row (two 16-byte stores)
 __global__ __launch_bounds__(256) void permute_split_kernel(PermArgs a, int64_t K, int64_t Kp, uint16_t *out,
                                                             int64_t nrows) {
-    // one element per thread: the lanes of a wave read consecutive k of a row (walking eight k per
-    // thread and storing 16-byte vectors spread each load over 64-byte strides: 0.74 s against 0.63 s
-    // of split permutes per BF16x3 update at o=50, v=500)
+    // one element per thread: the lanes of a wave read consecutive k of a row (walking eight k per thread and storing
+    // 16-byte vectors spread each load over 64-byte strides: 1.2 times the time of a BF16x3 update's split permutes)
     const int64_t lin = element_id();
     if (lin >= nrows * Kp)
         return;

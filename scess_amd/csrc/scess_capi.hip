@@ -543,8 +543,8 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     const int64_t wstride = vR * vR * vR;  // W in 8x8x8 blocks over vR^3
 
     // batch size: a multiple of 8 occupied triples per launch (8 for the int8 mode, 16 else), so that
-    // the XCD-ordered work-groups give each of the 8 XCDs whole triples (measured: the FP64 W-build at
-    // o=50, v=500 is 27% faster than with one triple per launch, at the same HBM bytes per triple);
+    // the XCD-ordered work-groups give each of the 8 XCDs whole triples (FP64 takes its items from queues, so it depends on
+    // this little: 1/64 of o=50, v=500 4.58 s with one triple per launch, 4.54 with eight);
     // fewer when the W sets (2 arrays x 2 sets x nbatch x vR^3) exceed a quarter of the free device memory.
     // FP64: 16 against 8 (o=20, v=200 0.549 s against 0.560 s: fewer half-empty ends of launches). For small v a launch
     // of 16 leaves the chip nearly empty, so it takes as many triples as make 8 rounds of the FP64 W-build's items over

@@ -860,7 +860,7 @@ hipError_t launch_gemm(const GemmArgs &g, int batch, hipStream_t s) {
             dma = dma && (g.prec == P64 || std::atoi(e) != 0);
         const bool vec = kc == 2 && (g.prec != P64 || dma);
         // 64 x 128 tiles for the direct-to-LDS pre-split BF16x3 products: twice the MFMAs per barrier for 1.5x the staged
-        // bytes (CCSD update at o=50, v=500: 6.66 s against 7.47 s with 64 x 64). SCESS_GEMM_WIDE=0 keeps 64 x 64 (tuning).
+        // bytes (CCSD update at o=50, v=500: 6.08 s against 7.14 s with 64 x 64). SCESS_GEMM_WIDE=0 keeps 64 x 64 (tuning).
         const char *ew = std::getenv("SCESS_GEMM_WIDE");
         const bool wide = dma && g.prec == PB3S && !(ew && std::atoi(ew) == 0);
 #define SCESS_KC(V, P, D)                                                                         \
@@ -1308,10 +1308,10 @@ static int back_blocks(int o, int v) {
 // Tiles of a term of the second kind
 static int back_tiles(int o, int v) { return ((v + 15) / 16 + 7) / 8 * back_cols(o, v); }
 
-// K ranges of a term of the second kind: 3072 work-groups (six rounds of the chip) from n triples, at most v
 // One round of the chip (o=10, v=75, 48 tiles: 12.7 ms spread, 13.0 not; o=20, v=200, 640 tiles: no difference)
 bool back_spread(int o, int v) { return back_blocks(o, v) < 512; }
 
+// K ranges of a term of the second kind: 3072 work-groups (six rounds of the chip) from n triples, at most v
 int back_splits(int n, int o, int v) { return std::max(1, std::min(v, 3072 / (6 * n * back_tiles(o, v)))); }
 
 hipError_t launch_back(const BackArgs &a0, const BackTarget *tg, const BackBatch &b, double *dT, double *dRn, hipStream_t s) {

@@ -692,10 +692,10 @@ __device__ inline bool seg_fx_on_a(bool fam1, int s) { return fam1 && (s == 0 ||
 // LDS rows are 128 bytes, 16-byte vector p of row r at slot p ^ swz(r); since swz(16 x + r) =
 // swz(r) ^ (2 x & 7), fragment (block x, step t) sits at lane offset so[t ^ x] + 2048 x: four offsets in all.
 //
-// Measured (E(T) per pass, same box; before: eight waves of 64 x 32 without balanced tiles, look-ahead or queue):
-// o=20, v=200 0.786 s -> 0.549 s, 1/16 of o=30, v=300 0.582 s -> 0.515 s. At v = 300 the pipes are busy 82-85% of
-// the cycles, at a clock that falls as they fill (busy x clock stayed at 1.76 GHz over four very different forms of
-// the kernel, 75% at 2.35 GHz to 85% at 2.08 GHz): the rest of the way to 78.6 TFLOP/s is power.
+// Measured (E(T) per pass; before: eight waves of 64 x 32 without balanced tiles, look-ahead or queue): o=20, v=200
+// 0.787 s -> 0.558 s, 1/16 of o=30, v=300 0.585 s -> 0.527 s. Alone at v = 300 the pipes are busy 85% of the cycles at
+// 2.26 GHz (63 TFLOP/s executed), with 84% of the L2 requests missing: a launch of 16 triples reads 110 GB at 4.8 TB/s, the
+// rate of a large copy. At v = 500 they are busy 87% at 2.36 GHz (68 TFLOP/s): there 46% miss and 2.6 TB/s suffice.
 // Segment s as in get_seg, one byte each: the orbital (0 = i, 1 = j, 2 = k) of the operand with the fixed index
 // (bits 0-1; X or TM), whether its rows are strided by v (bit 2: [row][fx], else [fx][row]), whether it is operand
 // A (bit 3), and the orbital pair q, r of the other operand T[q][r] or Rn[q][r] (bits 4-5, 6-7).
@@ -1235,8 +1235,8 @@ __global__ __launch_bounds__(F == 4 ? 512 : 256, (F == 1 || (F == 2 && S == 5)) 
 int i8_fixed_per_group(int slices) { return slices == 5 ? 2 : 1; }
 
 // MFMA blocks per wave edge, from timing sweeps: 2 (64x64 work-group tiles) for FP64 and FP32; 4 for BF16x3 where 64-wide
-// tiles need a fourth per edge: its three MFMAs per product leave it bound by the traffic of the operands, which halves
-// with the larger tile, but two 128-wide tiles pad v <= 192 too far (E(T), 2 / 4 blocks, ms: o=12, v=160 22.7 / 26.7, v=192
+// tiles need a fourth per edge: its three MFMAs per product want few operand bytes per MFMA, which halve with the larger
+// tile, but two 128-wide tiles pad v <= 192 too far (E(T), 2 / 4 blocks, ms: o=12, v=160 22.7 / 26.7, v=192
 // 37.3 / 38.6; 1/8 of o=16, v=200 16.9 / 13.0, v=224 21.5 / 15.6; 1/16 of o=16, v=239 12.9 / 10.0).
 int wbuild_tile(int prec, int v) {
     if (prec == PI8 || prec == P64)
