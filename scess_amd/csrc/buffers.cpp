@@ -32,14 +32,15 @@ BlockCache::BlockCache() {
 }
 
 BlockCache::~BlockCache() {
+    {
+        std::lock_guard<std::mutex> lk(g_caches_mu);
+        g_caches.erase(std::find(g_caches.begin(), g_caches.end(), this));
+    }
     flush();
-    std::lock_guard<std::mutex> lk(g_caches_mu);
-    g_caches.erase(std::find(g_caches.begin(), g_caches.end(), this));
 }
 
 // A block of this cache, or one of the runtime
 hipError_t BlockCache::take(void **p, size_t bytes, hipStream_t s) {
-    std::lock_guard<std::mutex> lk(m_);
     try {  // put() must not have to allocate
         used_.reserve(used_.size() + 1);
         free_.reserve(free_.size() + used_.size() + 1);
@@ -87,7 +88,6 @@ hipError_t BlockCache::get(void **p, size_t bytes, hipStream_t s) {
 void BlockCache::put(void *p) {
     if (!p)
         return;
-    std::lock_guard<std::mutex> lk(m_);
     for (size_t i = used_.size(); i-- > 0;)
         if (used_[i].p == p) {
             const Block b = used_[i];
@@ -104,17 +104,14 @@ void BlockCache::put(void *p) {
 }
 
 void BlockCache::flush() {
-    std::lock_guard<std::mutex> lk(m_);
     for (const Block &b : free_)
         (void)hipFreeAsync(b.p, b.s);
     free_.clear();
     cached_ = 0;
 }
 
-// The lock is held to the end: a context flushes its cache before its stream goes, and so waits for a thread that is here
-void BlockCache::trim(int device) {
-    std::lock_guard<std::mutex> lk(m_);
-    if (device_ < 0 || (device >= 0 && device != device_))
+void BlockCache::trim() {
+    if (device_ < 0)
         return;
     hipStream_t last = nullptr;
     for (const Block &b : free_) {
@@ -130,10 +127,15 @@ void BlockCache::trim(int device) {
     trim_pool(device_);
 }
 
+// A context ends in a Use that flushes, before its streams go, and leaves the list before its cache does: what is found here
+// has its stream or no blocks
 void BlockCache::trim_all(int device) {
     std::lock_guard<std::mutex> lk(g_caches_mu);
-    for (BlockCache *c : g_caches)
-        c->trim(device);
+    for (BlockCache *c : g_caches) {
+        std::unique_lock<std::recursive_mutex> use(c->use_, std::try_to_lock);
+        if (use.owns_lock() && c->device_ == device)
+            c->trim();
+    }
 }
 
 // ------------------------------------------------------------------- copies

@@ -13,7 +13,8 @@ namespace scess {
 // back to the runtime, and everything at the end of the context, on trim(), and where a context of the process finds the
 // device full. Stream ordered: a block is reused by work on the same stream (or ordered after it). A call's dozens of
 // allocations otherwise cost more than its kernels for small systems, and the mapping of freshly allocated memory some
-// milliseconds per GiB for large ones. Used by the context's thread; other threads only free kept blocks (trim_all).
+// milliseconds per GiB for large ones. Whoever uses it holds a Use for the length of the call; another thread only frees the
+// blocks of a context that is not in a call (trim_all).
 class BlockCache {
 public:
     static constexpr size_t kMaxCached = (size_t)6 << 30;
@@ -21,11 +22,14 @@ public:
     ~BlockCache();
     BlockCache(const BlockCache &) = delete;
     BlockCache &operator=(const BlockCache &) = delete;
+    struct Use {  // (a callback out of a call may make another one on the same context)
+        explicit Use(BlockCache &c) : lk(c.use_) {}
+        std::lock_guard<std::recursive_mutex> lk;
+    };
     hipError_t get(void **p, size_t bytes, hipStream_t s);
     void put(void *p);  // null is allowed
     void flush();       // the kept blocks go back to the runtime, in the order of their streams
-    // The kept blocks go back to the device, once the work that used them is done; not those of another device than `device`
-    void trim(int device = -1);
+    void trim();        // the kept blocks go back to the device, once the work that used them is done
     // p to at least `need` elements, without its contents; after an error p is null and cap 0
     template <class T> hipError_t grow(T *&p, size_t &cap, size_t need, hipStream_t s) {
         if (need <= cap)
@@ -46,8 +50,8 @@ private:
         hipStream_t s;
     };
     hipError_t take(void **p, size_t bytes, hipStream_t s);
-    static void trim_all(int device);  // the kept blocks of every context on the device
-    std::mutex m_;
+    static void trim_all(int device);  // of every context on the device that is not in a call, and of this thread's
+    std::recursive_mutex use_;
     std::vector<Block> free_, used_;
     size_t cached_ = 0;
     int device_ = -1;  // of the blocks; -1 before the first

@@ -204,9 +204,12 @@ void scess_destroy(scess_ctx *c) {
         return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    free_triples(c);
-    c->cc = scess::CcsdState{};
-    c->blocks.flush();
+    {
+        const scess::BlockCache::Use use(c->blocks);
+        free_triples(c);
+        c->cc = scess::CcsdState{};
+        c->blocks.flush();
+    }
     (void)hipStreamSynchronize(c->stream);
     (void)hipStreamSynchronize(c->stream2);
     (void)hipStreamDestroy(c->stream);
@@ -219,6 +222,7 @@ int scess_trim(scess_ctx *c) {
     if (!c)
         return SCESS_ERR_ARG;
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     c->blocks.trim();
     return SCESS_OK;
 }
@@ -273,6 +277,7 @@ int scess_t_set_inputs(scess_ctx *c, const scess_t_in *in, int prec_mask) {
     if ((prec_mask & 15) == 0 || (prec_mask & ~15))
         return fail(c, SCESS_ERR_ARG, "scess_t_set_inputs: prec_mask must be a non-empty subset of bits 0..3");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     free_triples(c);
     TriplesState &t = c->t;
@@ -534,6 +539,7 @@ int scess_t_forward_ex(scess_ctx *c, int prec, double *e_t, double *F_ijk, doubl
     if (!t.have_prec[prec])
         return fail(c, SCESS_ERR_STATE, "scess_t_forward: precision not packed by scess_t_set_inputs");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     const int64_t o = t.o, v = t.v, vR = t.vR;
     const int64_t nall = (int64_t)t.ijk_all.size() / 3;
     const int64_t nwork = (int64_t)t.work.size();
@@ -799,6 +805,7 @@ int scess_t_forward_noalloc(scess_ctx *c, int prec, double *e_t) {
     if (!c->scratch)
         return fail(c, SCESS_ERR_STATE, "scess_t_forward_noalloc: no scratch address for this device");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     const int64_t o = t.o, v = t.v, vR = t.vR;
     const int64_t nall = (int64_t)t.ijk_all.size() / 3;
     const int64_t nwork = (int64_t)t.work.size();
@@ -895,6 +902,7 @@ int scess_t_backward(scess_ctx *c, int prec, double dE, scess_t_grad *grad) {
     if (!t.have_prec[prec] || !t.have_prec[P64])
         return fail(c, SCESS_ERR_STATE, "scess_t_backward: needs SCESS_PREC_FP64 (and prec) packed");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     const int64_t o = t.o, v = t.v, vR = t.vR;
     const Operands &op = t.ops[prec];
     const Operands &o64 = t.ops[P64];
@@ -1258,6 +1266,7 @@ int scess_ccsd_set_inputs(scess_ctx *c, const scess_ccsd_in *in) {
         !in->oooo || (!in->vvvv && !in->chol_vv) || (in->chol_vv && in->naux < 1))
         return fail(c, SCESS_ERR_ARG, "scess_ccsd_set_inputs: missing block or non-positive size");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     try {
         scess::Engine &E = c->eng;
         scess::CcsdState &S = c->cc;
@@ -1322,6 +1331,7 @@ int scess_ccsd_update(scess_ctx *c, const double *t1, const double *t2, double *
     if (!c->cc.have)
         return fail(c, SCESS_ERR_STATE, "scess_ccsd_update: no inputs (call scess_ccsd_set_inputs first)");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     try {
         scess::Engine &E = c->eng;
         scess::CcsdState &S = c->cc;
@@ -1345,6 +1355,7 @@ int scess_ccsd_energy(scess_ctx *c, const double *t1, const double *t2, double *
     if (!c->cc.have)
         return fail(c, SCESS_ERR_STATE, "scess_ccsd_energy: no inputs");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     try {
         scess::Engine &E = c->eng;
         scess::CcsdState &S = c->cc;
@@ -1373,6 +1384,7 @@ int scess_transform_tei(scess_ctx *c, int64_t nao, int64_t nmo, const double *te
     if (!tei || !C || !out || nao <= 0 || nmo <= 0)
         return fail(c, SCESS_ERR_ARG, "scess_transform_tei: bad argument");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     try {
         scess::Engine &E = c->eng;
         // one index at a time, as TransformTEI (IntegralTransforms.cpp:33-58), last index first
@@ -1410,6 +1422,7 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
     if (!c->cc.have)
         return fail(c, SCESS_ERR_STATE, "scess_ccsd_solve: no inputs");
     HIP_TRY(c, hipSetDevice(c->device));
+    const scess::BlockCache::Use use(c->blocks);
     // thresholds of SolveRCCSD_DIIS (RCCSD.cpp:302-307)
     constexpr double ENERGY_CONVERGENCE = 1.0e-10, AMPLITUDE_CONVERGENCE = 1.0e-8;
     constexpr int MAX_ITERATIONS = 100, DIIS_START = 2, MAX_DIIS_VECS = 8;

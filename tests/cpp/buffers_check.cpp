@@ -9,6 +9,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -170,8 +171,18 @@ static void other_contexts() {
     a.trim();
     REQUIRE(dev.held == 0 && dev.live.empty());
     a.trim();
-    REQUIRE(a.get(&p, gib, stream(1)) == hipSuccess && p);
+    // not those of a context in a call on another thread
+    REQUIRE(a.get(&p, 5 * gib, stream(1)) == hipSuccess && p);
     a.put(p);
+    hipError_t e = hipSuccess;
+    {
+        const scess::BlockCache::Use use(a);
+        std::thread([&] { e = b.get(&q, 8 * gib, stream(2)); }).join();
+    }
+    REQUIRE(e == hipErrorOutOfMemory && !q);
+    std::thread([&] { e = b.get(&q, 8 * gib, stream(2)); }).join();
+    REQUIRE(e == hipSuccess && q);
+    b.put(q);
 }
 
 static std::vector<char> bytes(size_t n, unsigned seed) {
