@@ -833,17 +833,32 @@ void Engine::pair_check(const DTensor &t) {
     check(hipEventRecord(asym_done, stream), "hipEventRecord");
 }
 
+// well above what rounding leaves in the amplitudes of an update (o=5, v=24 to o=16, v=157: 2e-16, FP32 2e-8, BF16x3 5e-8
+// of the largest), below the error of the products themselves
+static double pair_tolerance(int prec) { return prec == P64 ? 1e-11 : prec == P32 ? 1e-6 : 1e-5; }
+
 bool Engine::pair_symmetric() {
     check(hipEventSynchronize(asym_done), "symmetry of t2");
-    // well above what rounding leaves in the amplitudes of an update (o=5, v=24 to o=16, v=157: 2e-16, FP32 2e-8, BF16x3 5e-8
-    // of the largest), below the error of the products themselves
-    const double tol = prec == P64 ? 1e-11 : prec == P32 ? 1e-6 : 1e-5;
     double d = 0.0, m = 0.0;
     for (int b = 0; b < asym_blocks; b++) {
         d = asym[2 * b] <= d ? d : asym[2 * b];  // NaN is kept
         m = std::max(m, asym[2 * b + 1]);
     }
-    return d <= tol * m;
+    return d <= pair_tolerance(prec) * m;
+}
+
+bool Engine::pair_symmetric(const double *t, int64_t o, int64_t v) const {
+    double d = 0.0, m = 0.0;
+    for (int64_t b = 0; b < v; b++)
+        for (int64_t a = 0; a < v; a++)
+            for (int64_t j = 0; j < o; j++)
+                for (int64_t i = j; i < o; i++) {
+                    const double p = t[i + o * (j + o * (a + v * b))], q = t[j + o * (i + o * (b + v * a))];
+                    const double e = std::fabs(p - q);
+                    d = e <= d ? d : e;  // NaN is kept
+                    m = std::max(m, std::max(std::fabs(p), std::fabs(q)));
+                }
+    return d <= pair_tolerance(prec) * m;
 }
 
 // Particle-particle ladder sum_cd (ac|bd) tau_ij^cd from the Cholesky factor, (a,b) tiles of TAB x TAB
@@ -996,10 +1011,8 @@ void CcsdState::ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R) {
     }
 }
 
-void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2, const bool *symmetric) {
+void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2, const std::function<bool()> &symmetric) {
     const int64_t O = o, Vv = v;
-    if (!vvvv_phys.p && !symmetric)
-        E.pair_check(t2);  // read where the ladder comes
     DTensor tau = E.alloc({O, O, Vv, Vv});
     make_tau(E, t1, t2, tau);
     DTensor Foo = E.alloc({O, O}), Fvv = E.alloc({Vv, Vv}), Fov = E.alloc({O, Vv});
@@ -1072,7 +1085,7 @@ void CcsdState::update(Engine &E, DTensor &t1, DTensor &t2, const bool *symmetri
         E.einsum("kcbd,ka->abcd", ovvv, &t1, Wvvvv, -1.0, 1.0);
         E.einsum("abcd,ijcd->ijab", Wvvvv, &tau, t2n, 1.0, 1.0);
     } else {
-        const bool sym = symmetric ? *symmetric : E.pair_symmetric();  // tau_ij^cd = tau_ji^dc
+        const bool sym = symmetric();  // tau_ij^cd = tau_ji^dc
         if (sym && E.prec == P64 && O * (O + 1) / 2 <= 65535)  // (pairs are a grid dimension)
             ladder_symmetric(E, tau, t2n);
         else  // (the other precisions keep their rounding: packing would split and round other values)

@@ -5,6 +5,7 @@
 #include "triples_internal.h"
 
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -54,9 +55,10 @@ struct Engine {
     static constexpr int kMaxDots = 8;
     void dots(const double *x, const double *const *y, int m, int64_t n, double *out);
     // Whether t (i, j, a, b) has t_ij^ab = t_ji^ba within the rounding of precision `prec`: pair_check() starts the
-    // comparison, pair_symmetric() waits for it
+    // comparison on the device, pair_symmetric() waits for it; or at once, for a ColMajor t on the host
     void pair_check(const DTensor &t);
     bool pair_symmetric();
+    bool pair_symmetric(const double *t, int64_t o, int64_t v) const;
 
 private:
     double *asym = nullptr;  // pinned: max |t_ij^ab - t_ji^ba| and max |t_ij^ab| of each block of the comparison
@@ -74,8 +76,8 @@ struct CcsdState {
     void make_tau(Engine &E, const DTensor &t1, const DTensor &t2, DTensor &tau);
     void ladder_from_factor(Engine &E, const DTensor &tau, DTensor &R);
     void ladder_symmetric(Engine &E, const DTensor &tau, DTensor &R);
-    // One Jacobi update (UpdateAmplitudes); symmetric: whether t_ij^ab = t_ji^ba is known to hold or not, null to find out
-    void update(Engine &E, DTensor &t1, DTensor &t2, const bool *symmetric = nullptr);
+    // One Jacobi update (UpdateAmplitudes); symmetric: whether t_ij^ab = t_ji^ba, asked where the ladder without vvvv comes
+    void update(Engine &E, DTensor &t1, DTensor &t2, const std::function<bool()> &symmetric);
     double energy(Engine &E, const DTensor &t1, const DTensor &t2);
 };
 

@@ -1177,6 +1177,8 @@ int engine_fail(scess_ctx *c, const std::exception &ex) {
     return fail(c, code, m);
 }
 
+constexpr int64_t kHostCompare = 1 << 16;
+
 // Contraction precision of the engine for one scope (FP64 again afterwards, also on exceptions)
 struct PrecScope {
     scess::Engine &E;
@@ -1338,7 +1340,12 @@ int scess_ccsd_update(scess_ctx *c, const double *t1, const double *t2, double *
         scess::DTensor d1 = upload_colmajor(E, t1, {S.o, S.v});
         scess::DTensor d2 = upload_colmajor(E, t2, {S.o, S.o, S.v, S.v});
         const PrecScope ps(E, c->ccsd_prec);
-        S.update(E, d1, d2);
+        // A small t2 is compared on the host, while the device works on the terms before the ladder: the device's
+        // comparison would cost it 15 us
+        const bool small = S.o * S.o * S.v * S.v <= kHostCompare;
+        if (!S.vvvv_phys.p && !small)
+            E.pair_check(d2);
+        S.update(E, d1, d2, [&] { return small ? E.pair_symmetric(t2, S.o, S.v) : E.pair_symmetric(); });
         download_colmajor(E, d1, t1_new);
         download_colmajor(E, d2, t2_new);
     } catch (const std::exception &ex) {
@@ -1462,7 +1469,7 @@ int scess_ccsd_solve(scess_ctx *c, double *t1_out, double *t2_out, scess_ccsd_re
             HIP_TRY(c, hipMemcpyAsync(prev.p, t1.p, 8 * n1, hipMemcpyDeviceToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(prev.p + n1, t2.p, 8 * n2, hipMemcpyDeviceToDevice, c->stream));
             const PrecScope ps(E, c->ccsd_prec);
-            S.update(E, t1, t2, &symmetric);
+            S.update(E, t1, t2, [&] { return symmetric; });
             HIP_TRY(c, hipMemcpyAsync(upd.p, t1.p, 8 * n1, hipMemcpyDeviceToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(upd.p + n1, t2.p, 8 * n2, hipMemcpyDeviceToDevice, c->stream));
             E.axpby(change.p, upd.p, prev.p, 1.0, -1.0, nt);

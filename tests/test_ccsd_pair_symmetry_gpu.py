@@ -22,9 +22,10 @@ def _system(o, v, seed, scale):
     return e, eri, blocks, np.asfortranarray(L[:, o:, o:].transpose(1, 2, 0))
 
 
-# v around the 32-wide tiles of the comparison; how far off: everywhere, or one element of the last tile
+# compared on the host up to 65536 elements, on the device from there on (33-wide: the 32-wide tiles' edge); how far off:
+# everywhere, or one element of the last tile
 @pytest.mark.parametrize("o,v,seed,one", [(1, 5, 1, False), (3, 7, 2, False), (2, 33, 3, False), (4, 24, 4, True),
-                                          (3, 65, 5, True)])
+                                          (3, 65, 5, True), (8, 33, 6, False), (8, 33, 7, True), (4, 65, 8, True)])
 def test_update_of_any_t2(o, v, seed, one):
     print(f"case ccsd any t2 o={o} v={v} one={one}", flush=True)
     e, eri, blocks, chol = _system(o, v, seed, 0.3)
