@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void ladder_scatter_kernel(const double *rp, c
 
 // out[2 b] = max |t_ij^ab - t_ji^ba|, out[2 b + 1] = max |t_ij^ab| over the work of block b, as bit patterns (which order as
 // the values, NaN above all); the (32 x 32 tile of a, b; pair i >= j) go round the blocks. Bound by one read of t; out is
-// pinned host memory, so that a small system pays for one launch and no copy.
+// pinned host memory: one launch and no copy.
 constexpr int kAsymBlocks = 1024;
 __global__ __launch_bounds__(256) void pair_asymmetry_kernel(const double *t, int o, int v, int nt, unsigned long long *out) {
     __shared__ double ji[32][33];
